@@ -421,244 +421,243 @@ __device__ __forceinline__ void copy_next_block(const FrontDev &F, const AptpSta
 // APTP: complete pivoting on the inner block (factor_block_diagonal, factor.rs:891-1153).
 // Returns the eliminated count; bp/bkind/bdiag/boff describe the pivots and *maxl the largest
 // |l| of the block.
+//
+// The pivot steps are one serial chain, so one wavefront (the workgroup's first; the others wait
+// at the closing barrier) runs them without any barrier, and everything is laid out for the
+// fewest instructions and LDS round trips per step:
+//  * The block is symmetric; every unordered pair {i, i + d mod 32}, d = 1 .. 16, has one owner.
+//    Lane (i = lane & 31, h = lane >> 5) keeps e[u] = a(i, j), j = i + 1 + u + 8h (mod 32), in
+//    registers: eight entries per lane with no lane idle (d = 16 would be owned twice; the copy
+//    of the rows i >= 16 is dead), and the diagonal in lanes h = 0.
+//  * Entries stay at their original indices; no row or column is moved.  pos[i] is the position
+//    the reference's swaps would have put row i at.  It only decides the order of the factors of
+//    an update (the row at the larger position gives l, the other w = l d) and ties.
+//  * A dead entry (eliminated, outside the block, the second copy) is NaN.  fmax ignores it, the
+//    diagonal of the LDS copy is NaN, so a pivot's own row gets NaN multipliers and dies in the
+//    ordinary update: no masks.
+//  * Argmax: the high words of the lanes' maxima are reduced by DPP; unless one lane and one of
+//    its entries alone has that high word (ties, or maxima equal in their upper 32 bits), the
+//    exact rule runs: largest value, then first in the column-major order of positions.
+//  * A full symmetric copy of the block in LDS gives a lane the pivot row's entries of its own row
+//    and of its eight columns in one round trip, beside the reciprocal of the pivot.
+// Measured on the 64^3 Helmholtz chain (see k_aptp_outer): the form it replaced, 256 threads
+// with four entries each, the block permuted through LDS and one barrier per step, took 40 us per
+// 32-column block.
 // ===========================================================================
-// The same complete pivoting by a whole workgroup of 256 threads: thread (row r = tid & 31,
-// column group cg = tid >> 5) owns the entries j = cg + 8u of row r and keeps them in registers.
-// One barrier per pivot step: scan of the own entries, argmax over the workgroup (DPP within
-// wavefronts, per-wavefront partials with the winner's signed value through LDS), barrier, then
-// the pivot decision and the step's symmetric swaps are folded into where each thread reads its
-// new entries: the block lives in two LDS buffers, each step reads the current one at the
-// swapped positions (new(r, c) = old(s(r), s(c)), s the step's swap sequence) and writes the
-// updated entries to the other.  Partials, diagonals and the row order are double-buffered the
-// same way.  Multipliers are kept by row identity in lbuf and placed into the block at the end.
-__device__ int block_factor_wg(double (*blk)[MAX_IB + 1], double (*blk2)[MAX_IB + 1], int *bp, int *bp2,
-                               int8_t *bkind, double *bdiag, double *boff, int bs, double small,
-                               double *maxl, double *wbv, int *wbp, double *wbs,
-                               double (*lbuf)[MAX_IB + 1], bool probe = false) {
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int r = tid & 31, cg = tid >> 5;
-#ifdef RV_PHASE_TIMING
-    unsigned long long tp[6] = {0, 0, 0, 0, 0, 0}, tq = clock64();
-#define RV_STEP_MARK(i) do { if (probe) { const unsigned long long tn_ = clock64(); tp[i] += tn_ - tq; tq = tn_; } } while (0)
-#else
-#define RV_STEP_MARK(i) do {} while (0)
-#endif
-    if (tid < MAX_IB) { bp[tid] = tid; bkind[tid] = 0; bdiag[tid] = 0.0; boff[tid] = 0.0; }
-    double e[4];
+// max(|a|, |b|), NaN operands ignored (the compiler's fmax canonicalises loop-carried operands
+// first, one more instruction each)
+__device__ __forceinline__ double max_abs(double a, double b) {
+    double r;
+    __asm__("v_max_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// unsigned maximum over the wavefront, uniform
+__device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
+    v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false));  // row_shr:1
+    v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false));  // row_shr:2
+    v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false));  // row_shr:4
+    v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false));  // row_shr:8
+    v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false));  // row_bcast:15
+    v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false));  // row_bcast:31
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// The pivot steps, by one wavefront.  S: 32 x 32 doubles (the symmetric copy), ptab: 32 ints
+// (positions), lbuf: the multipliers by row identity and pivot position.  On return bp holds the
+// row at each position and the diagonal of S the uneliminated diagonal entries.
+__device__ __forceinline__ int block_pivots(const double (*blk)[MAX_IB + 1], double *S, int *bp, int *ptab,
+                                            int8_t *bkind, double *bdiag, double *boff, int bs, double small,
+                                            double *maxl, double (*lbuf)[MAX_IB + 1]) {
+    static_assert(MAX_IB == 32, "lane layout of the block");
+    const int lane = threadIdx.x & 63, i = lane & 31, h = lane >> 5;
+    const double dead = __builtin_nan("");
+    if (lane < MAX_IB) { bkind[lane] = 0; bdiag[lane] = 0.0; boff[lane] = 0.0; ptab[lane] = lane; }
+    double e[8];
+    int jo[8], w1[8], w2[8];  // column, and the entry's two places in S
 #pragma unroll
-    for (int u = 0; u < 4; ++u) e[u] = blk[r][cg + 8 * u];
-    // the diagonal of the row at position r, kept by every thread of the row (recomputed each
-    // step with the arithmetic of the thread that owns the entry); the diagonal at column j is
-    // then held by the lane of row j with this thread's column group, in the same wavefront
-    double dreg = blk[r][r];
-    double (*X)[MAX_IB + 1] = blk;
-    double (*Y)[MAX_IB + 1] = blk2;
-    int *bpX = bp, *bpY = bp2;
-    int kk = 0, par = 0;
+    for (int u = 0; u < 8; ++u) {
+        const int j = (i + 1 + u + 8 * h) & 31;
+        const bool copy2 = u == 7 && h == 1 && i >= 16;
+        const double v = blk[max(i, j)][min(i, j)];
+        e[u] = (i < bs && j < bs && !copy2) ? v : dead;
+        jo[u] = j;
+        w1[u] = copy2 ? 33 * i : 32 * i + j;  // (the second copy writes its NaN to the diagonal)
+        w2[u] = copy2 ? 33 * i : 32 * j + i;
+    }
+    double dg = (h == 0 && i < bs) ? blk[i][i] : dead;
+    if (h == 0) S[33 * i] = dead;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) { S[w1[u]] = e[u]; S[w2[u]] = e[u]; }
+    int posr = i, idr = i;
+    int cur = 0;
     double ml = 0.0;
-    while (kk < bs) {
-        const int cur = kk;
-        // argmax |a_ij| over the remaining lower block, first in column-major scan order
-        double bv = 0.0, sv = 0.0;
-        int bpos = INT_MAX;
-        {
-            const bool row_live = r >= cur && r < bs;
+    wave_sync();
+    while (cur < bs) {
+        double m = max_abs(max_abs(max_abs(e[0], e[1]), max_abs(e[2], e[3])),
+                           max_abs(max_abs(e[4], e[5]), max_abs(e[6], e[7])));
+        m = max_abs(max_abs(m, dg), 0.0);
+        unsigned bits = (fabs(dg) == m) ? 256u : 0u;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int j = cg + 8 * u;
-                const double a = fabs(e[u]);
-                const bool take = row_live && j >= cur && j <= r && a > bv;
-                bv = take ? a : bv;
-                sv = take ? e[u] : sv;
-                bpos = take ? j * 64 + r : bpos;
+        for (int u = 0; u < 8; ++u) bits |= (fabs(e[u]) == m) ? 1u << u : 0u;
+        const unsigned hi = (unsigned)((unsigned long long)__double_as_longlong(m) >> 32);
+        const unsigned M = wave_max_u32(hi);
+        const unsigned long long mask = __ballot(hi == M);
+        const int Lw = __builtin_ctzll(mask);
+        const unsigned wb = (unsigned)__builtin_amdgcn_readlane((int)bits, Lw);
+        double gv;
+        int ia, ib;  // the winner's two rows (equal: a diagonal entry)
+        if (M >= 0x00100000u && (mask & (mask - 1)) == 0 && (wb & (wb - 1)) == 0) {
+            gv = readlane_f64(m, Lw);
+            ia = Lw & 31;
+            ib = (wb == 256u) ? ia : (ia + 1 + __builtin_ctz(wb) + 8 * (Lw >> 5)) & 31;
+        } else {
+            // largest value, equal values by position; no live entry above zero: position cur
+            gv = wave_fmax(m);
+            int key = (fabs(dg) == gv) ? 65 * posr : INT_MAX;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int pj = ptab[jo[u]];
+                key = (fabs(e[u]) == gv) ? min(key, 64 * min(posr, pj) + max(posr, pj)) : key;
             }
+            key = (gv > 0.0) ? __builtin_amdgcn_readfirstlane(wave_min_int(key)) : 65 * cur;
+            gv = readlane_f64(gv, 0);
+            ia = __builtin_amdgcn_readlane(idr, key & 63);
+            ib = __builtin_amdgcn_readlane(idr, key >> 6);
         }
-        // per-wavefront partials: value, position, and the winner's signed value and the two
-        // diagonals of its 2x2 test
-        double *pv_ = wbv + 4 * par, *ps_ = wbs + 4 * par, *pr_ = wbs + 8 + 4 * par, *pc_ = wbs + 16 + 4 * par;
-        int *pp_ = wbp + 4 * par;
-        const int jb = (bpos == INT_MAX) ? r : (bpos >> 6);
-        const double dc_ = __shfl(dreg, jb + 32 * (cg & 1));
-        RV_STEP_MARK(0);
-        {
-            const double vmax = wave_max_dpp(bv);
-            const int pos = wave_argmax_pos(bv, bpos, vmax);
-            if (pos != INT_MAX && bpos == pos) { ps_[wv] = sv; pr_[wv] = dreg; pc_[wv] = dc_; }
-            if (lane == 0) { pv_[wv] = vmax; pp_[wv] = pos; }
-        }
-        RV_STEP_MARK(1);
-        lds_barrier();
-        RV_STEP_MARK(2);
-        // all partials in one round trip, then the combination in registers
-        double qv[4], qs[4], qr[4], qc[4];
-        int qp[4];
-#pragma unroll
-        for (int w = 0; w < 4; ++w) { qv[w] = pv_[w]; qp[w] = pp_[w]; qs[w] = ps_[w]; qr[w] = pr_[w]; qc[w] = pc_[w]; }
-        // larger value wins, an equal value with the smaller position wins: a strict order over
-        // the partials' distinct positions, combined as a tree (two levels instead of three)
-        auto wins = [](double va, int pa, double vb, int pb) { return vb > va || (vb == va && pb < pa); };
-        const int w01 = wins(qv[0], qp[0], qv[1], qp[1]) ? 1 : 0;
-        const int w23 = wins(qv[2], qp[2], qv[3], qp[3]) ? 3 : 2;
-        const double v01 = w01 ? qv[1] : qv[0], v23 = (w23 == 3) ? qv[3] : qv[2];
-        const int p01 = w01 ? qp[1] : qp[0], p23 = (w23 == 3) ? qp[3] : qp[2];
-        const bool hi = wins(v01, p01, v23, p23);
-        const double gv = hi ? v23 : v01;
-        const int gp = hi ? p23 : p01;
-        const int gw = hi ? w23 : w01;
-        const double atm = (gw == 0) ? qs[0] : (gw == 1) ? qs[1] : (gw == 2) ? qs[2] : qs[3];
-        const double att = (gw == 0) ? qr[0] : (gw == 1) ? qr[1] : (gw == 2) ? qr[2] : qr[3];
-        const double amm = (gw == 0) ? qc[0] : (gw == 1) ? qc[1] : (gw == 2) ? qc[2] : qc[3];
         if (gv < small) break;
-        const int mr = (gp == INT_MAX) ? cur : (gp & 63);
-        const int mc = (gp == INT_MAX) ? cur : (gp >> 6);
-        // the step's swaps: first (a1 b1), then (a2 b2); s(x) = t1(t2(x)) maps a new position to
-        // the current one.  p11 (1x1) or p11, p22, p21 (2x2) is the pivot (block) as it will
-        // stand at position cur (and cur + 1): the winner's entry and the diagonals it carried.
-        int a1 = cur, b1 = cur, a2 = -1, b2 = -1, piv2 = 0;
-        double p11, p22 = 0.0, p21 = 0.0;
-        if (gp == INT_MAX) {
-            p11 = (&X[0][0])[__umul24((unsigned)cur, MAX_IB + 2)];
-        } else if (mr == mc) {
-            b1 = mr;
-            p11 = atm;
-        } else {
-            const int t = mr, mi = mc;
-            const double delta = amm * att - atm * atm;
-            if (fabs(delta) >= 0.5 * atm * atm) {
-                piv2 = 1;
-                b1 = mi;
-                a2 = cur + 1;
-                b2 = (t == cur) ? mi : t;
-                p11 = amm; p22 = att; p21 = atm;
-            } else {
-                const bool first = fabs(amm) >= fabs(att);
-                b1 = first ? mi : t;
-                p11 = first ? amm : att;
+        // t: the winner's row (larger position), mi: its column
+        const int qa = __builtin_amdgcn_readlane(posr, ia), qb = __builtin_amdgcn_readlane(posr, ib);
+        const int t = qa > qb ? ia : ib, mi = qa > qb ? ib : ia;
+        const int pt = max(qa, qb), pm = min(qa, qb);
+        const double att = readlane_f64(dg, t), amm = readlane_f64(dg, mi);
+        bool two = false;
+        int pid = t, pp = pt;  // 1x1: the pivot's row and position
+        double d = att;
+        if (t != mi) {
+            const double delta = amm * att - gv * gv;
+            if (fabs(delta) >= 0.5 * gv * gv) {
+                two = true;
+            } else if (fabs(amm) >= fabs(att)) {
+                pid = mi; pp = pm; d = amm;
             }
         }
-        auto sg = [&](int x) {
-            x = (x == a2) ? b2 : (x == b2 ? a2 : x);
-            return (x == a1) ? b1 : (x == b1 ? a1 : x);
-        };
-        // entry (x, y) of the lower block in the current buffer (24-bit multiplies: full rate)
-        const double *Xf = &X[0][0];
-        auto at = [&](int x, int y) { return Xf[__umul24((unsigned)x, MAX_IB + 1) + y]; };
-        auto val = [&](int x, int y) { return x >= y ? at(x, y) : at(y, x); };
-        // the step's permutation as a table in the lanes (lane l holds s(l & 31)), read by shuffle
-        const int sgl = sg(lane & 31);
-        const int sr = __shfl(sgl, r);
-        int sj[4];
-        double eo[4];
+        const int x1 = __builtin_amdgcn_readlane(idr, cur);  // the row standing at position cur
+        if (!two) {
+            const double *row = S + 32 * pid;
+            const double ci = row[i];
+            double cj[8];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            sj[u] = __shfl(sgl, cg + 8 * u);
-            eo[u] = val(sr, sj[u]);
-        }
-        const double drr = at(sr, sr);  // old diagonal of the row now at position r
-        const int rid = bpX[sr];  // identity of the row now at position r
-        RV_STEP_MARK(3);
-        const double pinv = 1.0 / (piv2 ? p11 * p22 - p21 * p21 : p11);
-        if (!piv2) {
-            const int sc = sg(cur);
-            const double dkk = p11;
-            const double ar = val(sr, sc);
-            double aj[4];
+            for (int u = 0; u < 8; ++u) cj[u] = row[jo[u]];
+            posr = (i == x1) ? pp : posr;
+            posr = (i == pid) ? cur : posr;
+            idr = (lane == pp) ? x1 : idr;
+            idr = (lane == cur) ? pid : idr;
+            ptab[i] = posr;
+            wave_sync();
+            int pj[8];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) aj[u] = val(sj[u], sc);
-            const double inv = pinv;
-            const bool row_live = r > cur && r < bs;
-            const double lr = ar * inv;
+            for (int u = 0; u < 8; ++u) pj[u] = ptab[jo[u]];
+            const double inv = 1.0 / d;
+            const double li = ci * inv, wi = li * d;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int j = cg + 8 * u;
-                const double ldl = (aj[u] * inv) * dkk;
-                const double nv = eo[u] - lr * ldl;
-                e[u] = (row_live && j > cur && j <= r) ? nv : eo[u];
+            for (int u = 0; u < 8; ++u) {
+                const double lj = cj[u] * inv, wj = lj * d;
+                const double p1 = li * wj, p2 = lj * wi;
+                e[u] = e[u] - (posr > pj[u] ? p1 : p2);
             }
-            // the new diagonal of the row (entry (r, r): eo = drr, aj = ar)
-            dreg = row_live ? drr - lr * ((ar * inv) * dkk) : drr;
-            if (cg == 0 && row_live) {
-                lbuf[rid][cur] = lr;
-                ml = fmax(ml, fabs(lr));
-            }
-            if (tid == 0) { bkind[cur] = 1; bdiag[cur] = dkk; }
-            kk += 1;
+            dg = dg - li * wi;
+            ml = max_abs(ml, li);
+            if (h == 0) lbuf[i][cur] = li;
+            if (lane == 0) { bkind[cur] = 1; bdiag[cur] = d; }
+            cur += 1;
         } else {
-            const int s1 = sg(cur), s2 = sg(cur + 1);
-            const double a11 = p11, a22 = p22, a21 = p21;
-            const double ai1 = val(sr, s1), ai2 = val(sr, s2);
-            double aj1[4], aj2[4];
+            // mi goes to position cur, then t to cur + 1 (t stands at mi's old position if it was
+            // the row at cur)
+            const double *r1 = S + 32 * mi, *r2 = S + 32 * t;
+            const double a11 = amm, a22 = att, a21 = r1[t];
+            const double ci1 = r1[i], ci2 = r2[i];
+            double cj1[8], cj2[8];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                aj1[u] = val(sj[u], s1);
-                aj2[u] = val(sj[u], s2);
-            }
-            const double inv_det = pinv;
-            const bool row_live = r > cur + 1 && r < bs;
-            const double l1r = (ai1 * a22 - ai2 * a21) * inv_det;
-            const double l2r = (ai2 * a11 - ai1 * a21) * inv_det;
+            for (int u = 0; u < 8; ++u) { cj1[u] = r1[jo[u]]; cj2[u] = r2[jo[u]]; }
+            posr = (i == x1) ? pm : posr;
+            posr = (i == mi) ? cur : posr;
+            idr = (lane == pm) ? x1 : idr;
+            idr = (lane == cur) ? mi : idr;
+            const int x2 = __builtin_amdgcn_readlane(idr, cur + 1), p2s = __builtin_amdgcn_readlane(posr, t);
+            posr = (i == x2) ? p2s : posr;
+            posr = (i == t) ? cur + 1 : posr;
+            idr = (lane == p2s) ? x2 : idr;
+            idr = (lane == cur + 1) ? t : idr;
+            ptab[i] = posr;
+            wave_sync();
+            int pj[8];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int j = cg + 8 * u;
-                const double l1j = (aj1[u] * a22 - aj2[u] * a21) * inv_det;
-                const double l2j = (aj2[u] * a11 - aj1[u] * a21) * inv_det;
-                const double wj1 = l1j * a11 + l2j * a21;
-                const double wj2 = l1j * a21 + l2j * a22;
-                const double nv = eo[u] - (l1r * wj1 + l2r * wj2);
-                e[u] = (row_live && j > cur + 1 && j <= r) ? nv : eo[u];
+            for (int u = 0; u < 8; ++u) pj[u] = ptab[jo[u]];
+            const double inv_det = 1.0 / (a11 * a22 - a21 * a21);
+            const double l1i = (ci1 * a22 - ci2 * a21) * inv_det;
+            const double l2i = (ci2 * a11 - ci1 * a21) * inv_det;
+            const double w1i = l1i * a11 + l2i * a21, w2i = l1i * a21 + l2i * a22;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const double l1j = (cj1[u] * a22 - cj2[u] * a21) * inv_det;
+                const double l2j = (cj2[u] * a11 - cj1[u] * a21) * inv_det;
+                const double w1j = l1j * a11 + l2j * a21, w2j = l1j * a21 + l2j * a22;
+                const double p1 = l1i * w1j + l2i * w2j, p2 = l1j * w1i + l2j * w2i;
+                e[u] = e[u] - (posr > pj[u] ? p1 : p2);
             }
-            {
-                // the new diagonal of the row (entry (r, r): eo = drr, aj1 = ai1, aj2 = ai2)
-                const double wr1 = l1r * a11 + l2r * a21;
-                const double wr2 = l1r * a21 + l2r * a22;
-                dreg = row_live ? drr - (l1r * wr1 + l2r * wr2) : drr;
-            }
-            if (cg == 0 && row_live) {
-                lbuf[rid][cur] = l1r;
-                lbuf[rid][cur + 1] = l2r;
-                ml = fmax(ml, fmax(fabs(l1r), fabs(l2r)));
-            }
-            if (tid == 0) {
+            dg = dg - (l1i * w1i + l2i * w2i);
+            ml = max_abs(max_abs(ml, l1i), l2i);
+            if (h == 0) { lbuf[i][cur] = l1i; lbuf[i][cur + 1] = l2i; }
+            if (lane == 0) {
                 bkind[cur] = 2; bkind[cur + 1] = 3;
                 bdiag[cur] = a11; bdiag[cur + 1] = a22; boff[cur] = a21;
             }
-            kk += 2;
+            cur += 2;
         }
-        // the next buffer; the next step's barrier orders these stores before its reads
 #pragma unroll
-        for (int u = 0; u < 4; ++u) (&Y[0][0])[__umul24((unsigned)r, MAX_IB + 1) + cg + 8 * u] = e[u];
-        if (cg == 0) bpY[r] = rid;
-        double (*tX)[MAX_IB + 1] = X; X = Y; Y = tX;
-        int *tb = bpX; bpX = bpY; bpY = tb;
-        par ^= 1;
-        RV_STEP_MARK(4);
+        for (int u = 0; u < 8; ++u) { S[w1[u]] = e[u]; S[w2[u]] = e[u]; }
+        wave_sync();
     }
-#ifdef RV_PHASE_TIMING
-    if (probe)
-        for (int i = 0; i < 5; ++i) atomicAdd(&g_phase[1][8 + i], tp[i]);
-#endif
-#undef RV_STEP_MARK
+    if (lane < MAX_IB) {
+        bp[lane] = idr;
+        S[33 * i] = dg;
+    }
+    *maxl = wave_max_dpp(ml);
+    return cur;
+}
+
+// All 256 threads: the block in blk (lower triangle) on entry; the factored block in position
+// order on return (D's off-diagonal of a 2x2 at (q + 1, q)).  blk2, lbuf, bp2: working LDS.
+__device__ __forceinline__ int block_factor_wg(double (*blk)[MAX_IB + 1], double (*blk2)[MAX_IB + 1], int *bp, int *bp2,
+                                               int8_t *bkind, double *bdiag, double *boff, int bs, double small,
+                                               double *maxl, double *wbv, int *wbp, double (*lbuf)[MAX_IB + 1]) {
+    const int tid = threadIdx.x;
+    double *S = &blk2[0][0];
+    if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) {
+        __builtin_amdgcn_s_setprio(3);
+        double ml;
+        const int kk = block_pivots(blk, S, bp, bp2, bkind, bdiag, boff, bs, small, &ml, lbuf);
+        __builtin_amdgcn_s_setprio(0);
+        if (tid == 0) { wbv[0] = ml; wbp[0] = kk; }
+    }
     lds_barrier();
-    // the final block and row order into blk / bp
-    if (X != blk) {
-        for (int x = tid; x < MAX_IB * MAX_IB; x += 256) {
-            const int p = x & (MAX_IB - 1), q = x >> 5;
-            blk[p][q] = X[p][q];
-        }
-        if (tid < MAX_IB) bp[tid] = bpX[tid];
-        lds_barrier();
+    const int kk = __builtin_amdgcn_readfirstlane(wbp[0]);
+    *maxl = wbv[0];
+    // position (p, q): a multiplier of pivot q of the row now at p, D, or an uneliminated entry
+    const int p = tid & (MAX_IB - 1);
+    const int rid = bp[p];
+#pragma unroll
+    for (int u = 0; u < MAX_IB / 8; ++u) {
+        const int q = (tid >> 5) + 8 * u;
+        if (q > p || p >= bs) continue;
+        double v;
+        if (q >= kk) v = S[32 * rid + bp[q]];
+        else if (p == q) v = bdiag[q];
+        else v = (bkind[q] == 2 && p == q + 1) ? boff[q] : lbuf[rid][q];
+        blk[p][q] = v;
     }
-    // multipliers into the block: the row now at position p is row bp[p] of the steps that
-    // formed them; the D off-diagonal of a 2x2 stays at (q+1, q)
-    for (int x = tid; x < MAX_IB * MAX_IB; x += 256) {
-        const int p = x & (MAX_IB - 1), q = x >> 5;
-        if (q < kk && p > q && p < bs && !(bkind[q] == 2 && p == q + 1)) blk[p][q] = lbuf[bp[p]][q];
-    }
-    // largest |l| of the block
-    const double wm = wave_max_dpp(ml);
-    if (lane == 0) wbv[wv] = wm;
     lds_barrier();
-    *maxl = fmax(fmax(wbv[0], wbv[1]), fmax(wbv[2], wbv[3]));
     return kk;
 }
 
@@ -800,8 +799,8 @@ __global__ __launch_bounds__(256) void k_block_apply(FrontDev *__restrict__ fr,
     __shared__ int bp[MAX_IB], operm[MAX_IB];
     __shared__ int8_t bkind[MAX_IB];
     __shared__ double bdiag[MAX_IB], boff[MAX_IB], dinv[MAX_IB];
-    __shared__ double wbv[8], wbs[24];
-    __shared__ int wbp[8], bp2[MAX_IB];
+    __shared__ double wbv[1];
+    __shared__ int wbp[1], bp2[MAX_IB];
     __shared__ double lbuf[MAX_IB][MAX_IB + 1], blk2[MAX_IB][MAX_IB + 1];
     const int tid = threadIdx.x;
     const int r = be + chunk * 256 + tid;
@@ -873,7 +872,7 @@ __global__ __launch_bounds__(256) void k_block_apply(FrontDev *__restrict__ fr,
     lds_barrier();
     RV_PHASE(0, 1);
     double bml;
-    bn = block_factor_wg(blk, blk2, bp, bp2, bkind, bdiag, boff, bs, small, &bml, wbv, wbp, wbs, lbuf);
+    bn = block_factor_wg(blk, blk2, bp, bp2, bkind, bdiag, boff, bs, small, &bml, wbv, wbp, lbuf);
     RV_PHASE(0, 2);
     // D off-diagonals of 2x2 pivots read as zeros of L11 (factor.rs:1898-1912)
     if (tid < bn) {
@@ -1097,8 +1096,8 @@ __device__ void lookahead_factor(FrontDev &F, AptpState &S, double (*Wr)[MAX_IB 
     __shared__ int bp[MAX_IB], bp2[MAX_IB], operm[MAX_IB];
     __shared__ int8_t bkind[MAX_IB];
     __shared__ double bdiag[MAX_IB], boff[MAX_IB];
-    __shared__ double wbv[8], wbs[24];
-    __shared__ int wbp[8];
+    __shared__ double wbv[1];
+    __shared__ int wbp[1];
     __shared__ int8_t kd[MAX_IB];
     __shared__ double dd[MAX_IB], od[MAX_IB];
     double (*Lr)[MAX_IB + 1] = Wr;            // L rows of the next block in this block's columns
@@ -1144,12 +1143,10 @@ __device__ void lookahead_factor(FrontDev &F, AptpState &S, double (*Wr)[MAX_IB 
     double bml;
 #ifdef RV_PHASE_TIMING
     if (probe) atomicAdd(&g_phase[1][2], clock64() - t0);
-    const int bn = block_factor_wg(Ct, Wr, bp, bp2, bkind, bdiag, boff, nbs, small, &bml, wbv, wbp, wbs,
-                                   Wr + MAX_IB, probe);
+#endif
+    const int bn = block_factor_wg(Ct, Wr, bp, bp2, bkind, bdiag, boff, nbs, small, &bml, wbv, wbp, Wr + MAX_IB);
+#ifdef RV_PHASE_TIMING
     if (probe) atomicAdd(&g_phase[1][3], clock64() - t0);
-#else
-    const int bn = block_factor_wg(Ct, Wr, bp, bp2, bkind, bdiag, boff, nbs, small, &bml, wbv, wbp, wbs,
-                                   Wr + MAX_IB);
 #endif
     double (*blk)[MAX_IB + 1] = Ct;
     if (tid < bn && bkind[tid] == 2) blk[tid + 1][tid] = 0.0;
@@ -1678,8 +1675,8 @@ struct ChainLeaderLds {
     int bp[MAX_IB], bp2[MAX_IB], nbp[MAX_IB], operm[MAX_IB], noperm[MAX_IB];
     int8_t bkind[MAX_IB], nbkind[MAX_IB];
     double bdiag[MAX_IB], boff[MAX_IB], dinv[MAX_IB], nbdiag[MAX_IB], nboff[MAX_IB];
-    double wbv[8], wbs[24];
-    int wbp[8];
+    double wbv[1];
+    int wbp[1];
     int sa[MAX_IB], sb[MAX_IB], U[2 * MAX_IB], src[2 * MAX_IB], ptmp[2 * MAX_IB];
     int nsw, cnt, s_end, s_fail, s_upd;
 };
@@ -1757,7 +1754,7 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
             lds_barrier();
             double bml;
             bn = block_factor_wg(L.blk, L.Wr, L.bp, L.bp2, L.bkind, L.bdiag, L.boff, bs, small, &bml, L.wbv, L.wbp,
-                                 L.wbs, L.Wr + MAX_IB);
+                                 L.Wr + MAX_IB);
             if (tid < bn && L.bkind[tid] == 2) L.blk[tid + 1][tid] = 0.0;
             lds_barrier();
             if (bn > 0) {
@@ -1836,7 +1833,7 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
             lds_barrier();
             next_tile_update(Lr, Wt, L.Ct, L.bkind, L.bdiag, L.boff, nbs, bs, nv);
             bn2 = block_factor_wg(L.Ct, L.Wr, L.nbp, L.bp2, L.nbkind, L.nbdiag, L.nboff, nbs, small, &bml2, L.wbv,
-                                  L.wbp, L.wbs, L.Wr + MAX_IB);
+                                  L.wbp, L.Wr + MAX_IB);
             if (tid < bn2 && L.nbkind[tid] == 2) L.Ct[tid + 1][tid] = 0.0;
             lds_barrier();
         }
