@@ -1538,6 +1538,21 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t co_rsrc(const gdouble *base) {
 __device__ __forceinline__ double co_ldb(__amdgpu_buffer_rsrc_t r, size_t off) {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)(off * sizeof(double)), 0, 16));
 }
+// The same with the front's own end as the range (rows past a panel's last column would leave
+// it); co_stb drops a store whose offset lies past the range.
+constexpr unsigned CO_OOB = 0x7FFFFFF8u;  // (a column offset added to it stays past the range)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t co_rsrc_front(const gdouble *A, size_t lda, size_t off) {
+    const size_t left = (lda * lda - off) * sizeof(double);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>((const double *)(A + off)), (short)0,
+                                             (int)(left < 0x7FFFFFF0 ? left : 0x7FFFFFF0), 0x00020000);
+}
+__device__ __forceinline__ double co_ldo(__amdgpu_buffer_rsrc_t r, unsigned off) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 16));
+}
+__device__ __forceinline__ void co_stb(__amdgpu_buffer_rsrc_t r, unsigned off, double v) {
+    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, (int)off, 0, 16);
+}
 __device__ __forceinline__ double co_ldd(const double *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1683,7 +1698,7 @@ struct ChainLeaderLds {
 constexpr int CHAIN_LC_COLS = 128;  // trailing columns per round of the panel update
 struct ChainPanelLds {
     double blk[MAX_IB][MAX_IB + 1];      // L11 of the current block
-    double WT[MAX_IB][64 + 1];           // W = L D of a 64-row sub-tile, transposed
+    double WT[2][MAX_IB][64 + 1];        // W = L D of the panel's 64-row sub-tiles, transposed
     union {                              // one at a time, in this order within a sub-tile:
         double LT[MAX_IB][64 + 1];       //   its L in the passed columns, transposed
         double Lc[MAX_IB][MAX_IB + 1];   //   L rows of the failed block rows
@@ -1938,22 +1953,126 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
     }
 }
 
+// A value the compiler has to take as new: address arithmetic formed from it is neither hoisted
+// out of the block loop nor kept from one phase to the next.  (Left to itself the compiler holds
+// some hundred loop-invariant offsets of the unrolled loads and stores below in registers across
+// the loop and spills the data instead: 440 spilled registers, 39 us per substitution.)
+__device__ __forceinline__ int fresh(int x) {
+    __asm__ volatile("" : "+v"(x));
+    return x;
+}
+__device__ __forceinline__ int fresh_uniform(int x) {
+    x = __builtin_amdgcn_readfirstlane(x);
+    __asm__ volatile("" : "+s"(x));
+    return x;
+}
+
+// Columns [c0, c0 + ncol) of the L rows of an update round, transposed into LDS: the loads (cl_load,
+// in flight as long as the caller likes) and the LDS stores.
+constexpr int CHAIN_NL = CHAIN_LC_COLS * MAX_IB / 256;
+__device__ __forceinline__ void cl_load(double (&v)[CHAIN_NL], const gdouble *A, size_t lda, int c0, int ncol, int k,
+                                        int nelim) {
+    // thread: column tid % 128, elimination steps j = tid / 128 + 2 u; outside: past the range, zero
+    static_assert(CHAIN_LC_COLS == 128, "thread layout of a round's L rows");
+    const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + c0 + (size_t)k * lda);
+    const int tid = fresh(threadIdx.x), l8 = fresh_uniform((int)lda * 8);
+    const int cc = tid & 127, jh = tid >> 7;
+    const unsigned off = cc * 8 + jh * l8;
+#pragma unroll
+    for (int u = 0; u < CHAIN_NL; ++u) {
+        const unsigned o = off + 2 * u * l8;
+        v[u] = co_ldo(rb, (cc < ncol && 2 * u + jh < nelim) ? o : CO_OOB);
+    }
+}
+__device__ __forceinline__ void cl_store(const double (&v)[CHAIN_NL], double (*LcT)[CHAIN_LC_COLS + 2]) {
+    const int tid = fresh(threadIdx.x), cc = tid & 127, jh = tid >> 7;
+#pragma unroll
+    for (int u = 0; u < CHAIN_NL; ++u) LcT[2 * u + jh][cc] = v[u];
+}
+
+// Update round: thread (tx, ty) holds rows R0 + tx + 16 i (i < 4) x columns c0 + 4 ty + q + 64 p
+// (q < 4, p < 2) of the front in cv; each sum runs over j ascending from zero.
+__device__ __forceinline__ void cu_load(double (&cv)[4][8], __amdgpu_buffer_rsrc_t rc, size_t lda, bool on = true) {
+    const int tid = fresh(threadIdx.x), l8 = fresh_uniform((int)lda * 8);
+    const int tx = tid & 15, ty = tid >> 4;
+    const unsigned vo = on ? (unsigned)(tx * 8 + 4 * ty * l8) : CO_OOB;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const unsigned o = vo + ((q & 3) + 64 * (q >> 2)) * l8;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) cv[i][q] = co_ldo(rc, o + 128 * i);
+    }
+}
+__device__ __forceinline__ void cu_sums(double (&acc)[4][8], const double (*WT)[64 + 1],
+                                        const double (*LcT)[CHAIN_LC_COLS + 2], int nelim) {
+    const int tid = fresh(threadIdx.x), tx = tid & 15, ty = tid >> 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) acc[i][q] = 0.0;
+    auto step = [&](int j) {
+        double wv[4], lc[8];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) wv[i] = WT[j][tx + 16 * i];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) lc[q] = LcT[j][4 * ty + (q & 3) + 64 * (q >> 2)];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int q = 0; q < 8; ++q) acc[i][q] += wv[i] * lc[q];
+    };
+    if (nelim == MAX_IB) {
+#pragma unroll 4
+        for (int j = 0; j < MAX_IB; ++j) step(j);
+    } else {
+        for (int j = 0; j < nelim; ++j) step(j);
+    }
+}
+// rows >= be below r1, lower triangle; the leader's tile (rows and columns below lead) left out
+__device__ __forceinline__ void cu_store(const double (&cv)[4][8], const double (&acc)[4][8],
+                                         __amdgpu_buffer_rsrc_t rc, size_t lda, int R0, int r1, int c0, int ncol,
+                                         int be, int lead) {
+    const int tid = fresh(threadIdx.x), l8 = fresh_uniform((int)lda * 8);
+    const int tx = tid & 15, ty = tid >> 4;
+    const int vo = tx * 8 + 4 * ty * l8;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const int cc = 4 * ty + (q & 3) + 64 * (q >> 2), col = c0 + cc;
+        const int o = vo + ((q & 3) + 64 * (q >> 2)) * l8;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = R0 + tx + 16 * i;
+            const bool ok = r >= be && r < r1 && cc < ncol && r >= col && !(r < lead && col < lead);
+            co_stb(rc, ok ? (unsigned)(o + 128 * i) : CO_OOB, cv[i][q] - acc[i][q]);
+        }
+    }
+}
+
 // Panel rows of chunk c: [ob_start + c * CH, min(ob_start + (c + 1) * CH, m)).
+//
+// The chain of one inner block through a panel is latency: device-scope loads of 1-3 us each and
+// the signals between workgroups.  With one chunk per panel (every level without delays) and no
+// failed column, W = L D goes from the substitution's registers straight to LDS, the columns to
+// update are loaded before the wait for the other panels' checks, the L rows of the second round
+// of columns during the first round's products, and the row permutation of earlier columns runs
+// after the panel has reported: a block's update takes 16.4 us from 28.4 (64^3 Helmholtz), 10.8
+// from 21.8 (40^3).
 template <int CH>
 __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync &C, ChainPanelLds &L, int pidx, int NP, int nit,
                             int ib, double threshold) {
     static_assert(CH == 64 || CH == 128, "panel rows per workgroup: 64 or 128 (the apply's LDS rows)");
 
-    const int tid = threadIdx.x;
     const int m = F.m;
-    const size_t lda = m;
     gdouble *A = gbl(F.F);
     gdouble *const bk = gbl(S.backup);
     const int ob_start = S.ob_start, obe = S.ob_start + S.ob_cols;
     const int nchunk = (m - ob_start + CH - 1) / CH;
+    const bool single = nchunk <= NP;  // at most one chunk per panel
     const double bound = 1.0 / threshold;
     for (int it = 0; it < nit; ++it) {
         if (!chain_wait(&C.rec.v, it + 1, &C.err.v)) return;
+        const int tid = fresh(threadIdx.x);
+        const size_t lda = (size_t)(unsigned)fresh_uniform(m);
         const ChainRec &R = C.recs[it];
         if (tid < MAX_IB) {
             L.bp[tid] = co_ldi(&R.bperm[tid]);
@@ -1971,52 +2090,60 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
         const int k = __builtin_amdgcn_readfirstlane(L.rec[0]), bs = __builtin_amdgcn_readfirstlane(L.rec[1]);
         const int bn = __builtin_amdgcn_readfirstlane(L.rec[2]), end_pos = __builtin_amdgcn_readfirstlane(L.rec[3]);
         const int be = k + bs;
+        // the panel's one chunk has rows below the block: its update takes the short path when
+        // the block has no failed column
+        const int r0p = ob_start + pidx * CH, r1p = min(r0p + CH, m);
+        const bool fast = single && pidx < nchunk && r1p > be && bn == bs;
+        double pml = 0.0;  // (fast) the row's largest |l|
         if (bn > 0) {
+            // L11 and the first chunk's rows, all loads in flight together
+            double v[MAX_IB / 8];
             {
                 const int i = tid & (MAX_IB - 1), j0 = tid / MAX_IB;
                 const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + k + (size_t)k * lda);
-                double v[MAX_IB / 8];
 #pragma unroll
                 for (int u = 0; u < MAX_IB / 8; ++u) {
                     const int j = j0 + 8 * u;
-                    const double x = co_ldb(rb, (size_t)min(i, bs - 1) + (size_t)min(j, bs - 1) * lda);
-                    v[u] = (i < bs && j < i) ? x : 0.0;
+                    v[u] = co_ldo(rb, (i < bs && j < i) ? 8u * (i + j * (unsigned)lda) : CO_OOB);
                 }
+            }
+            // a row's block entries in column order (zeros outside the front's live rows and
+            // beyond the block, by the resource's range)
+            double yn[MAX_IB];
+            auto load_rows = [&](int c) {
+                const int r = ob_start + c * CH + tid, l8 = fresh_uniform((int)lda * 8), nb = fresh_uniform(bs);
+                const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + (size_t)k * lda);
+                const unsigned off = (tid < CH && r >= be && r < m) ? 8u * r : CO_OOB;
+#pragma unroll
+                for (int j = 0; j < MAX_IB; ++j) yn[j] = co_ldo(rb, j < nb ? off + min(j, nb) * l8 : CO_OOB);
+            };
+            load_rows(pidx);
+            {
+                const int i = tid & (MAX_IB - 1), j0 = tid / MAX_IB;
 #pragma unroll
                 for (int u = 0; u < MAX_IB / 8; ++u) L.blk[i][j0 + 8 * u] = v[u];
+                pivots_dinv(L.bkind, L.bdiag, L.boff, L.dinv, bn);
+                lds_barrier();
             }
-            pivots_dinv(L.bkind, L.bdiag, L.boff, L.dinv, bn);
-            lds_barrier();
             for (int c = pidx; c < nchunk; c += NP) {
                 const int r0 = ob_start + c * CH, r1 = min(r0 + CH, m);
+                if (c != pidx) load_rows(c);
                 if (r1 <= be || tid >= CH) continue;
                 // (wavefront-uniform: CH is a multiple of 64)
                 const int r = r0 + tid;
                 const bool live = r >= be && r < r1;
                 double y[MAX_IB];
                 {
-                    // the row's block entries in column order (one base, constant offsets; rows
-                    // clamped into the front, unused values discarded), backed up as they are
-                    // (restore_diagonal_with_perm reads the backup in column order), then
-                    // gathered into pivot order through the wavefront's own LDS rows
-                    const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + (size_t)k * lda);
-                    const size_t ro = (size_t)min(r, m - 1);
-                    double yn[MAX_IB];
+                    // backed up as they are (restore_diagonal_with_perm reads the backup in
+                    // column order), then gathered into pivot order through the wavefront's own
+                    // LDS rows
+                    {
+                        const __amdgpu_buffer_rsrc_t rb = co_rsrc(bk);
+                        const int l8 = fresh_uniform((int)lda * 8), nb = fresh_uniform(bs);
+                        const unsigned off = live ? 8u * (r - k) : CO_OOB;
 #pragma unroll
-                    for (int j = 0; j < MAX_IB; ++j) {
-                        const double v = co_ldb(rb, ro + (size_t)j * lda);
-                        yn[j] = (live && j < bs) ? v : 0.0;
-                    }
-                    if (live) {
-                        gdouble *brow = bk + (r - k);
-                        if (bs == MAX_IB) {
-#pragma unroll
-                            for (int j = 0; j < MAX_IB; ++j) co_st(brow + (size_t)j * lda, yn[j]);
-                        } else {
-#pragma unroll
-                            for (int j = 0; j < MAX_IB; ++j)
-                                if (j < bs) co_st(brow + (size_t)j * lda, yn[j]);
-                        }
+                        for (int j = 0; j < MAX_IB; ++j)
+                            if (j < nb) co_stb(rb, off + min(j, nb) * l8, yn[j]);
                     }
                     double *yb = L.Yb[tid];
 #pragma unroll
@@ -2028,16 +2155,15 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
                 }
                 panel_trsm_d(y, L.blk, bn, L.bkind, L.dinv, L.bdiag, L.boff);
                 int first = INT_MAX;
+                {
+                    const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + (size_t)k * lda);
+                    const int l8 = fresh_uniform((int)lda * 8), nb = fresh_uniform(bs);
+                    const unsigned off = live ? 8u * r : CO_OOB;
+#pragma unroll
+                    for (int j = 0; j < MAX_IB; ++j)
+                        if (j < nb) co_stb(rb, off + min(j, nb) * l8, y[j]);
+                }
                 if (live) {
-                    gdouble *row = A + r;
-                    if (bs == MAX_IB) {
-#pragma unroll
-                        for (int j = 0; j < MAX_IB; ++j) co_st(row + (size_t)(k + j) * lda, y[j]);
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < MAX_IB; ++j)
-                            if (j < bs) co_st(row + (size_t)(k + j) * lda, y[j]);
-                    }
 #pragma unroll
                     for (int q = MAX_IB - 1; q >= 0; --q)
                         if (q < bn && fabs(y[q]) >= bound) first = q;
@@ -2045,27 +2171,80 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
                 }
                 first = wave_min_int(first);
                 if ((tid & 63) == 0 && first != INT_MAX) atomicMin(&C.applied[it].aux, first);
+                if (fast) {
+                    // W = L D (compute_ld_into factor.rs:1536-1563) of the row, used if no column fails
+                    const int lc = tid & 31;
+                    const int kdl = L.bkind[lc];
+                    const double bdl = L.bdiag[lc], bol = L.boff[lc];
+                    double (*WT)[64 + 1] = L.WT[tid >> 6];
+#pragma unroll
+                    for (int j = 0; j < MAX_IB; ++j) {
+                        const int kd = __builtin_amdgcn_readlane(kdl, j);
+                        const double dj = readlane_f64(bdl, j);
+                        double w = y[j] * dj;
+                        if (kd == 2 && j + 1 < MAX_IB) w = w + y[j + 1 < MAX_IB ? j + 1 : j] * readlane_f64(bol, j);
+                        if (kd == 3 && j > 0) w = y[j > 0 ? j - 1 : 0] * readlane_f64(bol, j > 0 ? j - 1 : 0) + w;
+                        WT[j][tid & 63] = (kd == 0) ? 0.0 : w;
+                        pml = max_abs(pml, y[j]);
+                    }
+                }
             }
         }
         stores_done_barrier();
         if (tid == 0) __hip_atomic_fetch_add(&C.applied[it].v, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // (fast) the first round's columns of the first sub-tile: this panel's own rows
+        double cv[4][8];
+        const int R0f = (r0p + 63 < be) ? r0p + 64 : r0p;  // first sub-tile with rows below the block
+        __amdgpu_buffer_rsrc_t rc = co_rsrc_front(A, lda, (size_t)min(R0f, m - 1) + (size_t)min(be, m - 1) * lda);
+        cu_load(cv, rc, lda, fast && be < obe);
         if (!chain_wait_aux(C.applied[it], NP, &C.err.v, &L.s_fail)) return;
+        int permute_from = -1;
         if (bn > 0) {
             int nelim = min(L.s_fail, bn);
             if (nelim > 0 && L.bkind[nelim - 1] == 2) nelim -= 1;
             nelim = __builtin_amdgcn_readfirstlane(nelim);
             const int nbs = min(end_pos - be, ib);
             const bool ahead = nelim == bs && nbs > 0 && it + 1 < nit;
+            const int lead = ahead ? be + nbs : be;
             const int nf = bs - nelim;
             double ml = 0.0;
+            // a panel without rows below the block has nothing to do when no column failed
+            const bool idle = single && nf == 0 && (pidx >= nchunk || r1p <= be);
+            if (fast && nf == 0) {
+                ml = pml;
+                // rounds (sub-tile, 128 columns); a round's columns are loaded at the end of the one
+                // before it
+                int R0 = R0f, c0 = be;
+                double lv[CHAIN_NL];
+                cl_load(lv, A, lda, be, min(CHAIN_LC_COLS, obe - be), k, nelim);
+                while (R0 < r1p && c0 < obe) {
+                    const int ncol = min(CHAIN_LC_COLS, obe - c0);
+                    int R1 = R0, c1 = c0 + CHAIN_LC_COLS;
+                    if (c1 >= obe || R0 + 63 < c1) { R1 = R0 + 64; c1 = be; }  // no row reaches the columns from c1
+                    const bool more = R1 < r1p;
+                    __syncthreads();  // the previous round's LDS reads are done
+                    cl_store(lv, L.LcT);
+                    cl_load(lv, A, lda, more ? c1 : be, more ? min(CHAIN_LC_COLS, obe - c1) : 0, k, nelim);
+                    __syncthreads();
+                    double acc[4][8];
+                    cu_sums(acc, L.WT[(R0 - r0p) >> 6], L.LcT, nelim);
+                    cu_store(cv, acc, rc, lda, R0, r1p, c0, ncol, be, lead);
+                    R0 = R1;
+                    c0 = c1;
+                    if (!more) break;
+                    rc = co_rsrc_front(A, lda, (size_t)R0 + (size_t)c0 * lda);
+                    cu_load(cv, rc, lda);
+                }
+            }
             // 64-row sub-tiles of the panel's rows at or below the block
-            for (int c = pidx; c < nchunk; c += NP) {
+            for (int c = (fast && nf == 0) || idle ? nchunk : pidx; c < nchunk; c += NP) {
                 const int r0c = ob_start + c * CH, r1 = min(r0c + CH, m);
                 for (int R0 = r0c; R0 < r1; R0 += 64) {
                     if (R0 + 64 <= k) continue;  // (uniform)
                     __syncthreads();             // the previous sub-tile's LDS reads are done
                     // L rows of the sub-tile in the passed columns -> LT[j][row]; W = L D
                     // (ld_entry, compute_ld_into factor.rs:1536-1563) -> WT[j][row]
+                    double (*WT)[64 + 1] = L.WT[0];
                     {
                         const int rr = tid & 63, jg = tid >> 6, r = R0 + rr;
                         const bool valid = r >= k && r < r1;
@@ -2099,7 +2278,7 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
                             const double v2 = lj * dj + L.LT[j + 1 < MAX_IB ? j + 1 : j][rr] * L.boff[j];
                             const double v3 = L.LT[j > 0 ? j - 1 : 0][rr] * L.boff[j > 0 ? j - 1 : 0] + lj * dj;
                             const double v = (kd == 1) ? v1 : (kd == 2) ? v2 : (kd == 3) ? v3 : 0.0;
-                            L.WT[j][rr] = (j < nelim) ? v : 0.0;
+                            WT[j][rr] = (j < nelim) ? v : 0.0;
                         }
                     }
                     __syncthreads();
@@ -2141,7 +2320,7 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
                                     const int jf = j - nelim;
                                     if (r >= be || r - k - nelim >= jf) {
                                         double sx = 0.0;
-                                        for (int c2 = 0; c2 < nelim; ++c2) sx += L.WT[c2][rr] * L.Lc[jf][c2];
+                                        for (int c2 = 0; c2 < nelim; ++c2) sx += WT[c2][rr] * L.Lc[jf][c2];
                                         if (!have_v) v = co_ld(row + cj);
                                         v = v - sx;
                                         have_v = true;
@@ -2151,118 +2330,62 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
                             }
                         }
                     }
-                    // trailing columns of the outer block, CHAIN_LC_COLS per round: thread (tx, ty)
-                    // forms rows R0 + tx + 16 i (i < 4) x columns c0 + 4 ty + q + 64 p (q < 4,
-                    // p < 2), each sum over j ascending from zero, subtracted once; the round's
-                    // L rows staged transposed in LDS
+                    // trailing columns of the outer block, CHAIN_LC_COLS per round, the round's L
+                    // rows staged transposed in LDS
                     if (nelim == 0 || R0 + 63 < be) continue;  // (uniform)
-                    const int tx = tid & 15, ty = tid >> 4;
                     for (int c0 = be; c0 < obe; c0 += CHAIN_LC_COLS) {
                         const int ncol = min(CHAIN_LC_COLS, obe - c0);
                         if (R0 + 63 < c0) break;  // (uniform) no row of the sub-tile reaches them
                         __syncthreads();
+                        rc = co_rsrc_front(A, lda, (size_t)R0 + (size_t)c0 * lda);
                         {
-                            constexpr int NL = CHAIN_LC_COLS * MAX_IB / 256;
-                            double v[NL];
-                            const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + c0 + (size_t)k * lda);
-#pragma unroll
-                            for (int u = 0; u < NL; ++u) {
-                                const int e = tid + 256 * u, cc = e % CHAIN_LC_COLS, j = e / CHAIN_LC_COLS;
-                                const double x = co_ldb(rb, (size_t)(cc < ncol ? cc : 0) + (size_t)(j < nelim ? j : 0) * lda);
-                                v[u] = (cc < ncol && j < nelim) ? x : 0.0;
-                            }
-#pragma unroll
-                            for (int u = 0; u < NL; ++u) {
-                                const int e = tid + 256 * u;
-                                L.LcT[e / CHAIN_LC_COLS][e % CHAIN_LC_COLS] = v[u];
-                            }
+                            double lv[CHAIN_NL];
+                            cl_load(lv, A, lda, c0, ncol, k, nelim);
+                            cl_store(lv, L.LcT);
                         }
                         __syncthreads();
-                        double acc[4][8];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-#pragma unroll
-                            for (int q = 0; q < 8; ++q) acc[i][q] = 0.0;
-                        if (nelim == MAX_IB) {
-#pragma unroll 4
-                            for (int j = 0; j < MAX_IB; ++j) {
-                                double wv[4], lc[8];
-#pragma unroll
-                                for (int i = 0; i < 4; ++i) wv[i] = L.WT[j][tx + 16 * i];
-#pragma unroll
-                                for (int q = 0; q < 8; ++q) lc[q] = L.LcT[j][4 * ty + (q & 3) + 64 * (q >> 2)];
-#pragma unroll
-                                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                                    for (int q = 0; q < 8; ++q) acc[i][q] += wv[i] * lc[q];
-                            }
-                        } else {
-                            for (int j = 0; j < nelim; ++j) {
-                                double wv[4], lc[8];
-#pragma unroll
-                                for (int i = 0; i < 4; ++i) wv[i] = L.WT[j][tx + 16 * i];
-#pragma unroll
-                                for (int q = 0; q < 8; ++q) lc[q] = L.LcT[j][4 * ty + (q & 3) + 64 * (q >> 2)];
-#pragma unroll
-                                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                                    for (int q = 0; q < 8; ++q) acc[i][q] += wv[i] * lc[q];
-                            }
-                        }
-                        const __amdgpu_buffer_rsrc_t rbc = co_rsrc(A + R0 + (size_t)c0 * lda);
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int r = R0 + tx + 16 * i;
-                            gdouble *row = A + r;
-                            double cv[8];
-                            bool ok[8];
-#pragma unroll
-                            for (int q = 0; q < 8; ++q) {
-                                const int cc = 4 * ty + (q & 3) + 64 * (q >> 2), col = c0 + cc;
-                                const bool tile_ahead = ahead && r < be + nbs && col < be + nbs;
-                                ok[q] = r >= be && r < r1 && cc < ncol && r >= col && !tile_ahead;
-                                const double x = co_ldb(rbc, (size_t)(min(r, m - 1) - R0) + (size_t)(cc < ncol ? cc : 0) * lda);
-                                cv[q] = ok[q] ? x : 0.0;
-                            }
-#pragma unroll
-                            for (int q = 0; q < 8; ++q) {
-                                const int col = c0 + 4 * ty + (q & 3) + 64 * (q >> 2);
-                                if (ok[q]) co_st(row + (size_t)col * lda, cv[q] - acc[i][q]);
-                            }
-                        }
+                        double cs[4][8], acc[4][8];
+                        cu_load(cs, rc, lda);
+                        cu_sums(acc, WT, L.LcT, nelim);
+                        cu_store(cs, acc, rc, lda, R0, r1, c0, ncol, be, lead);
                     }
                 }
             }
             ml = wave_fmax(ml);
             if ((tid & 63) == 0) atomic_max_nonneg(&F.max_l_bits, ml);
-            // block rows permuted in the columns factored before this block, this panel's share
-            {
-                const int per = (k + NP - 1) / NP;
-                const int cb = pidx * per, ce = min(k, cb + per);
-                const int i = tid & 31, half = (tid >> 5) & 1, wv = tid >> 6;
-                if (i < bs) {
-                    const int sr = L.bp[i];
-                    // 128 columns per step, all loads issued before the stores
-                    for (int cs = cb; cs < ce; cs += 128) {
-                        const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + k + (size_t)cs * lda);
-                        double v[16];
+            permute_from = nf;
+        }
+        // block rows permuted in the columns factored before this block, this panel's share: with
+        // failed columns before the panel reports (the leader then moves some of these rows), else
+        // after (the rows are final)
+        auto permute_rows = [&] {
+            const int per = (k + NP - 1) / NP;
+            const int cb = pidx * per, ce = min(k, cb + per);
+            const int i = tid & 31, half = (tid >> 5) & 1, wv = tid >> 6;
+            if (i < bs) {
+                const int sr = L.bp[i];
+                // 128 columns per step, all loads issued before the stores
+                for (int cs = cb; cs < ce; cs += 128) {
+                    const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + k + (size_t)cs * lda);
+                    double v[16];
 #pragma unroll
-                        for (int u = 0; u < 16; ++u) {
-                            const int cc = 2 * wv + half + 8 * u;  // column cs + cc
-                            const double x = co_ldb(rb, (size_t)sr + (size_t)(cs + cc < ce ? cc : 0) * lda);
-                            v[u] = x;
-                        }
+                    for (int u = 0; u < 16; ++u) {
+                        const int cc = 2 * wv + half + 8 * u;  // column cs + cc
+                        const double x = co_ldb(rb, (size_t)sr + (size_t)(cs + cc < ce ? cc : 0) * lda);
+                        v[u] = x;
+                    }
 #pragma unroll
-                        for (int u = 0; u < 16; ++u) {
-                            const int c = cs + 2 * wv + half + 8 * u;
-                            if (c < ce) co_st(A + (k + i) + (size_t)c * lda, v[u]);
-                        }
+                    for (int u = 0; u < 16; ++u) {
+                        const int c = cs + 2 * wv + half + 8 * u;
+                        if (c < ce) co_st(A + (k + i) + (size_t)c * lda, v[u]);
                     }
                 }
             }
-        }
+        };
+        if (permute_from > 0) permute_rows();
         stores_done_barrier();
         if (tid == 0) __hip_atomic_fetch_add(&C.updated[it].v, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (permute_from == 0) permute_rows();
     }
 }
 
