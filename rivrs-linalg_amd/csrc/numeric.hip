@@ -629,9 +629,12 @@ __device__ __forceinline__ int block_pivots(const double (*blk)[MAX_IB + 1], dou
 
 // All 256 threads: the block in blk (lower triangle) on entry; the factored block in position
 // order on return (D's off-diagonal of a 2x2 at (q + 1, q)).  blk2, lbuf, bp2: working LDS.
+// Wavefronts 1 to 3 call `beside` while the first runs the pivot steps.
+template <class Beside>
 __device__ __forceinline__ int block_factor_wg(double (*blk)[MAX_IB + 1], double (*blk2)[MAX_IB + 1], int *bp, int *bp2,
                                                int8_t *bkind, double *bdiag, double *boff, int bs, double small,
-                                               double *maxl, double *wbv, int *wbp, double (*lbuf)[MAX_IB + 1]) {
+                                               double *maxl, double *wbv, int *wbp, double (*lbuf)[MAX_IB + 1],
+                                               Beside beside) {
     const int tid = threadIdx.x;
     double *S = &blk2[0][0];
     if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) {
@@ -640,6 +643,8 @@ __device__ __forceinline__ int block_factor_wg(double (*blk)[MAX_IB + 1], double
         const int kk = block_pivots(blk, S, bp, bp2, bkind, bdiag, boff, bs, small, &ml, lbuf);
         __builtin_amdgcn_s_setprio(0);
         if (tid == 0) { wbv[0] = ml; wbp[0] = kk; }
+    } else {
+        beside();
     }
     lds_barrier();
     const int kk = __builtin_amdgcn_readfirstlane(wbp[0]);
@@ -872,7 +877,7 @@ __global__ __launch_bounds__(256) void k_block_apply(FrontDev *__restrict__ fr,
     lds_barrier();
     RV_PHASE(0, 1);
     double bml;
-    bn = block_factor_wg(blk, blk2, bp, bp2, bkind, bdiag, boff, bs, small, &bml, wbv, wbp, lbuf);
+    bn = block_factor_wg(blk, blk2, bp, bp2, bkind, bdiag, boff, bs, small, &bml, wbv, wbp, lbuf, [] {});
     RV_PHASE(0, 2);
     // D off-diagonals of 2x2 pivots read as zeros of L11 (factor.rs:1898-1912)
     if (tid < bn) {
@@ -1144,7 +1149,8 @@ __device__ void lookahead_factor(FrontDev &F, AptpState &S, double (*Wr)[MAX_IB 
 #ifdef RV_PHASE_TIMING
     if (probe) atomicAdd(&g_phase[1][2], clock64() - t0);
 #endif
-    const int bn = block_factor_wg(Ct, Wr, bp, bp2, bkind, bdiag, boff, nbs, small, &bml, wbv, wbp, Wr + MAX_IB);
+    const int bn = block_factor_wg(Ct, Wr, bp, bp2, bkind, bdiag, boff, nbs, small, &bml, wbv, wbp, Wr + MAX_IB,
+                                   [] {});
 #ifdef RV_PHASE_TIMING
     if (probe) atomicAdd(&g_phase[1][3], clock64() - t0);
 #endif
@@ -1486,6 +1492,7 @@ struct ChainRec {
     int bperm[MAX_IB];
     int bkind[MAX_IB];
     double bdiag[MAX_IB], boff[MAX_IB];
+    double l11[MAX_IB * MAX_IB];  // strictly lower part, zeros elsewhere, column-major
 };
 // Every counter on a cache line of its own: the waits poll them from many workgroups at once,
 // and a line shared by several counters would queue every poll and update behind the others.
@@ -1499,8 +1506,9 @@ struct alignas(128) ChainCounter {
 struct ChainSync {
     ChainCounter rec;                       // inner-block records published by the leader
     ChainCounter err;                       // a wait of this front ran out
-    ChainCounter applied[CHAIN_MAX_IT];     // panels done with the check of block it; aux: its
-                                            // first failing column (INT_MAX before)
+    ChainCounter applied[CHAIN_MAX_IT];     // panels done with the check of block it, and the two
+                                            // wavefronts of the leader that store its tile; aux:
+                                            // its first failing column (INT_MAX before)
     ChainCounter updated[CHAIN_MAX_IT];     // panels done with the updates of block it
     ChainRec recs[CHAIN_MAX_IT];
 };
@@ -1626,6 +1634,166 @@ __device__ __forceinline__ bool chain_wait_aux(ChainCounter &c, int target, int 
     return ok;
 }
 
+// A value the compiler has to take as new: address arithmetic formed from it is neither hoisted
+// out of the block loop nor kept from one phase to the next.  (Left to itself the compiler holds
+// some hundred loop-invariant offsets of the unrolled loads and stores below in registers across
+// the loop and spills the data instead: 440 spilled registers, 39 us per substitution.)
+__device__ __forceinline__ int fresh(int x) {
+    __asm__ volatile("" : "+v"(x));
+    return x;
+}
+__device__ __forceinline__ int fresh_uniform(int x) {
+    x = __builtin_amdgcn_readfirstlane(x);
+    __asm__ volatile("" : "+s"(x));
+    return x;
+}
+
+// One wavefront: wait until c.v >= target; *aux receives the aux read with it.  False when the
+// front's wait ran out.
+__device__ __forceinline__ bool wave_poll(ChainCounter &c, int target, int *err, int *aux) {
+    long long it = 0;
+    for (;;) {
+        const unsigned long long w =
+            __hip_atomic_load((unsigned long long *)&c.v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int v = __builtin_amdgcn_readfirstlane((int)(unsigned)(w & 0xffffffffu));
+        *aux = __builtin_amdgcn_readfirstlane((int)(unsigned)(w >> 32));
+        if (v >= target) return true;
+        if ((++it & 63) == 0 && (it > CHAIN_SPIN_LIMIT || __builtin_amdgcn_readfirstlane(co_ldi(err)))) {
+            if ((threadIdx.x & 63) == 0) atomicOr(err, 1);
+            return false;
+        }
+        __builtin_amdgcn_s_sleep(4);
+        __asm__ volatile("" ::: "memory");
+    }
+}
+
+// Substitution with L11 and D^-1 (factor.rs:1295-1408), four lanes per panel row: lane h of a
+// row's quad holds columns 4 t + h, t = 0 .. 7, so the serial chain of 496 multiply-subtract
+// pairs per row runs four columns wide and a panel's 64 rows fill the workgroup's four
+// wavefronts (one row per lane kept one wavefront busy: 4 us against 1).  Every column receives
+// its terms in ascending order, as the row form.
+template <int CTRL>
+__device__ __forceinline__ double quad_perm(double v) { return dpp_f64<CTRL>(v); }
+
+template <int I, bool FULL>
+struct QuadStep {
+    static __device__ __forceinline__ void load(double (&c)[8], const double (*blk)[MAX_IB + 1], int h) {
+#pragma unroll
+        for (int t = I >> 2; t < 8; ++t) c[t] = blk[4 * t + h][I];
+    }
+    static __device__ __forceinline__ void run(double (&y)[8], const double (*blk)[MAX_IB + 1], int h, int bn,
+                                               const double (&c0)[8], const double (&c1)[8]) {
+        if constexpr (I < MAX_IB - 1) {
+            if (!FULL && I >= bn) return;
+            double c2[8];
+            if constexpr (I + 2 < MAX_IB - 1) QuadStep<I + 2, FULL>::load(c2, blk, h);
+            const double yi = quad_perm<(I & 3) * 0x55>(y[I >> 2]);
+            double p[8];
+#pragma unroll
+            for (int t = I >> 2; t < 8; ++t) p[t] = c0[t] * yi;
+#pragma unroll
+            for (int t = I >> 2; t < 8; ++t) {
+                const double v = y[t] - p[t];
+                const bool upd = (t > (I >> 2) || h > (I & 3)) && (FULL || 4 * t + h < bn);
+                y[t] = upd ? v : y[t];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            QuadStep<I + 1, FULL>::run(y, blk, h, bn, c1, c2);
+        }
+    }
+};
+
+// A block's pivots as the substitution takes them: y g for a 1x1; (y a - z b) g for a 2x2, z the
+// row's entry of the other column; W = L D is l d, or l d + z b.
+struct PivotCoef {
+    double a[MAX_IB], b[MAX_IB], g[MAX_IB], d[MAX_IB];
+    int kd[MAX_IB];
+    int has2;
+};
+// (the first wavefront; bkind .. boff in LDS)
+__device__ __forceinline__ void pivot_coefs(const int8_t *bkind, const double *bdiag, const double *boff, int bn,
+                                            PivotCoef &P) {
+    const int c = threadIdx.x & 31;
+    const int kd = c < bn ? bkind[c] : 0;
+    const int f = (kd == 3 && c > 0) ? c - 1 : c, s = min(f + 1, MAX_IB - 1);  // columns of a 2x2
+    const double d = bdiag[c], df = bdiag[f], ds = bdiag[s], of = boff[f];
+    const double den = kd == 1 ? d : df * ds - of * of;
+    const double g = 1.0 / den;
+    const unsigned long long two = __ballot(kd >= 2);
+    if (threadIdx.x < MAX_IB) {
+        P.a[c] = kd == 2 ? ds : df;
+        P.b[c] = of;
+        P.g[c] = g;
+        P.d[c] = d;
+        P.kd[c] = kd;
+        if (c == 0) P.has2 = two != 0;
+    }
+}
+
+// z[t]: the entry of the other column of a 2x2 pivot (kinds kd[t])
+__device__ __forceinline__ void quad_partner(const double (&y)[8], const int (&kd)[8], int h, double (&z)[8]) {
+    double up[8], dn[8];  // lane h's neighbours: column c + 1 and c - 1
+#pragma unroll
+    for (int t = 0; t < 8; ++t) { up[t] = quad_perm<0x39>(y[t]); dn[t] = quad_perm<0x93>(y[t]); }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        const double u = (h == 3) ? (t < 7 ? up[t < 7 ? t + 1 : 7] : 0.0) : up[t];
+        const double l = (h == 0) ? (t > 0 ? dn[t > 0 ? t - 1 : 0] : 0.0) : dn[t];
+        z[t] = (kd[t] == 2) ? u : l;
+    }
+}
+
+__device__ __forceinline__ void quad_substitute(double (&y)[8], const double (*blk)[MAX_IB + 1], int bn,
+                                                const PivotCoef &P) {
+    const int h = fresh(threadIdx.x) & 3;
+    double c0[8], c1[8];
+    if (bn == MAX_IB) {
+        QuadStep<0, true>::load(c0, blk, h);
+        QuadStep<1, true>::load(c1, blk, h);
+        QuadStep<0, true>::run(y, blk, h, bn, c0, c1);
+    } else {
+        QuadStep<0, false>::load(c0, blk, h);
+        QuadStep<1, false>::load(c1, blk, h);
+        QuadStep<0, false>::run(y, blk, h, bn, c0, c1);
+    }
+    int kd[8];
+    double g[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) { kd[t] = P.kd[4 * t + h]; g[t] = P.g[4 * t + h]; }
+    if (P.has2) {
+        double z[8];
+        quad_partner(y, kd, h, z);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const double v = y[t] * P.a[4 * t + h] - z[t] * P.b[4 * t + h];
+            y[t] = (kd[t] >= 2) ? v * g[t] : (kd[t] == 1) ? y[t] * g[t] : y[t];
+        }
+    } else {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) y[t] = (kd[t] == 1) ? y[t] * g[t] : y[t];
+    }
+}
+
+// W = L D of the row's entries (compute_ld_into factor.rs:1536-1563)
+__device__ __forceinline__ void quad_ld(const double (&y)[8], const PivotCoef &P, double (&w)[8]) {
+    const int h = fresh(threadIdx.x) & 3;
+    int kd[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        kd[t] = P.kd[4 * t + h];
+        w[t] = (kd[t] != 0) ? y[t] * P.d[4 * t + h] : 0.0;
+    }
+    if (P.has2) {
+        double z[8];
+        quad_partner(y, kd, h, z);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const double v = w[t] + z[t] * P.b[4 * t + h];
+            w[t] = (kd[t] >= 2) ? v : w[t];
+        }
+    }
+}
+
 // Symmetric line permutation (apply_swaps) with device-scope accesses to the front.
 __device__ __forceinline__ void apply_swaps_co(FrontDev &F, AptpState &S, const int *sa, const int *sb, int nsw, int *U, int *src,
                                int *cnt, int *ptmp) {
@@ -1686,14 +1854,18 @@ __device__ __forceinline__ void apply_swaps_co(FrontDev &F, AptpState &S, const 
 struct ChainLeaderLds {
     double blk[MAX_IB][MAX_IB + 1];      // the current block, factored (L11)
     double Ct[MAX_IB][MAX_IB + 1];       // the next block's tile, factored ahead
+    double Nv[MAX_IB][MAX_IB + 1];       // that tile before its factorization
     double Wr[2 * MAX_IB][MAX_IB + 1];   // next block's L rows and W, then the factor's buffers
+    double Yn[MAX_IB][MAX_IB + 1];       // next block's rows in the current block's columns
+    double Cn[MAX_IB][MAX_IB + 1];       // next block's tile as it stands
     int bp[MAX_IB], bp2[MAX_IB], nbp[MAX_IB], operm[MAX_IB], noperm[MAX_IB];
     int8_t bkind[MAX_IB], nbkind[MAX_IB];
-    double bdiag[MAX_IB], boff[MAX_IB], dinv[MAX_IB], nbdiag[MAX_IB], nboff[MAX_IB];
+    double bdiag[MAX_IB], boff[MAX_IB], nbdiag[MAX_IB], nboff[MAX_IB];
+    PivotCoef pc;
     double wbv[1];
     int wbp[1];
     int sa[MAX_IB], sb[MAX_IB], U[2 * MAX_IB], src[2 * MAX_IB], ptmp[2 * MAX_IB];
-    int nsw, cnt, s_end, s_fail, s_upd;
+    int nsw, cnt, s_end, s_fail, s_upd, s_pf, s_err;
 };
 constexpr int CHAIN_LC_COLS = 128;  // trailing columns per round of the panel update
 struct ChainPanelLds {
@@ -1703,11 +1875,12 @@ struct ChainPanelLds {
         double LT[MAX_IB][64 + 1];       //   its L in the passed columns, transposed
         double Lc[MAX_IB][MAX_IB + 1];   //   L rows of the failed block rows
         double LcT[MAX_IB][CHAIN_LC_COLS + 2];  // L rows of a round's columns, transposed
-        double Yb[128][MAX_IB + 1];      // (apply) panel rows in column order, by thread
+        double Yb[64][MAX_IB + 1];       // (apply) rows of a sub-tile in column order
     };
     int bp[MAX_IB];
     int8_t bkind[MAX_IB];
-    double bdiag[MAX_IB], boff[MAX_IB], dinv[MAX_IB];
+    double bdiag[MAX_IB], boff[MAX_IB];
+    PivotCoef pc;
     int rec[4];
     int s_fail;
 };
@@ -1716,16 +1889,66 @@ union ChainLds {
     ChainPanelLds pn;
 };
 
-__device__ __forceinline__ void pivots_dinv(const int8_t *bkind, const double *bdiag, const double *boff,
-                                            double *dinv, int bn) {
+// A block's record (all threads; complete once every thread's stores are).
+__device__ __forceinline__ void write_record(ChainRec &R, int k, int bs, int bn, int end_pos, const int *bp,
+                                             const int8_t *bkind, const double *bdiag, const double *boff,
+                                             const double (*blk)[MAX_IB + 1]) {
     const int tid = threadIdx.x;
-    if (tid < bn) {
-        const int kd = bkind[tid];
-        if (kd == 1) dinv[tid] = 1.0 / bdiag[tid];
-        else if (kd == 2) dinv[tid] = 1.0 / (bdiag[tid] * bdiag[tid + 1] - boff[tid] * boff[tid]);
+    const int i = tid & (MAX_IB - 1), j0 = tid / MAX_IB;
+#pragma unroll
+    for (int u = 0; u < MAX_IB / 8; ++u) {
+        const int j = j0 + 8 * u;
+        co_std(&R.l11[i + MAX_IB * j], (j < i && i < bs) ? blk[i][j] : 0.0);
+    }
+    if (tid < MAX_IB) {
+        co_sti(&R.bperm[tid], bp[tid]);
+        co_sti(&R.bkind[tid], tid < bn ? bkind[tid] : 0);
+        co_std(&R.bdiag[tid], bdiag[tid]);
+        co_std(&R.boff[tid], boff[tid]);
+    }
+    if (tid == 64) {
+        co_sti(&R.k, k);
+        co_sti(&R.bs, bs);
+        co_sti(&R.bn, bn);
+        co_sti(&R.end_pos, end_pos);
     }
 }
 
+// The operands of the block after the current one, as threads t of nt: its rows [r0, r0 + nr) in the
+// current block's columns [c0, c0 + bs) and its tile, zeros beyond.
+template <int NT>
+__device__ __forceinline__ void load_operands(ChainLeaderLds &L, const gdouble *A, size_t lda, const gint *perm,
+                                              int c0, int bs, int r0, int nr, int t) {
+    constexpr int NU = (2 * MAX_IB * MAX_IB + NT - 1) / NT;
+    const __amdgpu_buffer_rsrc_t ry = co_rsrc(A + r0 + (size_t)c0 * lda), rt = co_rsrc(A + r0 + (size_t)r0 * lda);
+    const unsigned l8 = (unsigned)lda * 8u;
+    double v[NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+        const int e = t + NT * u, i = e & (MAX_IB - 1), j = (e >> 5) & (MAX_IB - 1);
+        const unsigned off = 8u * i + j * l8;
+        const double x = co_ldo(ry, (e < 1024 && i < nr && j < bs) ? off : CO_OOB);
+        const double z = co_ldo(rt, (e >= 1024 && e < 2048 && i < nr && j <= i) ? off : CO_OOB);
+        v[u] = (e < 1024) ? x : z;
+    }
+    const int p = (t < MAX_IB && t < nr) ? perm[r0 + t] : 0;
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+        const int e = t + NT * u, i = e & (MAX_IB - 1), j = (e >> 5) & (MAX_IB - 1);
+        if (e < 1024) L.Yn[i][j] = v[u];
+        else if (e < 2048) L.Cn[i][j] = v[u];
+    }
+    if (t < MAX_IB) L.noperm[t] = p;
+}
+
+// The pivot chain of a front's outer block.  Per inner block, once its record is out: substitution
+// of the next block's rows and its tile's update (4 + 2 of the 23 us), the next block's pivots on
+// the first wavefront, its record; when the panels' checks of the current block are in, the next
+// record's flag goes up at once and the bookkeeping of the finished block follows.  Beside the
+// pivots the other wavefronts wait for the panels' updates of the current block and bring the
+// operands of the block after the next into LDS, and before them two wavefronts store the current
+// block's tile while the other two substitute.  The record is written before the checks are known;
+// a failed column discards it and the block factored ahead.
 __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSync &C, ChainLeaderLds &L, int nit, int NP,
                              int ib, double small) {
     const int tid = threadIdx.x;
@@ -1736,32 +1959,34 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
     gint *const perm = gbl(F.perm);
     int k = S.kpos, end_pos = S.end_pos, nib = S.nib;
     int n1 = 0, n2 = 0;
-    bool have = false;  // the current block was factored ahead and is in the front
+    bool have = false;  // the current block was factored ahead; its record is out
     bool upd_prev = false;  // the panels' updates of the previous block are known complete
+    bool pf = false;    // the next block's operands are in LDS
     int bn = 0;
+    if (tid == 0) L.s_err = 0;
     for (int it = 0; it < nit; ++it) {
         const int bs = min(end_pos - k, ib);
+        const int be = k + bs, nbs = min(end_pos - be, ib);
+        const int ii = tid & (MAX_IB - 1), jg = tid / MAX_IB;
         if (!have) {
             // a fresh block: the panels' updates of the previous block are in place
             if (it > 0 && !upd_prev && !chain_wait(&C.updated[it - 1].v, NP, &C.err.v)) return;
             upd_prev = true;
             {
                 // every load issued before any is used (one round trip)
-                const int i = tid & (MAX_IB - 1), j0 = tid / MAX_IB;
                 const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + k + (size_t)k * lda);
                 double v[MAX_IB / 8];
 #pragma unroll
                 for (int u = 0; u < MAX_IB / 8; ++u) {
-                    const int j = j0 + 8 * u;
-                    const double x = co_ldb(rb, (size_t)min(i, bs > 0 ? bs - 1 : 0) + (size_t)min(j, bs > 0 ? bs - 1 : 0) * lda);
-                    v[u] = (i < bs && j <= i) ? x : 0.0;
+                    const int j = jg + 8 * u;
+                    v[u] = co_ldo(rb, (ii < bs && j <= ii) ? 8u * ii + 8u * j * (unsigned)lda : CO_OOB);
                 }
 #pragma unroll
                 for (int u = 0; u < MAX_IB / 8; ++u) {
-                    const int j = j0 + 8 * u;
-                    if (i < bs && j <= i) {
-                        L.blk[i][j] = v[u];
-                        co_st(bk + i + (size_t)j * lda, v[u]);
+                    const int j = jg + 8 * u;
+                    if (ii < bs && j <= ii) {
+                        L.blk[ii][j] = v[u];
+                        co_st(bk + ii + (size_t)j * lda, v[u]);
                     }
                 }
             }
@@ -1769,153 +1994,140 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
             lds_barrier();
             double bml;
             bn = block_factor_wg(L.blk, L.Wr, L.bp, L.bp2, L.bkind, L.bdiag, L.boff, bs, small, &bml, L.wbv, L.wbp,
-                                 L.Wr + MAX_IB);
+                                 L.Wr + MAX_IB, [] {});
             if (tid < bn && L.bkind[tid] == 2) L.blk[tid + 1][tid] = 0.0;
+            if (tid < 64) pivot_coefs(L.bkind, L.bdiag, L.boff, bn, L.pc);
             lds_barrier();
             if (bn > 0) {
-                const int i = tid & 31;
-                for (int j = tid >> 5; j < bs; j += 8)
-                    if (i < bs && j <= i) co_st(A + (k + i) + (size_t)(k + j) * lda, L.blk[i][j]);
+                for (int j = jg; j < bs; j += 8)
+                    if (ii < bs && j <= ii) co_st(A + (k + ii) + (size_t)(k + j) * lda, L.blk[ii][j]);
                 if (tid < bs) perm[k + tid] = L.operm[L.bp[tid]];
             }
             if (tid == 0) atomic_max_nonneg(&F.max_l_bits, bml);
+            write_record(C.recs[it], k, bs, bn, end_pos, L.bp, L.bkind, L.bdiag, L.boff, L.blk);
+            pf = false;
         }
-        pivots_dinv(L.bkind, L.bdiag, L.boff, L.dinv, bn);
-        // the next block ahead: its L rows (the panel substitution of rows be..be+nbs-1), its tile
-        // after this block's update, and its factorization.  Its operands are loaded before the
-        // record goes out: the panels overwrite those rows' block entries once they have it.
-        const int be = k + bs, nbs = min(end_pos - be, ib);
+        // the next block ahead (its operands are loaded before the record goes out: the panels
+        // overwrite those rows' block entries once they have it)
         const bool ahead = bs > 0 && bn == bs && nbs > 0 && it + 1 < nit;
-        double y[MAX_IB], cv[MAX_IB / 8];
-        if (ahead) {
-            if (it > 0 && !upd_prev && !chain_wait(&C.updated[it - 1].v, NP, &C.err.v)) return;
-            const bool live = tid < nbs;
-            {
-                const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + be + (size_t)k * lda);
-                const size_t ro = (size_t)(live ? tid : 0);
+        if (!have) {
+            if (ahead) load_operands<256>(L, A, lda, perm, k, bs, be, nbs, tid);
+            stores_done_barrier();
+            if (tid == 0) {
+                co_sti(&C.rec.v, it + 1);
+                __hip_atomic_fetch_add(&C.applied[it].v, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        } else if (tid >= 128) {
+            // the current block's tile, its backup and its rows' order: two wavefronts
+            const int t = tid - 128, j0 = t / MAX_IB;
 #pragma unroll
-                for (int j = 0; j < MAX_IB; ++j) {
-                    const double x = co_ldb(rb, ro + (size_t)L.bp[j < bs ? j : 0] * lda);
-                    y[j] = (live && j < bs) ? x : 0.0;
+            for (int u = 0; u < MAX_IB / 4; ++u) {
+                const int j = j0 + 4 * u;
+                if (ii < bs && j <= ii) {
+                    co_st(A + (k + ii) + (size_t)(k + j) * lda, L.blk[ii][j]);
+                    co_st(bk + ii + (size_t)j * lda, L.Nv[ii][j]);
                 }
             }
-            const int ii = tid & 31, jg = tid >> 5;
-            {
-                const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + be + (size_t)be * lda);
-#pragma unroll
-                for (int u = 0; u < MAX_IB / 8; ++u) {
-                    const int j = jg + 8 * u;
-                    const double x = co_ldb(rb, (size_t)min(ii, nbs - 1) + (size_t)min(j, nbs - 1) * lda);
-                    cv[u] = (ii < nbs && j <= ii) ? x : 0.0;
-                }
-            }
-            if (tid < MAX_IB) L.noperm[tid] = (tid < nbs) ? perm[be + tid] : 0;
+            if (bn > 0 && t < bs) perm[k + t] = L.operm[L.bp[t]];
+            __builtin_amdgcn_s_waitcnt(0);
+            if ((tid & 63) == 0) __hip_atomic_fetch_add(&C.applied[it].v, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        // record it (the barrier also completes the loads above)
-        ChainRec &R = C.recs[it];
-        if (tid < MAX_IB) {
-            co_sti(&R.bperm[tid], L.bp[tid]);
-            co_sti(&R.bkind[tid], tid < bn ? L.bkind[tid] : 0);
-            co_std(&R.bdiag[tid], L.bdiag[tid]);
-            co_std(&R.boff[tid], L.boff[tid]);
-        }
-        if (tid == 0) {
-            co_sti(&R.k, k);
-            co_sti(&R.bs, bs);
-            co_sti(&R.bn, bn);
-            co_sti(&R.end_pos, end_pos);
-        }
-        stores_done_barrier();
-        if (tid == 0) co_sti(&C.rec.v, it + 1);
         int bn2 = 0;
         double bml2 = 0.0, nv[MAX_IB / 8];
         if (ahead) {
             double (*Lr)[MAX_IB + 1] = L.Wr;
             double (*Wt)[MAX_IB + 1] = L.Wr + MAX_IB;
-            if (tid < 64) {
-                // (wavefront 0 whole: rows beyond the block hold zeros)
-                panel_trsm_d(y, L.blk, bn, L.bkind, L.dinv, L.bdiag, L.boff);
-                if (tid < MAX_IB) {
+            if (tid < 128) {
+                const int row = tid >> 2, h = tid & 3;
+                double y[8];
 #pragma unroll
-                    for (int j = 0; j < MAX_IB; ++j) Lr[tid][j] = y[j];
-                }
-            }
-            {
-                const int ii = tid & 31, jg = tid >> 5;
+                for (int t = 0; t < 8; ++t) y[t] = L.Yn[row][L.bp[4 * t + h]];
+                quad_substitute(y, L.blk, bn, L.pc);
 #pragma unroll
-                for (int u = 0; u < MAX_IB / 8; ++u) L.Ct[ii][jg + 8 * u] = cv[u];
+                for (int t = 0; t < 8; ++t) Lr[row][4 * t + h] = y[t];
             }
+#pragma unroll
+            for (int u = 0; u < MAX_IB / 8; ++u) L.Ct[ii][jg + 8 * u] = L.Cn[ii][jg + 8 * u];
             lds_barrier();
+            if (tid < MAX_IB) L.operm[tid] = L.noperm[tid];
+            if (tid == 0) L.s_pf = 0;
             next_tile_update(Lr, Wt, L.Ct, L.bkind, L.bdiag, L.boff, nbs, bs, nv);
+#pragma unroll
+            for (int u = 0; u < MAX_IB / 8; ++u) L.Nv[ii][jg + 8 * u] = nv[u];
+            const int be2 = be + nbs, nbs2 = min(end_pos - be2, ib);
             bn2 = block_factor_wg(L.Ct, L.Wr, L.nbp, L.bp2, L.nbkind, L.nbdiag, L.nboff, nbs, small, &bml2, L.wbv,
-                                  L.wbp, L.Wr + MAX_IB);
+                                  L.wbp, L.Wr + MAX_IB, [&] {
+                // with a failed column in the current block this block is discarded (and the panels
+                // have more to do): nothing to bring
+                if (nbs2 <= 0 || it + 2 >= nit) return;
+                int aux;
+                if (!wave_poll(C.applied[it], NP + 2, &C.err.v, &aux)) { L.s_err = 1; return; }
+                if (aux < bs) return;
+                if (!wave_poll(C.updated[it], NP, &C.err.v, &aux)) { L.s_err = 1; return; }
+                load_operands<192>(L, A, lda, perm, be, nbs, be2, nbs2, tid - 64);
+                if (tid == 64) L.s_pf = 1;
+            });
             if (tid < bn2 && L.nbkind[tid] == 2) L.Ct[tid + 1][tid] = 0.0;
+            if (tid < 64) pivot_coefs(L.nbkind, L.nbdiag, L.nboff, bn2, L.pc);
             lds_barrier();
+            if (L.s_err) return;
+            write_record(C.recs[it + 1], be, nbs, bn2, end_pos, L.nbp, L.nbkind, L.nbdiag, L.nboff, L.Ct);
+            __builtin_amdgcn_s_waitcnt(0);
         }
         // the check of block it; the panels' update count of the block comes along (complete, it
-        // saves the wait before the next block's operands are loaded)
-        if (!chain_wait_aux(C.applied[it], NP, &C.err.v, &L.s_fail, &C.updated[it], NP, &L.s_upd)) return;
-        const bool upd_done = L.s_upd != 0;
-        upd_prev = upd_done;
+        // saves a wait).  The barriers inside complete the next record's stores.
+        if (!chain_wait_aux(C.applied[it], NP + 2, &C.err.v, &L.s_fail, &C.updated[it], NP, &L.s_upd)) return;
+        upd_prev = L.s_upd != 0;
         int nelim = 0;
         if (bn > 0) {
             nelim = min(L.s_fail, bn);
             if (nelim > 0 && L.bkind[nelim - 1] == 2) nelim -= 1;
         }
+        const bool commit = ahead && nelim == bs;
+        if (commit && tid == 0) co_sti(&C.rec.v, it + 2);
         // D and the pivot counts of the accepted columns (k_block_finish)
-        int is1 = 0, is2 = 0;
-        if (tid < nelim) {
-            const int kd = L.bkind[tid];
-            const int c = k + tid;
-            if (kd == 1) {
-                gbl(F.dkind)[c] = 1; gbl(F.ddiag)[c] = L.bdiag[tid]; gbl(F.doff)[c] = 0.0;
-                is1 = 1;
-            } else if (kd == 2 && tid + 1 < nelim) {
-                gbl(F.dkind)[c] = 2; gbl(F.dkind)[c + 1] = 3;
-                gbl(F.ddiag)[c] = L.bdiag[tid]; gbl(F.ddiag)[c + 1] = L.bdiag[tid + 1];
-                gbl(F.doff)[c] = L.boff[tid]; gbl(F.doff)[c + 1] = 0.0;
-                is2 = 1;
-            }
-        }
-        n1 += __syncthreads_count(is1);
-        n2 += __syncthreads_count(is2);
-        if (nib < MAX_OB_IB && tid == 0) S.ib_ne[nib] = (int8_t)nelim;
-        ++nib;
-        if (ahead && nelim == bs) {
-            // keep the block factored ahead: the panels left its tile to this workgroup
-            {
-                const int ii = tid & 31, jg = tid >> 5;
-#pragma unroll
-                for (int u = 0; u < MAX_IB / 8; ++u) {
-                    const int j = jg + 8 * u;
-                    if (ii < nbs && j <= ii) {
-                        co_st(A + (be + ii) + (size_t)(be + j) * lda, L.Ct[ii][j]);
-                        co_st(bk + ii + (size_t)j * lda, nv[u]);
-                    }
+        if (tid < 64) {
+            int is1 = 0, is2 = 0;
+            if (tid < nelim) {
+                const int kd = L.bkind[tid];
+                const int c = k + tid;
+                if (kd == 1) {
+                    gbl(F.dkind)[c] = 1; gbl(F.ddiag)[c] = L.bdiag[tid]; gbl(F.doff)[c] = 0.0;
+                    is1 = 1;
+                } else if (kd == 2 && tid + 1 < nelim) {
+                    gbl(F.dkind)[c] = 2; gbl(F.dkind)[c + 1] = 3;
+                    gbl(F.ddiag)[c] = L.bdiag[tid]; gbl(F.ddiag)[c + 1] = L.bdiag[tid + 1];
+                    gbl(F.doff)[c] = L.boff[tid]; gbl(F.doff)[c + 1] = 0.0;
+                    is2 = 1;
                 }
             }
-            if (bn2 > 0 && tid < nbs) perm[be + tid] = L.noperm[L.nbp[tid]];
+            n1 += __popcll(__ballot(is1));
+            n2 += __popcll(__ballot(is2));
+        }
+        if (nib < MAX_OB_IB && tid == 0) S.ib_ne[nib] = (int8_t)nelim;
+        ++nib;
+        if (commit) {
             if (tid == 0) atomic_max_nonneg(&F.max_l_bits, bml2);
-            for (int e = tid; e < MAX_IB * MAX_IB; e += 256) {
-                const int i = e & (MAX_IB - 1), j = e / MAX_IB;
-                L.blk[i][j] = L.Ct[i][j];
-            }
+#pragma unroll
+            for (int u = 0; u < MAX_IB / 8; ++u) L.blk[ii][jg + 8 * u] = L.Ct[ii][jg + 8 * u];
             if (tid < MAX_IB) {
                 L.bp[tid] = L.nbp[tid];
                 L.bkind[tid] = (tid < bn2) ? L.nbkind[tid] : 0;
                 L.bdiag[tid] = L.nbdiag[tid];
                 L.boff[tid] = L.nboff[tid];
             }
+            pf = L.s_pf != 0;
             lds_barrier();
             bn = bn2;
             k = be;
             have = true;
+            if (pf) upd_prev = true;
         } else {
             have = false;
             if (bn == 0 || nelim < bs) {
                 // failed columns (the whole block when nothing was eliminated) move to the end of
                 // the outer block, after every panel's restore and cross terms
-                if (!upd_done && !chain_wait(&C.updated[it].v, NP, &C.err.v)) return;
+                if (!upd_prev && !chain_wait(&C.updated[it].v, NP, &C.err.v)) return;
                 upd_prev = true;
                 if (tid == 0) {
                     int n = 0;
@@ -1951,20 +2163,6 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
         F.n1 += n1;
         F.n2 += n2;
     }
-}
-
-// A value the compiler has to take as new: address arithmetic formed from it is neither hoisted
-// out of the block loop nor kept from one phase to the next.  (Left to itself the compiler holds
-// some hundred loop-invariant offsets of the unrolled loads and stores below in registers across
-// the loop and spills the data instead: 440 spilled registers, 39 us per substitution.)
-__device__ __forceinline__ int fresh(int x) {
-    __asm__ volatile("" : "+v"(x));
-    return x;
-}
-__device__ __forceinline__ int fresh_uniform(int x) {
-    x = __builtin_amdgcn_readfirstlane(x);
-    __asm__ volatile("" : "+s"(x));
-    return x;
 }
 
 // Columns [c0, c0 + ncol) of the L rows of an update round, transposed into LDS: the loads (cl_load,
@@ -2069,24 +2267,53 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
     const int nchunk = (m - ob_start + CH - 1) / CH;
     const bool single = nchunk <= NP;  // at most one chunk per panel
     const double bound = 1.0 / threshold;
+    constexpr int NS = CH / 64;  // sub-tiles of a chunk; thread (row = tid / 4, h = tid % 4) of each
+    double y[NS][8];             // columns 4 t + h of the row's block entries
+    int pre_k = -1, pre_bs = 0;  // block whose rows are in y already
+    // a chunk's block entries in column order (zeros outside the front's live rows and beyond the
+    // block, by the resource's range)
+    auto load_rows = [&](int c, int k, int bs) {
+        const int t4 = fresh(threadIdx.x), row = t4 >> 2, h = t4 & 3;
+        const unsigned l8 = (unsigned)fresh_uniform(m * 8);
+        const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + (size_t)k * m);
+#pragma unroll
+        for (int u = 0; u < NS; ++u) {
+            const int r = ob_start + c * CH + 64 * u + row;
+            const unsigned off = (r >= k + bs && r < m) ? 8u * r + h * l8 : CO_OOB;
+#pragma unroll
+            for (int t = 0; t < 8; ++t) y[u][t] = co_ldo(rb, 4 * t + h < bs ? off + 4 * t * l8 : CO_OOB);
+        }
+    };
     for (int it = 0; it < nit; ++it) {
         if (!chain_wait(&C.rec.v, it + 1, &C.err.v)) return;
         const int tid = fresh(threadIdx.x);
         const size_t lda = (size_t)(unsigned)fresh_uniform(m);
         const ChainRec &R = C.recs[it];
-        if (tid < MAX_IB) {
-            L.bp[tid] = co_ldi(&R.bperm[tid]);
-            L.bkind[tid] = (int8_t)co_ldi(&R.bkind[tid]);
-            L.bdiag[tid] = co_ldd(&R.bdiag[tid]);
-            L.boff[tid] = co_ldd(&R.boff[tid]);
+        {
+            double v[MAX_IB / 8];
+#pragma unroll
+            for (int u = 0; u < MAX_IB / 8; ++u) v[u] = co_ldo(co_rsrc(gbl(R.l11)), 8u * (tid + 256 * u));
+            if (tid < 64) {
+                const __amdgpu_buffer_rsrc_t ri = co_rsrc((const gdouble *)gbl(&R.k));
+                const int c = tid & 31;
+                const int p = __builtin_amdgcn_raw_buffer_load_b32(ri, 16 + 4 * c, 0, 16);
+                const int kd = __builtin_amdgcn_raw_buffer_load_b32(ri, 16 + 4 * MAX_IB + 4 * c, 0, 16);
+                const double dg = co_ldo(ri, 16 + 8 * MAX_IB + 8 * c);
+                const double of = co_ldo(ri, 16 + 16 * MAX_IB + 8 * c);
+                const int hd = __builtin_amdgcn_raw_buffer_load_b32(ri, 4 * (c & 3), 0, 16);
+                L.bp[c] = p;
+                L.bkind[c] = (int8_t)kd;
+                L.bdiag[c] = dg;
+                L.boff[c] = of;
+                L.rec[c & 3] = hd;
+                wave_sync();
+                pivot_coefs(L.bkind, L.bdiag, L.boff, MAX_IB, L.pc);  // (kind 0 beyond the eliminated columns)
+            }
+            const int i = tid & (MAX_IB - 1), j0 = tid / MAX_IB;
+#pragma unroll
+            for (int u = 0; u < MAX_IB / 8; ++u) L.blk[i][j0 + 8 * u] = v[u];
         }
-        if (tid == 0) {
-            L.rec[0] = co_ldi(&R.k);
-            L.rec[1] = co_ldi(&R.bs);
-            L.rec[2] = co_ldi(&R.bn);
-            L.rec[3] = co_ldi(&R.end_pos);
-        }
-        __syncthreads();
+        lds_barrier();
         const int k = __builtin_amdgcn_readfirstlane(L.rec[0]), bs = __builtin_amdgcn_readfirstlane(L.rec[1]);
         const int bn = __builtin_amdgcn_readfirstlane(L.rec[2]), end_pos = __builtin_amdgcn_readfirstlane(L.rec[3]);
         const int be = k + bs;
@@ -2094,110 +2321,67 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
         // the block has no failed column
         const int r0p = ob_start + pidx * CH, r1p = min(r0p + CH, m);
         const bool fast = single && pidx < nchunk && r1p > be && bn == bs;
-        double pml = 0.0;  // (fast) the row's largest |l|
         if (bn > 0) {
-            // L11 and the first chunk's rows, all loads in flight together
-            double v[MAX_IB / 8];
-            {
-                const int i = tid & (MAX_IB - 1), j0 = tid / MAX_IB;
-                const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + k + (size_t)k * lda);
-#pragma unroll
-                for (int u = 0; u < MAX_IB / 8; ++u) {
-                    const int j = j0 + 8 * u;
-                    v[u] = co_ldo(rb, (i < bs && j < i) ? 8u * (i + j * (unsigned)lda) : CO_OOB);
-                }
-            }
-            // a row's block entries in column order (zeros outside the front's live rows and
-            // beyond the block, by the resource's range)
-            double yn[MAX_IB];
-            auto load_rows = [&](int c) {
-                const int r = ob_start + c * CH + tid, l8 = fresh_uniform((int)lda * 8), nb = fresh_uniform(bs);
-                const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + (size_t)k * lda);
-                const unsigned off = (tid < CH && r >= be && r < m) ? 8u * r : CO_OOB;
-#pragma unroll
-                for (int j = 0; j < MAX_IB; ++j) yn[j] = co_ldo(rb, j < nb ? off + min(j, nb) * l8 : CO_OOB);
-            };
-            load_rows(pidx);
-            {
-                const int i = tid & (MAX_IB - 1), j0 = tid / MAX_IB;
-#pragma unroll
-                for (int u = 0; u < MAX_IB / 8; ++u) L.blk[i][j0 + 8 * u] = v[u];
-                pivots_dinv(L.bkind, L.bdiag, L.boff, L.dinv, bn);
-                lds_barrier();
-            }
+            if (pre_k != k || pre_bs != bs) load_rows(pidx, k, bs);
             for (int c = pidx; c < nchunk; c += NP) {
-                const int r0 = ob_start + c * CH, r1 = min(r0 + CH, m);
-                if (c != pidx) load_rows(c);
-                if (r1 <= be || tid >= CH) continue;
-                // (wavefront-uniform: CH is a multiple of 64)
-                const int r = r0 + tid;
-                const bool live = r >= be && r < r1;
-                double y[MAX_IB];
-                {
-                    // backed up as they are (restore_diagonal_with_perm reads the backup in
-                    // column order), then gathered into pivot order through the wavefront's own
-                    // LDS rows
-                    {
-                        const __amdgpu_buffer_rsrc_t rb = co_rsrc(bk);
-                        const int l8 = fresh_uniform((int)lda * 8), nb = fresh_uniform(bs);
-                        const unsigned off = live ? 8u * (r - k) : CO_OOB;
-#pragma unroll
-                        for (int j = 0; j < MAX_IB; ++j)
-                            if (j < nb) co_stb(rb, off + min(j, nb) * l8, yn[j]);
-                    }
-                    double *yb = L.Yb[tid];
-#pragma unroll
-                    for (int j = 0; j < MAX_IB; ++j) yb[j] = yn[j];
-                    // (the lane reads back only what it wrote: LDS operations of a wavefront
-                    // are performed in order)
-#pragma unroll
-                    for (int j = 0; j < MAX_IB; ++j) y[j] = yb[L.bp[j]];
-                }
-                panel_trsm_d(y, L.blk, bn, L.bkind, L.dinv, L.bdiag, L.boff);
+                if (c != pidx) load_rows(c, k, bs);
+                const int row = tid >> 2, h = tid & 3;
+                const unsigned l8 = (unsigned)fresh_uniform((int)lda * 8);
                 int first = INT_MAX;
-                {
-                    const __amdgpu_buffer_rsrc_t rb = co_rsrc(A + (size_t)k * lda);
-                    const int l8 = fresh_uniform((int)lda * 8), nb = fresh_uniform(bs);
-                    const unsigned off = live ? 8u * r : CO_OOB;
 #pragma unroll
-                    for (int j = 0; j < MAX_IB; ++j)
-                        if (j < nb) co_stb(rb, off + min(j, nb) * l8, y[j]);
-                }
-                if (live) {
+                for (int u = 0; u < NS; ++u) {
+                    const int rb0 = ob_start + c * CH + 64 * u, r = rb0 + row;
+                    if (rb0 + 63 < be || rb0 >= m) continue;  // (uniform)
+                    const bool live = r >= be && r < m;
+                    // backed up as they are (restore_diagonal_with_perm reads the backup in
+                    // column order), then gathered into pivot order through LDS rows of the
+                    // wavefront's own (its LDS operations are performed in order)
+                    const __amdgpu_buffer_rsrc_t rk = co_rsrc(bk), ra = co_rsrc(A + (size_t)k * lda);
+                    const unsigned ok = live ? 8u * (r - k) + h * l8 : CO_OOB, oa = live ? 8u * r + h * l8 : CO_OOB;
+                    double *yb = L.Yb[row];
 #pragma unroll
-                    for (int q = MAX_IB - 1; q >= 0; --q)
-                        if (q < bn && fabs(y[q]) >= bound) first = q;
-                    if (first != INT_MAX && L.bkind[first] == 3) first -= 1;
+                    for (int t = 0; t < 8; ++t) {
+                        co_stb(rk, 4 * t + h < bs ? ok + 4 * t * l8 : CO_OOB, y[u][t]);
+                        yb[4 * t + h] = y[u][t];
+                    }
+                    wave_sync();
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) y[u][t] = yb[L.bp[4 * t + h]];
+                    wave_sync();
+                    quad_substitute(y[u], L.blk, bn, L.pc);
+#pragma unroll
+                    for (int t = 7; t >= 0; --t) {
+                        const int q = 4 * t + h;
+                        co_stb(ra, q < bs ? oa + 4 * t * l8 : CO_OOB, y[u][t]);
+                        if (live && q < bn && fabs(y[u][t]) >= bound) first = min(first, L.pc.kd[q] == 3 ? q - 1 : q);
+                    }
                 }
                 first = wave_min_int(first);
                 if ((tid & 63) == 0 && first != INT_MAX) atomicMin(&C.applied[it].aux, first);
-                if (fast) {
-                    // W = L D (compute_ld_into factor.rs:1536-1563) of the row, used if no column fails
-                    const int lc = tid & 31;
-                    const int kdl = L.bkind[lc];
-                    const double bdl = L.bdiag[lc], bol = L.boff[lc];
-                    double (*WT)[64 + 1] = L.WT[tid >> 6];
-#pragma unroll
-                    for (int j = 0; j < MAX_IB; ++j) {
-                        const int kd = __builtin_amdgcn_readlane(kdl, j);
-                        const double dj = readlane_f64(bdl, j);
-                        double w = y[j] * dj;
-                        if (kd == 2 && j + 1 < MAX_IB) w = w + y[j + 1 < MAX_IB ? j + 1 : j] * readlane_f64(bol, j);
-                        if (kd == 3 && j > 0) w = y[j > 0 ? j - 1 : 0] * readlane_f64(bol, j > 0 ? j - 1 : 0) + w;
-                        WT[j][tid & 63] = (kd == 0) ? 0.0 : w;
-                        pml = max_abs(pml, y[j]);
-                    }
-                }
             }
         }
         stores_done_barrier();
         if (tid == 0) __hip_atomic_fetch_add(&C.applied[it].v, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        double pml = 0.0;  // (fast) the thread's largest |l|
+        if (fast) {
+            // W = L D, used if no column fails
+#pragma unroll
+            for (int u = 0; u < NS; ++u) {
+                double w[8];
+                quad_ld(y[u], L.pc, w);
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    L.WT[u][4 * t + (tid & 3)][tid >> 2] = w[t];
+                    pml = max_abs(pml, y[u][t]);
+                }
+            }
+        }
         // (fast) the first round's columns of the first sub-tile: this panel's own rows
         double cv[4][8];
         const int R0f = (r0p + 63 < be) ? r0p + 64 : r0p;  // first sub-tile with rows below the block
         __amdgpu_buffer_rsrc_t rc = co_rsrc_front(A, lda, (size_t)min(R0f, m - 1) + (size_t)min(be, m - 1) * lda);
         cu_load(cv, rc, lda, fast && be < obe);
-        if (!chain_wait_aux(C.applied[it], NP, &C.err.v, &L.s_fail)) return;
+        if (!chain_wait_aux(C.applied[it], NP + 2, &C.err.v, &L.s_fail)) return;
         int permute_from = -1;
         if (bn > 0) {
             int nelim = min(L.s_fail, bn);
@@ -2385,6 +2569,13 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
         if (permute_from > 0) permute_rows();
         stores_done_barrier();
         if (tid == 0) __hip_atomic_fetch_add(&C.updated[it].v, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // without failed columns nothing moves: the next block starts at be, its rows can come now
+        pre_k = -1;
+        if (permute_from == 0 && single && pidx < nchunk && it + 1 < nit && end_pos > be) {
+            pre_k = be;
+            pre_bs = min(end_pos - be, ib);
+            load_rows(pidx, pre_k, pre_bs);
+        }
         if (permute_from == 0) permute_rows();
     }
 }
