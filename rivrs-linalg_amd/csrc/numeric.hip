@@ -417,6 +417,20 @@ __device__ __forceinline__ void copy_next_block(const FrontDev &F, const AptpSta
     }
 }
 
+// A value the compiler has to take as new: address arithmetic formed from it is neither hoisted
+// out of the block loop nor kept from one phase to the next.  (Left to itself the compiler holds
+// some hundred loop-invariant offsets of the unrolled loads and stores below in registers across
+// the loop and spills the data instead: 440 spilled registers, 39 us per substitution.)
+__device__ __forceinline__ int fresh(int x) {
+    __asm__ volatile("" : "+v"(x));
+    return x;
+}
+__device__ __forceinline__ int fresh_uniform(int x) {
+    x = __builtin_amdgcn_readfirstlane(x);
+    __asm__ volatile("" : "+s"(x));
+    return x;
+}
+
 // ===========================================================================
 // APTP: complete pivoting on the inner block (factor_block_diagonal, factor.rs:891-1153).
 // Returns the eliminated count; bp/bkind/bdiag/boff describe the pivots and *maxl the largest
@@ -435,14 +449,21 @@ __device__ __forceinline__ void copy_next_block(const FrontDev &F, const AptpSta
 //  * A dead entry (eliminated, outside the block, the second copy) is NaN.  fmax ignores it, the
 //    diagonal of the LDS copy is NaN, so a pivot's own row gets NaN multipliers and dies in the
 //    ordinary update: no masks.
-//  * Argmax: the high words of the lanes' maxima are reduced by DPP; unless one lane and one of
-//    its entries alone has that high word (ties, or maxima equal in their upper 32 bits), the
-//    exact rule runs: largest value, then first in the column-major order of positions.
+//  * Argmax: an entry's key is the high word of its magnitude with the column index in the low
+//    five bits; as a float its NaN is ignored and its order is the magnitudes' (which is why
+//    blocks with entries above 2^1000 always take the exact rule).  Keys are reduced by v_max3 and
+//    DPP, so the winner's row is its lane and its column the key's low bits.  It stands if no
+//    other lane's key and no other entry of its row reaches its leading 15 mantissa bits;
+//    otherwise (near-equal values, ties, tiny values) the exact rule runs: largest value, then
+//    first in the column-major order of positions.
 //  * A full symmetric copy of the block in LDS gives a lane the pivot row's entries of its own row
 //    and of its eight columns in one round trip, beside the reciprocal of the pivot.
-// Measured on the 64^3 Helmholtz chain (see k_aptp_outer): the form it replaced, 256 threads
-// with four entries each, the block permuted through LDS and one barrier per step, took 40 us per
-// 32-column block.
+// A wavefront issues an operation every 5 to 6 cycles here (8 to 9 when it depends on the one
+// before), an LDS round trip takes 70, a DPP stage 17, a division 76: a step with a diagonal
+// winner is some 190 operations, 1320 cycles.  A 32-column block takes 18 us with diagonal
+// winners and 23 us with entries of random signs and sizes, 25 us before the argmax worked on
+// keys, 40 us as 256 threads with four entries each, one barrier per step and the block permuted
+// through LDS.
 // ===========================================================================
 // max(|a|, |b|), NaN operands ignored (the compiler's fmax canonicalises loop-carried operands
 // first, one more instruction each)
@@ -463,165 +484,213 @@ __device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
     return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-// The pivot steps, by one wavefront.  S: 32 x 32 doubles (the symmetric copy), ptab: 32 ints
-// (positions), lbuf: the multipliers by row identity and pivot position.  On return bp holds the
+// maximum of three keys as floats (NaN ignored)
+__device__ __forceinline__ unsigned key_max3(unsigned a, unsigned b, unsigned c) {
+    unsigned r;
+    __asm__("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ unsigned hi_word(double v) {
+    return (unsigned)((unsigned long long)__double_as_longlong(v) >> 32);
+}
+
+// The pivot steps, by one wavefront.  S: 32 x 32 doubles (the symmetric copy), lbuf: the
+// multipliers by row identity and pivot position.  On return bp holds the
 // row at each position and the diagonal of S the uneliminated diagonal entries.
-__device__ __forceinline__ int block_pivots(const double (*blk)[MAX_IB + 1], double *S, int *bp, int *ptab,
+__device__ __forceinline__ int block_pivots(const double (*blk)[MAX_IB + 1], double *S, int *bp,
                                             int8_t *bkind, double *bdiag, double *boff, int bs, double small,
                                             double *maxl, double (*lbuf)[MAX_IB + 1]) {
     static_assert(MAX_IB == 32, "lane layout of the block");
-    const int lane = threadIdx.x & 63, i = lane & 31, h = lane >> 5;
+    const int lane = fresh(threadIdx.x) & 63, i = lane & 31, h = lane >> 5;
     const double dead = __builtin_nan("");
-    if (lane < MAX_IB) { bkind[lane] = 0; bdiag[lane] = 0.0; boff[lane] = 0.0; ptab[lane] = lane; }
     double e[8];
     int jo[8], w1[8], w2[8];  // column, and the entry's two places in S
+    bool wild = false;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
         const int j = (i + 1 + u + 8 * h) & 31;
         const bool copy2 = u == 7 && h == 1 && i >= 16;
         const double v = blk[max(i, j)][min(i, j)];
-        e[u] = (i < bs && j < bs && !copy2) ? v : dead;
+        const bool live = i < bs && j < bs;
+        wild |= live && (hi_word(v) & 0x7fffffffu) >= 0x7e700000u;
+        e[u] = (live && !copy2) ? v : dead;
         jo[u] = j;
         w1[u] = copy2 ? 33 * i : 32 * i + j;  // (the second copy writes its NaN to the diagonal)
         w2[u] = copy2 ? 33 * i : 32 * j + i;
     }
-    double dg = (h == 0 && i < bs) ? blk[i][i] : dead;
+    double dg = blk[i][i];
+    wild |= i < bs && (hi_word(dg) & 0x7fffffffu) >= 0x7e700000u;
+    dg = (h == 0 && i < bs) ? dg : dead;
     if (h == 0) S[33 * i] = dead;
 #pragma unroll
     for (int u = 0; u < 8; ++u) { S[w1[u]] = e[u]; S[w2[u]] = e[u]; }
-    int posr = i, idr = i;
+    // a winning key above this is a value of at least `small` and far from the denormals
+    const unsigned floor_key =
+        __any(wild) ? 0xffffffffu : (unsigned)__builtin_amdgcn_readfirstlane((int)max(hi_word(small) | 31u, 0x01000000u));
+    int posr = i, idr = i, pj[8];   // position of the lane's row and columns; row at position `lane`
+#pragma unroll
+    for (int u = 0; u < 8; ++u) pj[u] = jo[u];
+    int kindr = 0;                  // lane c: kind and D of pivot c
+    double bdr = 0.0, bor = 0.0;
     int cur = 0;
     double ml = 0.0;
     wave_sync();
-    while (cur < bs) {
-        double m = max_abs(max_abs(max_abs(e[0], e[1]), max_abs(e[2], e[3])),
-                           max_abs(max_abs(e[4], e[5]), max_abs(e[6], e[7])));
-        m = max_abs(max_abs(m, dg), 0.0);
-        unsigned bits = (fabs(dg) == m) ? 256u : 0u;
+    bool more = bs > 0;
+    while (more) {
+        unsigned long long mo, mg;
+        unsigned M;
+        // 1x1 pivots at the largest diagonal entry, clearly the largest entry of the block
+        for (;;) {
+            constexpr unsigned KEY = 0x7fffffe0u;
+            unsigned ku[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) bits |= (fabs(e[u]) == m) ? 1u << u : 0u;
-        const unsigned hi = (unsigned)((unsigned long long)__double_as_longlong(m) >> 32);
-        const unsigned M = wave_max_u32(hi);
-        const unsigned long long mask = __ballot(hi == M);
-        const int Lw = __builtin_ctzll(mask);
-        const unsigned wb = (unsigned)__builtin_amdgcn_readlane((int)bits, Lw);
-        double gv;
-        int ia, ib;  // the winner's two rows (equal: a diagonal entry)
-        if (M >= 0x00100000u && (mask & (mask - 1)) == 0 && (wb & (wb - 1)) == 0) {
-            gv = readlane_f64(m, Lw);
-            ia = Lw & 31;
-            ib = (wb == 256u) ? ia : (ia + 1 + __builtin_ctz(wb) + 8 * (Lw >> 5)) & 31;
-        } else {
-            // largest value, equal values by position; no live entry above zero: position cur
-            gv = wave_fmax(m);
-            int key = (fabs(dg) == gv) ? 65 * posr : INT_MAX;
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int pj = ptab[jo[u]];
-                key = (fabs(e[u]) == gv) ? min(key, 64 * min(posr, pj) + max(posr, pj)) : key;
-            }
-            key = (gv > 0.0) ? __builtin_amdgcn_readfirstlane(wave_min_int(key)) : 65 * cur;
-            gv = readlane_f64(gv, 0);
-            ia = __builtin_amdgcn_readlane(idr, key & 63);
-            ib = __builtin_amdgcn_readlane(idr, key >> 6);
-        }
-        if (gv < small) break;
-        // t: the winner's row (larger position), mi: its column
-        const int qa = __builtin_amdgcn_readlane(posr, ia), qb = __builtin_amdgcn_readlane(posr, ib);
-        const int t = qa > qb ? ia : ib, mi = qa > qb ? ib : ia;
-        const int pt = max(qa, qb), pm = min(qa, qb);
-        const double att = readlane_f64(dg, t), amm = readlane_f64(dg, mi);
-        bool two = false;
-        int pid = t, pp = pt;  // 1x1: the pivot's row and position
-        double d = att;
-        if (t != mi) {
-            const double delta = amm * att - gv * gv;
-            if (fabs(delta) >= 0.5 * gv * gv) {
-                two = true;
-            } else if (fabs(amm) >= fabs(att)) {
-                pid = mi; pp = pm; d = amm;
-            }
-        }
-        const int x1 = __builtin_amdgcn_readlane(idr, cur);  // the row standing at position cur
-        if (!two) {
+            for (int u = 0; u < 8; ++u) ku[u] = (hi_word(e[u]) & KEY) | (unsigned)jo[u];
+            const unsigned kg = key_max3((hi_word(dg) & KEY) | (unsigned)i, 0u, 0u);
+            const unsigned ko =
+                key_max3(key_max3(ku[0], ku[1], ku[2]), key_max3(ku[3], ku[4], ku[5]), key_max3(ku[6], ku[7], 0u));
+            M = wave_max_u32(max(kg, ko));
+            // the row of the winner's column, which is the pivot's for a diagonal winner (the barrier
+            // to the compiler keeps its loads here, in flight while the winner is checked)
+            const int pid = M & 31;
             const double *row = S + 32 * pid;
             const double ci = row[i];
             double cj[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) cj[u] = row[jo[u]];
+            __asm__ volatile("" ::: "memory");
+            const unsigned T = M > floor_key ? M & ~31u : 0u;  // (0: every lane, so not this path)
+            mo = __ballot(ko >= T);
+            mg = __ballot(kg >= T);
+            if ((mo | (mg & (mg - 1))) != 0) break;
+            const double d = readlane_f64(dg, pid);
+            const int pp = __builtin_amdgcn_readlane(posr, pid);
+            const int x1 = __builtin_amdgcn_readlane(idr, cur);  // the row standing at position cur
             posr = (i == x1) ? pp : posr;
-            posr = (i == pid) ? cur : posr;
             idr = (lane == pp) ? x1 : idr;
             idr = (lane == cur) ? pid : idr;
-            ptab[i] = posr;
-            wave_sync();
-            int pj[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) pj[u] = ptab[jo[u]];
             const double inv = 1.0 / d;
             const double li = ci * inv, wi = li * d;
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
+                pj[u] = (jo[u] == x1) ? pp : pj[u];
                 const double lj = cj[u] * inv, wj = lj * d;
                 const double p1 = li * wj, p2 = lj * wi;
                 e[u] = e[u] - (posr > pj[u] ? p1 : p2);
             }
             dg = dg - li * wi;
             ml = max_abs(ml, li);
-            if (h == 0) lbuf[i][cur] = li;
-            if (lane == 0) { bkind[cur] = 1; bdiag[cur] = d; }
+            lbuf[i][cur] = li;
+            kindr = (lane == cur) ? 1 : kindr;
+            bdr = (lane == cur) ? d : bdr;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) { S[w1[u]] = e[u]; S[w2[u]] = e[u]; }
+            wave_sync();
+            cur = __builtin_amdgcn_readfirstlane(cur + 1);
+            if (cur >= bs) { more = false; break; }
+        }
+        if (!more) break;
+        int ia, ib = M & 31;
+        const unsigned long long mask = mo | mg;
+        if (M > floor_key && (mask & (mask - 1)) == 0 && mg == 0) {
+            ia = __builtin_ctzll(mask) & 31;
+            // another entry of the winner's lane (all in row ia, or its diagonal) as large
+            const double ca = S[32 * ia + i], g = fabs(readlane_f64(ca, ib));
+            if ((__ballot(fabs(ca) >= g) & ~(0x100000001ull << ib)) != 0 || fabs(readlane_f64(dg, ia)) >= g) ia = -1;
+        } else {
+            ia = -1;
+        }
+        if (ia < 0) {
+            // largest value, equal values by position; no live entry above zero: position cur
+            const double m = max_abs(max_abs(max_abs(e[0], e[1]), max_abs(e[2], e[3])),
+                                     max_abs(max_abs(e[4], e[5]), max_abs(e[6], e[7])));
+            const double gv = wave_max_dpp(max_abs(max_abs(m, dg), 0.0));
+            int key = (fabs(dg) == gv) ? 65 * posr : INT_MAX;
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                key = (fabs(e[u]) == gv) ? min(key, 64 * min(posr, pj[u]) + max(posr, pj[u])) : key;
+            key = (gv > 0.0) ? __builtin_amdgcn_readfirstlane(wave_min_int(key)) : 65 * cur;
+            ia = __builtin_amdgcn_readlane(idr, key & 63);
+            ib = __builtin_amdgcn_readlane(idr, key >> 6);
+            if (gv < small) { more = false; break; }
+        }
+        // t: the winner's row (larger position), mi: its column
+        const int qa = __builtin_amdgcn_readlane(posr, ia), qb = __builtin_amdgcn_readlane(posr, ib);
+        const int t = qa > qb ? ia : ib, mi = qa > qb ? ib : ia;
+        const double att = readlane_f64(dg, t), amm = readlane_f64(dg, mi);
+        const double *r1 = S + 32 * mi, *r2 = S + 32 * t;
+        const double a21 = r1[t];
+        bool two = false;
+        if (t != mi) {
+            const double delta = amm * att - a21 * a21;
+            two = fabs(delta) >= 0.5 * a21 * a21;
+        }
+        // the pivot's rows: a 2x2 takes mi to position cur, then t to cur + 1; a 1x1 the row with
+        // the larger diagonal to cur
+        const bool first = two || fabs(amm) >= fabs(att);
+        auto move_to = [&](int pos, int id) {
+            const int x = __builtin_amdgcn_readlane(idr, pos), q = __builtin_amdgcn_readlane(posr, id);
+            posr = (i == x) ? q : (i == id) ? pos : posr;
+            idr = (lane == q) ? x : idr;
+            idr = (lane == pos) ? id : idr;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) pj[u] = (jo[u] == x) ? q : (jo[u] == id) ? pos : pj[u];
+        };
+        move_to(cur, first ? mi : t);
+        if (!two) {
+            const double *rp = first ? r1 : r2;
+            const double d = first ? amm : att;
+            const double inv = 1.0 / d;
+            const double li = rp[i] * inv, wi = li * d;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const double lj = rp[jo[u]] * inv, wj = lj * d;
+                const double p1 = li * wj, p2 = lj * wi;
+                e[u] = e[u] - (posr > pj[u] ? p1 : p2);
+            }
+            dg = dg - li * wi;
+            ml = max_abs(ml, li);
+            lbuf[i][cur] = li;
+            kindr = (lane == cur) ? 1 : kindr;
+            bdr = (lane == cur) ? d : bdr;
             cur += 1;
         } else {
-            // mi goes to position cur, then t to cur + 1 (t stands at mi's old position if it was
-            // the row at cur)
-            const double *r1 = S + 32 * mi, *r2 = S + 32 * t;
-            const double a11 = amm, a22 = att, a21 = r1[t];
-            const double ci1 = r1[i], ci2 = r2[i];
-            double cj1[8], cj2[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) { cj1[u] = r1[jo[u]]; cj2[u] = r2[jo[u]]; }
-            posr = (i == x1) ? pm : posr;
-            posr = (i == mi) ? cur : posr;
-            idr = (lane == pm) ? x1 : idr;
-            idr = (lane == cur) ? mi : idr;
-            const int x2 = __builtin_amdgcn_readlane(idr, cur + 1), p2s = __builtin_amdgcn_readlane(posr, t);
-            posr = (i == x2) ? p2s : posr;
-            posr = (i == t) ? cur + 1 : posr;
-            idr = (lane == p2s) ? x2 : idr;
-            idr = (lane == cur + 1) ? t : idr;
-            ptab[i] = posr;
-            wave_sync();
-            int pj[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) pj[u] = ptab[jo[u]];
+            move_to(cur + 1, t);
+            const double a11 = amm, a22 = att;
             const double inv_det = 1.0 / (a11 * a22 - a21 * a21);
+            const double ci1 = r1[i], ci2 = r2[i];
             const double l1i = (ci1 * a22 - ci2 * a21) * inv_det;
             const double l2i = (ci2 * a11 - ci1 * a21) * inv_det;
             const double w1i = l1i * a11 + l2i * a21, w2i = l1i * a21 + l2i * a22;
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const double l1j = (cj1[u] * a22 - cj2[u] * a21) * inv_det;
-                const double l2j = (cj2[u] * a11 - cj1[u] * a21) * inv_det;
+                const double cj1 = r1[jo[u]], cj2 = r2[jo[u]];
+                const double l1j = (cj1 * a22 - cj2 * a21) * inv_det;
+                const double l2j = (cj2 * a11 - cj1 * a21) * inv_det;
                 const double w1j = l1j * a11 + l2j * a21, w2j = l1j * a21 + l2j * a22;
                 const double p1 = l1i * w1j + l2i * w2j, p2 = l1j * w1i + l2j * w2i;
                 e[u] = e[u] - (posr > pj[u] ? p1 : p2);
             }
             dg = dg - (l1i * w1i + l2i * w2i);
             ml = max_abs(max_abs(ml, l1i), l2i);
-            if (h == 0) { lbuf[i][cur] = l1i; lbuf[i][cur + 1] = l2i; }
-            if (lane == 0) {
-                bkind[cur] = 2; bkind[cur + 1] = 3;
-                bdiag[cur] = a11; bdiag[cur + 1] = a22; boff[cur] = a21;
-            }
+            lbuf[i][cur] = l1i;
+            lbuf[i][cur + 1] = l2i;
+            kindr = (lane == cur) ? 2 : (lane == cur + 1) ? 3 : kindr;
+            bdr = (lane == cur) ? a11 : (lane == cur + 1) ? a22 : bdr;
+            bor = (lane == cur) ? a21 : bor;
             cur += 2;
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) { S[w1[u]] = e[u]; S[w2[u]] = e[u]; }
         wave_sync();
+        cur = __builtin_amdgcn_readfirstlane(cur);
+        more = cur < bs;
     }
     if (lane < MAX_IB) {
         bp[lane] = idr;
         S[33 * i] = dg;
+        bkind[lane] = (int8_t)kindr;
+        bdiag[lane] = bdr;
+        boff[lane] = bor;
     }
     *maxl = wave_max_dpp(ml);
     return cur;
@@ -640,7 +709,7 @@ __device__ __forceinline__ int block_factor_wg(double (*blk)[MAX_IB + 1], double
     if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) {
         __builtin_amdgcn_s_setprio(3);
         double ml;
-        const int kk = block_pivots(blk, S, bp, bp2, bkind, bdiag, boff, bs, small, &ml, lbuf);
+        const int kk = block_pivots(blk, S, bp, bkind, bdiag, boff, bs, small, &ml, lbuf);
         __builtin_amdgcn_s_setprio(0);
         if (tid == 0) { wbv[0] = ml; wbp[0] = kk; }
     } else {
@@ -1510,6 +1579,8 @@ struct ChainSync {
                                             // wavefronts of the leader that store its tile; aux:
                                             // its first failing column (INT_MAX before)
     ChainCounter updated[CHAIN_MAX_IT];     // panels done with the updates of block it
+    ChainCounter early[CHAIN_MAX_IT];       // panels that own rows of the block after the next and
+                                            // have updated their first columns (no column failed)
     ChainRec recs[CHAIN_MAX_IT];
 };
 
@@ -1520,6 +1591,7 @@ __device__ __forceinline__ void chain_reset(ChainSync &C) {
         C.applied[i].v = 0;
         C.applied[i].aux = INT_MAX;
         C.updated[i].v = 0;
+        C.early[i].v = 0;
     }
 }
 
@@ -1632,20 +1704,6 @@ __device__ __forceinline__ bool chain_wait_aux(ChainCounter &c, int target, int 
     const bool ok = s_ok != 0;
     __syncthreads();  // s_ok is read by all before the next wait writes it
     return ok;
-}
-
-// A value the compiler has to take as new: address arithmetic formed from it is neither hoisted
-// out of the block loop nor kept from one phase to the next.  (Left to itself the compiler holds
-// some hundred loop-invariant offsets of the unrolled loads and stores below in registers across
-// the loop and spills the data instead: 440 spilled registers, 39 us per substitution.)
-__device__ __forceinline__ int fresh(int x) {
-    __asm__ volatile("" : "+v"(x));
-    return x;
-}
-__device__ __forceinline__ int fresh_uniform(int x) {
-    x = __builtin_amdgcn_readfirstlane(x);
-    __asm__ volatile("" : "+s"(x));
-    return x;
 }
 
 // One wavefront: wait until c.v >= target; *aux receives the aux read with it.  False when the
@@ -1949,9 +2007,11 @@ __device__ __forceinline__ void load_operands(ChainLeaderLds &L, const gdouble *
 // operands of the block after the next into LDS, and before them two wavefronts store the current
 // block's tile while the other two substitute.  The record is written before the checks are known;
 // a failed column discards it and the block factored ahead.
+template <int CH>
 __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSync &C, ChainLeaderLds &L, int nit, int NP,
                              int ib, double small) {
     const int tid = threadIdx.x;
+    const int ob_start = S.ob_start;
     const int m = F.m;
     const size_t lda = m;
     gdouble *A = gbl(F.F);
@@ -2063,7 +2123,14 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
                 int aux;
                 if (!wave_poll(C.applied[it], NP + 2, &C.err.v, &aux)) { L.s_err = 1; return; }
                 if (aux < bs) return;
-                if (!wave_poll(C.updated[it], NP, &C.err.v, &aux)) { L.s_err = 1; return; }
+                // the panels that own the rows report their first columns early; with several chunks
+                // per panel the whole update is awaited
+                const bool single = (m - ob_start + CH - 1) / CH <= NP;
+                const int own = (be2 + nbs2 - 1 - ob_start) / CH == (be2 - ob_start) / CH ? 1 : 2;
+                if (!wave_poll(single ? C.early[it] : C.updated[it], single ? own : NP, &C.err.v, &aux)) {
+                    L.s_err = 1;
+                    return;
+                }
                 load_operands<192>(L, A, lda, perm, be, nbs, be2, nbs2, tid - 64);
                 if (tid == 64) L.s_pf = 1;
             });
@@ -2121,7 +2188,6 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
             bn = bn2;
             k = be;
             have = true;
-            if (pf) upd_prev = true;
         } else {
             have = false;
             if (bn == 0 || nelim < bs) {
@@ -2390,6 +2456,7 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
             const int nbs = min(end_pos - be, ib);
             const bool ahead = nelim == bs && nbs > 0 && it + 1 < nit;
             const int lead = ahead ? be + nbs : be;
+            const int be2 = be + nbs, nbs2 = min(end_pos - be2, ib);
             const int nf = bs - nelim;
             double ml = 0.0;
             // a panel without rows below the block has nothing to do when no column failed
@@ -2413,6 +2480,13 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
                     double acc[4][8];
                     cu_sums(acc, L.WT[(R0 - r0p) >> 6], L.LcT, nelim);
                     cu_store(cv, acc, rc, lda, R0, r1p, c0, ncol, be, lead);
+                    if (ahead && c0 == be && R0 < be2 + nbs2 && min(R0 + 64, r1p) > be2 && (R0 + 64 >= be2 + nbs2 || R0 + 64 >= r1p)) {
+                        // (uniform) the leader's operands: rows of the block after the next, the last
+                        // of this panel's sub-tiles that hold some
+                        stores_done_barrier();
+                        if (tid == 0)
+                            __hip_atomic_fetch_add(&C.early[it].v, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
                     R0 = R1;
                     c0 = c1;
                     if (!more) break;
@@ -2542,7 +2616,10 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
         // block rows permuted in the columns factored before this block, this panel's share: with
         // failed columns before the panel reports (the leader then moves some of these rows), else
         // after (the rows are final)
-        auto permute_rows = [&] {
+        auto permute_rows = [&]() -> bool {
+            if (k == 0 || bs <= 0) return true;
+            // a panel may still read these rows for its update by the block before
+            if (it > 0 && !chain_wait(&C.updated[it - 1].v, NP, &C.err.v)) return false;
             const int per = (k + NP - 1) / NP;
             const int cb = pidx * per, ce = min(k, cb + per);
             const int i = tid & 31, half = (tid >> 5) & 1, wv = tid >> 6;
@@ -2565,8 +2642,9 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
                     }
                 }
             }
+            return true;
         };
-        if (permute_from > 0) permute_rows();
+        if (permute_from > 0 && !permute_rows()) return;
         stores_done_barrier();
         if (tid == 0) __hip_atomic_fetch_add(&C.updated[it].v, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // without failed columns nothing moves: the next block starts at be, its rows can come now
@@ -2576,7 +2654,7 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
             pre_bs = min(end_pos - be, ib);
             load_rows(pidx, pre_k, pre_bs);
         }
-        if (permute_from == 0) permute_rows();
+        if (permute_from == 0 && !permute_rows()) return;
     }
 }
 
@@ -2593,7 +2671,7 @@ __global__ __launch_bounds__(256, 2) void k_aptp_outer(FrontDev *__restrict__ fr
     ChainSync &C = cs[itm.x];
     const int nit = (S.ob_cols + ib - 1) / ib;
     if (itm.y == 0) {
-        chain_leader(F, S, C, lds.ld, nit, itm.w, ib, small);
+        chain_leader<CH>(F, S, C, lds.ld, nit, itm.w, ib, small);
         if (threadIdx.x == 0 && co_ldi(&C.err.v)) atomicOr(&F.flags, FRONT_CHAIN_ERR);
     } else {
         chain_panel<CH>(F, S, C, lds.pn, itm.y - 1, itm.w, nit, ib, threshold);
