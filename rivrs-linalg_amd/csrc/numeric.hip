@@ -2801,7 +2801,6 @@ __global__ __launch_bounds__(256) void k_outer_next(FrontDev *__restrict__ fr,
 
 // ===========================================================================
 // Threshold partial pivoting (tpp_factor / tpp_factor_rect, factor.rs:2268-2947).
-// One wavefront per front; every lane follows the same control flow.
 // mode 0: whole front from column 0; mode 1: fallback from F.ne.
 // ===========================================================================
 // Raw buffer loads (gfx9 resource: stride 0, range-checked against num_records): an offset at or
@@ -2818,136 +2817,58 @@ __device__ __forceinline__ double buf_load_f64(__amdgpu_buffer_rsrc_t r, unsigne
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0));
 }
 
-constexpr int TPP_B = 4;  // rows per lane whose loads are issued together (a front below 256 rows: one batch)
-// TJ (template parameter of the update routines): columns of a trailing update per memory round
-// trip; more columns, fewer round trips, more registers (fewer wavefronts per SIMD)
-
-// Reductions over the NT threads of a workgroup (NT a multiple of 64; every thread calls them in
-// the same order): the wavefront result, then the wavefronts' results through LDS in wavefront
-// order.  Called in uniform control flow only.
-template <int NT>
-__device__ __forceinline__ double blk_fmax(double v) {
-    v = wave_fmax(v);
-    if constexpr (NT == 64) {
-        return v;
-    } else {
-        __shared__ double s_[NT / 64];
-        __syncthreads();
-        if ((threadIdx.x & 63) == 0) s_[threadIdx.x >> 6] = v;
-        __syncthreads();
-        double r = s_[0];
-#pragma unroll
-        for (int w = 1; w < NT / 64; ++w) r = fmax(r, s_[w]);
-        return r;
-    }
-}
-template <int NT>
-__device__ __forceinline__ bool blk_any(bool b) {
-    if constexpr (NT == 64) {
-        return __any(b);
-    } else {
-        return __syncthreads_or(b) != 0;
-    }
-}
-// larger value wins; equal values -> smaller index
-template <int NT>
-__device__ __forceinline__ void blk_argmax(double &v, int &idx) {
-    wave_argmax(v, idx);
-    if constexpr (NT > 64) {
-        __shared__ double sv_[NT / 64];
-        __shared__ int si_[NT / 64];
-        __syncthreads();
-        if ((threadIdx.x & 63) == 0) { sv_[threadIdx.x >> 6] = v; si_[threadIdx.x >> 6] = idx; }
-        __syncthreads();
-        v = sv_[0];
-        idx = si_[0];
-#pragma unroll
-        for (int w = 1; w < NT / 64; ++w)
-            if (sv_[w] > v || (sv_[w] == v && si_[w] < idx)) { v = sv_[w]; idx = si_[w]; }
-    }
+// Reductions over one wavefront (every lane active), the result in all lanes.  max_abs: magnitudes,
+// NaN ignored.
+__device__ __forceinline__ double wave_max_abs(double v) {
+    v = max_abs(v, dpp_f64<0xB1>(v));
+    v = max_abs(v, dpp_f64<0x4E>(v));
+    v = max_abs(v, dpp_f64<0x141>(v));
+    v = max_abs(v, dpp_f64<0x140>(v));
+    return max_abs(max_abs(readlane_f64(v, 0), readlane_f64(v, 16)), max_abs(readlane_f64(v, 32), readlane_f64(v, 48)));
 }
 
-// A: the front (its first n columns are read and written).
-template <class P, int NT = 64>
-struct TppCtx {
+// A front from its first uneliminated column on, in local indices: m rows, n fully-summed columns,
+// lower triangle, column-major.  P: LDS (a staged front) or global memory.
+template <class P>
+struct TppMat {
     P A;
-    size_t lda;
-    int m, n;  // rows, fully-summed columns
-    int lane;
+    size_t ld;
+    int m, n;
+    __device__ __forceinline__ size_t at(int r, int q) const {
+        return (r >= q) ? r + q * ld : q + r * ld;
+    }
 };
 
-template <class P, int NT>
-__device__ __forceinline__ double tpp_sym(const TppCtx<P, NT> &c, int r, int q) {
-    return (r >= q) ? c.A[r + q * c.lda] : c.A[q + r * c.lda];
-}
+// Pivot tests by one wavefront each (threshold partial pivoting's candidates are independent until
+// one is taken, so a workgroup tests as many at once as it has wavefronts).
+constexpr int TPP_B = 4;  // entries per lane whose loads are issued together (a line below 256: one batch)
 
-// Column idx from row `from` (its row part [from, idx), then its column part [idx, m)) holds no
-// entry of magnitude >= small.  Both parts go through one batch of loads per pass.
-template <class P, int NT>
-__device__ bool tpp_col_small(const TppCtx<P, NT> &c, int idx, int from, double small) {
-    bool big = false;
-    const int nrow = idx - from, tot = nrow + (c.m - idx);
-    for (int e0 = c.lane; e0 < tot; e0 += NT * TPP_B) {
-        double v[TPP_B];
-#pragma unroll
-        for (int t = 0; t < TPP_B; ++t) {
-            const int e = e0 + NT * t;
-            const size_t off = (e < nrow) ? idx + (size_t)(from + e) * c.lda : (size_t)(idx + e - nrow) + idx * c.lda;
-            v[t] = (e < tot) ? fabs(c.A[off]) : 0.0;
-        }
-#pragma unroll
-        for (int t = 0; t < TPP_B; ++t)
-            if (e0 + NT * t < tot && v[t] >= small) big = true;
-    }
-    return !blk_any<NT>(big);
-}
-
-template <class P, int NT>
-__device__ int tpp_row_abs_max(const TppCtx<P, NT> &c, int p, int from, int to) {
-    if (from >= to) return from;
-    const double f0 = fabs(tpp_sym(c, p, from));
-    double bv = -1.0;
-    int bi = INT_MAX;
-    for (int q0 = from + 1 + c.lane; q0 < to; q0 += NT * TPP_B) {
-        double v[TPP_B];
-#pragma unroll
-        for (int t = 0; t < TPP_B; ++t) v[t] = (q0 + NT * t < to) ? fabs(tpp_sym(c, p, q0 + NT * t)) : 0.0;
-#pragma unroll
-        for (int t = 0; t < TPP_B; ++t)  // ascending q per lane, as the one-by-one scan
-            if (q0 + NT * t < to && v[t] > bv) { bv = v[t]; bi = q0 + NT * t; }
-    }
-    blk_argmax<NT>(bv, bi);
-    if (f0 != f0) return from;
-    return (bi != INT_MAX && bv > f0) ? bi : from;
-}
-
-// max |entry| of row/column col from column nelim (row part [nelim, col), column part (col, m)),
-// index `exclude` left out; both parts go through one batch of loads per pass.
-template <class P, int NT>
-__device__ double tpp_rc_max_excl(const TppCtx<P, NT> &c, int col, int nelim, int exclude) {
+// max |entry| of line (row part left of it, column part below it) from index `from`, without the
+// diagonal and index ex; NaN ignored, 0 when there is none.  *big: one of them is >= small.
+template <class P>
+__device__ __forceinline__ double tpp_line_max(const TppMat<P> &M, int line, int from, int ex, double small = 0.0,
+                                               bool *big = nullptr) {
+    const int lane = threadIdx.x & 63;
     double best = 0.0;
-    const int nrow = col - nelim, tot = nrow + (c.m - col - 1);
-    for (int e0 = c.lane; e0 < tot; e0 += NT * TPP_B) {
+    bool b = false;
+    for (int q0 = from + lane; q0 < M.m; q0 += 64 * TPP_B) {
         double v[TPP_B];
-        int q[TPP_B];
+#pragma unroll
+        for (int t = 0; t < TPP_B; ++t) v[t] = M.A[M.at(line, min(q0 + 64 * t, M.m - 1))];
 #pragma unroll
         for (int t = 0; t < TPP_B; ++t) {
-            const int e = e0 + NT * t;
-            q[t] = (e < nrow) ? nelim + e : col + 1 + (e - nrow);  // the entry's other index
-            const size_t off = (e < nrow) ? col + (size_t)q[t] * c.lda : (size_t)q[t] + col * c.lda;
-            v[t] = (e < tot) ? fabs(c.A[off]) : 0.0;
+            const int q = q0 + 64 * t;
+            const bool in = q < M.m && q != line && q != ex;
+            best = in ? max_abs(best, v[t]) : best;
+            b |= in && fabs(v[t]) >= small;
         }
-#pragma unroll
-        for (int t = 0; t < TPP_B; ++t)
-            if (e0 + NT * t < tot && q[t] != exclude) best = fmax(best, v[t]);
     }
-    return blk_fmax<NT>(best);
+    if (big) *big = __any(b);
+    return wave_max_abs(best);
 }
 
-template <class P, int NT>
-__device__ bool tpp_test_2x2(const TppCtx<P, NT> &c, int t, int p, double maxt, double maxp, double u,
-                             double small) {
-    const double a11 = c.A[t + t * c.lda], a21 = c.A[p + t * c.lda], a22 = c.A[p + p * c.lda];
+__device__ __forceinline__ bool tpp_test_2x2(double a11, double a21, double a22, double maxt, double maxp, double u,
+                                             double small) {
     const double maxpiv = fmax(fmax(fabs(a11), fabs(a21)), fabs(a22));
     if (maxpiv < small) return false;
     const double detscale = 1.0 / maxpiv;
@@ -2964,270 +2885,346 @@ __device__ bool tpp_test_2x2(const TppCtx<P, NT> &c, int t, int p, double maxt, 
     return u * fmax(x1, x2) < 1.0;
 }
 
-template <class P, int NT>
-__device__ void tpp_swap(const TppCtx<P, NT> &c, gint *perm, int i, int j) {
+enum { TPP_NONE = 0, TPP_ZERO = 1, TPP_2X2 = 2, TPP_1X1 = 3 };
+
+// Candidate p (> from) of a step at column `from`: a column without an entry of magnitude >= small,
+// a 2x2 with t, the largest entry of its row among [from, p) (the first of equals), or a 1x1.
+template <class P>
+__device__ __forceinline__ int tpp_candidate(const TppMat<P> &M, int p, int from, double u, double small, int *tout) {
+    const int lane = threadIdx.x & 63;
+    // one pass over the line: per lane the row part's largest entry (first index), the largest of
+    // the rest kept per entry for the exclusion of t
+    double bv = -1.0, oth = 0.0;
+    int bi = INT_MAX;
+    bool big = false;
+    for (int q0 = from + lane; q0 < M.m; q0 += 64 * TPP_B) {
+        double v[TPP_B];
+#pragma unroll
+        for (int t = 0; t < TPP_B; ++t) v[t] = fabs(M.A[M.at(p, min(q0 + 64 * t, M.m - 1))]);
+#pragma unroll
+        for (int t = 0; t < TPP_B; ++t) {
+            const int q = q0 + 64 * t;
+            const bool row = q < p, up = row && v[t] > bv;
+            const double lose = up ? bv : v[t];  // what is not the lane's best of the row part
+            big |= q < M.m && v[t] >= small;
+            oth = (q != p && q < M.m && lose > oth) ? lose : oth;
+            bi = up ? q : bi;
+            bv = up ? v[t] : bv;
+        }
+    }
+    if (!__any(big)) return TPP_ZERO;
+    const double bm = wave_max_abs(bv < 0.0 ? 0.0 : bv);
+    const double f0 = fabs(M.A[M.at(p, from)]);
+    const unsigned long long hit = __ballot(bv == bm);
+    int t = from;
+    if (f0 == f0 && hit != 0)
+        t = (hit & (hit - 1)) == 0 ? __builtin_amdgcn_readlane(bi, __builtin_ctzll(hit))
+                                   : __builtin_amdgcn_readfirstlane(wave_min_int(bv == bm ? bi : INT_MAX));
+    const double app = M.A[p + p * M.ld], apt = M.A[M.at(p, t)], att = M.A[t + t * M.ld];
+    // max over the line without t: a lane whose own best is t gives its others
+    const double maxp = wave_max_abs(max_abs(oth, (bi == t || bv < 0.0) ? 0.0 : bv));
+    const double maxt = tpp_line_max(M, t, from, p);
+    *tout = t;
+    if (tpp_test_2x2(att, apt, app, maxt, maxp, u, small)) return TPP_2X2;
+    return (fabs(app) >= u * fmax(maxp, fabs(apt))) ? TPP_1X1 : TPP_NONE;
+}
+
+// Symmetric exchange of lines i < j (all threads; the pairs of line q are disjoint).
+template <int NT, class P>
+__device__ __forceinline__ void tpp_swap(const TppMat<P> &M, int *lperm, int i, int j) {
     if (i == j) return;
     if (i > j) { const int t = i; i = j; j = t; }
-    P A = c.A;
-    const size_t lda = c.lda;
-    // the pairs exchanged for line q (row parts left of i, between i and j, column parts below j)
-    // are disjoint: every load of a pass is issued before its stores
-    for (int q0 = c.lane; q0 < c.m; q0 += NT * TPP_B) {
+    for (int q0 = threadIdx.x; q0 < M.m; q0 += NT * TPP_B) {
         size_t a1[TPP_B], a2[TPP_B];
         double x1[TPP_B], x2[TPP_B];
 #pragma unroll
         for (int t = 0; t < TPP_B; ++t) {
             const int q = q0 + NT * t;
-            const bool ok = q < c.m && q != i && q != j;
-            a1[t] = !ok ? i + (size_t)i * lda : (q < i) ? i + (size_t)q * lda : (size_t)q + i * lda;
-            a2[t] = !ok ? i + (size_t)i * lda : (q < j) ? j + (size_t)q * lda : (size_t)q + j * lda;
-            x1[t] = A[a1[t]];
-            x2[t] = A[a2[t]];
+            const bool ok = q < M.m && q != i && q != j;
+            a1[t] = ok ? M.at(i, q) : i + i * M.ld;
+            a2[t] = ok ? M.at(j, q) : i + i * M.ld;
+            x1[t] = M.A[a1[t]];
+            x2[t] = M.A[a2[t]];
         }
 #pragma unroll
         for (int t = 0; t < TPP_B; ++t) {
             const int q = q0 + NT * t;
-            if (q < c.m && q != i && q != j) { A[a1[t]] = x2[t]; A[a2[t]] = x1[t]; }
+            if (q < M.m && q != i && q != j) { M.A[a1[t]] = x2[t]; M.A[a2[t]] = x1[t]; }
         }
     }
-    if (c.lane == 0) {
-        const double t = A[i + i * lda]; A[i + i * lda] = A[j + j * lda]; A[j + j * lda] = t;
-        const int pt = perm[i]; perm[i] = perm[j]; perm[j] = pt;
+    if (threadIdx.x == 0) {
+        const double t = M.A[i + i * M.ld]; M.A[i + i * M.ld] = M.A[j + j * M.ld]; M.A[j + j * M.ld] = t;
+        const int pt = lperm[i]; lperm[i] = lperm[j]; lperm[j] = pt;
     }
     __syncthreads();
 }
 
-template <int TJ, class P, int NT>
-__device__ double tpp_apply_1x1(const TppCtx<P, NT> &c, int ne) {
-    P A = c.A;
-    const size_t lda = c.lda;
-    const double d = A[ne + ne * lda];
-    const double inv = 1.0 / d;
+// Elimination of the 1x1 at ne (two = false) or the 2x2 at ne, ne + 1: the columns scaled to L, then
+// the fully-summed columns updated, TJ per wavefront and pass.  Returns the thread's largest |l|.
+template <int NT, int TJ, int RB, class P>
+__device__ __forceinline__ double tpp_apply(const TppMat<P> &M, int ne, bool two) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    P A = M.A;
+    const size_t ld = M.ld;
+    const int nx = ne + (two ? 2 : 1);
+    const double a11 = A[ne + ne * ld];
+    double a21 = 0.0, a22 = 0.0;
+    if (two) { a21 = A[(ne + 1) + ne * ld]; a22 = A[(ne + 1) + (ne + 1) * ld]; }
+    const double inv = 1.0 / (two ? a11 * a22 - a21 * a21 : a11);
     double ml = 0.0;
-    // TPP_B rows per lane at a time, every load of a batch before its stores
-    for (int i0 = ne + 1 + c.lane; i0 < c.m; i0 += NT * TPP_B) {
-        double v[TPP_B];
-#pragma unroll
-        for (int t = 0; t < TPP_B; ++t) v[t] = (i0 + NT * t < c.m) ? A[(i0 + NT * t) + ne * lda] : 0.0;
-#pragma unroll
-        for (int t = 0; t < TPP_B; ++t)
-            if (i0 + NT * t < c.m) {
-                const double l = v[t] * inv;
-                A[(i0 + NT * t) + ne * lda] = l;
-                ml = fmax(ml, fabs(l));
-            }
-    }
-    ml = blk_fmax<NT>(ml);
-    __syncthreads();
-    for (int i0 = ne + 1 + c.lane; i0 < c.m; i0 += NT * TPP_B) {
-        double li[TPP_B];
-#pragma unroll
-        for (int t = 0; t < TPP_B; ++t) li[t] = (i0 + NT * t < c.m) ? A[(i0 + NT * t) + ne * lda] : 0.0;
-        // TJ columns per memory round trip: their loads (range-checked buffer loads, zero
-        // outside the column's live rows: no branch, no wait per load) before any store
-        for (int j0 = ne + 1; j0 < c.n; j0 += TJ) {
-            const __amdgpu_buffer_rsrc_t rc = buf_rsrc((const double *)(A + (size_t)j0 * lda));
-            double ldl[TJ], cv[TJ][TPP_B];
-#pragma unroll
-            for (int q = 0; q < TJ; ++q) {
-                const int j = j0 + q;
-                ldl[q] = (j < c.n) ? A[j + ne * lda] * d : 0.0;
-#pragma unroll
-                for (int t = 0; t < TPP_B; ++t) {
-                    const int i = i0 + NT * t;
-                    const bool ok = j < c.n && i >= j && i < c.m;
-                    cv[q][t] = buf_load_f64(rc, ok ? (unsigned)(i + (size_t)q * lda) * 8u : BUF_OOB);
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < TJ; ++q) {
-                const int j = j0 + q;
-#pragma unroll
-                for (int t = 0; t < TPP_B; ++t) {
-                    const int i = i0 + NT * t;
-                    if (j < c.n && i >= j && i < c.m) A[i + j * lda] = cv[q][t] - li[t] * ldl[q];
-                }
-            }
-        }
-    }
-    __syncthreads();
-    return ml;
-}
-
-template <int TJ, class P, int NT>
-__device__ double tpp_apply_2x2(const TppCtx<P, NT> &c, int ne) {
-    P A = c.A;
-    const size_t lda = c.lda;
-    const double a11 = A[ne + ne * lda], a21 = A[(ne + 1) + ne * lda], a22 = A[(ne + 1) + (ne + 1) * lda];
-    const double det = a11 * a22 - a21 * a21;
-    const double inv_det = 1.0 / det;
-    double ml = 0.0;
-    for (int i0 = ne + 2 + c.lane; i0 < c.m; i0 += NT * TPP_B) {
+    for (int i0 = nx + tid; i0 < M.m; i0 += NT * TPP_B) {
         double v1[TPP_B], v2[TPP_B];
 #pragma unroll
         for (int t = 0; t < TPP_B; ++t) {
-            const int i = i0 + NT * t;
-            v1[t] = (i < c.m) ? A[i + ne * lda] : 0.0;
-            v2[t] = (i < c.m) ? A[i + (ne + 1) * lda] : 0.0;
+            const int i = min(i0 + NT * t, M.m - 1);
+            v1[t] = A[i + ne * ld];
+            v2[t] = two ? A[i + (ne + 1) * ld] : 0.0;
         }
 #pragma unroll
         for (int t = 0; t < TPP_B; ++t) {
             const int i = i0 + NT * t;
-            if (i < c.m) {
-                const double ai1 = v1[t], ai2 = v2[t];
-                const double l1 = (ai1 * a22 - ai2 * a21) * inv_det;
-                const double l2 = (ai2 * a11 - ai1 * a21) * inv_det;
-                A[i + ne * lda] = l1;
-                A[i + (ne + 1) * lda] = l2;
-                ml = fmax(fmax(ml, fabs(l1)), fabs(l2));
-            }
-        }
-    }
-    ml = blk_fmax<NT>(ml);
-    __syncthreads();
-    for (int i0 = ne + 2 + c.lane; i0 < c.m; i0 += NT * TPP_B) {
-        double l1[TPP_B], l2[TPP_B];
-#pragma unroll
-        for (int t = 0; t < TPP_B; ++t) {
-            const int i = i0 + NT * t;
-            l1[t] = (i < c.m) ? A[i + ne * lda] : 0.0;
-            l2[t] = (i < c.m) ? A[i + (ne + 1) * lda] : 0.0;
-        }
-        for (int j0 = ne + 2; j0 < c.n; j0 += TJ) {
-            const __amdgpu_buffer_rsrc_t rc = buf_rsrc((const double *)(A + (size_t)j0 * lda));
-            double wj1[TJ], wj2[TJ], cv[TJ][TPP_B];
-#pragma unroll
-            for (int q = 0; q < TJ; ++q) {
-                const int j = j0 + q;
-                const double lj1 = (j < c.n) ? A[j + ne * lda] : 0.0;
-                const double lj2 = (j < c.n) ? A[j + (ne + 1) * lda] : 0.0;
-                wj1[q] = lj1 * a11 + lj2 * a21;
-                wj2[q] = lj1 * a21 + lj2 * a22;
-#pragma unroll
-                for (int t = 0; t < TPP_B; ++t) {
-                    const int i = i0 + NT * t;
-                    const bool ok = j < c.n && i >= j && i < c.m;
-                    cv[q][t] = buf_load_f64(rc, ok ? (unsigned)(i + (size_t)q * lda) * 8u : BUF_OOB);
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < TJ; ++q) {
-                const int j = j0 + q;
-#pragma unroll
-                for (int t = 0; t < TPP_B; ++t) {
-                    const int i = i0 + NT * t;
-                    if (j < c.n && i >= j && i < c.m) A[i + j * lda] = cv[q][t] - (l1[t] * wj1[q] + l2[t] * wj2[q]);
-                }
+            if (i >= M.m) continue;
+            if (two) {
+                const double l1 = (v1[t] * a22 - v2[t] * a21) * inv;
+                const double l2 = (v2[t] * a11 - v1[t] * a21) * inv;
+                A[i + ne * ld] = l1;
+                A[i + (ne + 1) * ld] = l2;
+                ml = max_abs(max_abs(ml, l1), l2);
+            } else {
+                const double l = v1[t] * inv;
+                A[i + ne * ld] = l;
+                ml = max_abs(ml, l);
             }
         }
     }
     __syncthreads();
-    if (c.lane == 0) A[(ne + 1) + ne * lda] = 0.0;
+    for (int j0 = nx + wv * TJ; j0 < M.n; j0 += (NT / 64) * TJ) {
+        double w1[TJ], w2[TJ];
+#pragma unroll
+        for (int q = 0; q < TJ; ++q) {
+            const int j = min(j0 + q, M.n - 1);
+            const double lj1 = A[j + ne * ld];
+            if (two) {
+                const double lj2 = A[j + (ne + 1) * ld];
+                w1[q] = lj1 * a11 + lj2 * a21;
+                w2[q] = lj1 * a21 + lj2 * a22;
+            } else {
+                w1[q] = lj1 * a11;
+                w2[q] = 0.0;
+            }
+        }
+        // RB rows per lane at a time, every load of a batch before its stores
+        for (int i0 = j0 + lane; i0 < M.m; i0 += 64 * RB) {
+            double c[TJ][RB], l1[RB], l2[RB];
+#pragma unroll
+            for (int r = 0; r < RB; ++r) {
+                const int i = min(i0 + 64 * r, M.m - 1);
+                l1[r] = A[i + ne * ld];
+                l2[r] = two ? A[i + (ne + 1) * ld] : 0.0;
+#pragma unroll
+                for (int q = 0; q < TJ; ++q) c[q][r] = A[i + min(j0 + q, M.n - 1) * ld];
+            }
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+#pragma unroll
+                for (int q = 0; q < TJ; ++q) {
+                    const int i = i0 + 64 * r;
+                    const double x = two ? l1[r] * w1[q] + l2[r] * w2[q] : l1[r] * w1[q];
+                    if (j0 + q < M.n && i >= j0 + q && i < M.m) A[i + (j0 + q) * ld] = c[q][r] - x;
+                }
+        }
+    }
     __syncthreads();
+    if (two) {
+        if (tid == 0) A[(ne + 1) + ne * ld] = 0.0;
+        __syncthreads();
+    }
     return ml;
 }
 
-// Threshold partial pivoting of one front from column nelim (the wavefront of the calling
-// workgroup).
-template <int TJ, class P, int NT>
-__device__ void tpp_run(const TppCtx<P, NT> &c, FrontDev &F, int nelim, double u, double small) {
-    const int n = c.n;
-    gint *perm = gbl(F.perm);
-    int n1 = 0, n2 = 0;
-    double maxl = 0.0;
+// Threshold partial pivoting of a front's columns from c0 on.  Returns the columns eliminated; the
+// row order in lperm.
+template <int NT, int TJ, int RB, class P>
+__device__ __forceinline__ int tpp_run(const TppMat<P> &M, FrontDev &F, int c0, int *lperm, double u, double small) {
+    constexpr int NW = NT / 64;
+    __shared__ int s_code[NW], s_t[NW], s_ok;
+    __shared__ double s_ml[NW];
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = M.n;
+    int nelim = 0, n1 = 0, n2 = 0;
+    double ml = 0.0;
+    for (int i = tid; i < n; i += NT) lperm[i] = i;
+    __syncthreads();
     auto set1 = [&](int col, double v) {
-        if (c.lane == 0) { gbl(F.dkind)[col] = 1; gbl(F.ddiag)[col] = v; gbl(F.doff)[col] = 0.0; }
+        if (tid == 0) { gbl(F.dkind)[c0 + col] = 1; gbl(F.ddiag)[c0 + col] = v; gbl(F.doff)[c0 + col] = 0.0; }
     };
     while (nelim < n) {
-        if (tpp_col_small(c, nelim, nelim, small)) {
+        // rounds of candidates: in the first, wavefront 0 looks at column nelim itself
+        int code = TPP_NONE, p = nelim, t = nelim;
+        bool last_ok = false;
+        int base = nelim;
+        for (;;) {
+            const int c = base + wv;
+            int cd = TPP_NONE, ct = 0;
+            if (c == nelim) {
+                bool big;
+                const double mp = tpp_line_max(M, nelim, nelim, -1, small, &big);
+                const double d = fabs(M.A[nelim + nelim * M.ld]);
+                if (!big && !(d >= small)) cd = TPP_ZERO;
+                if ((tid & 63) == 0) s_ok = d >= u * mp;
+            } else if (c < n) {
+                cd = tpp_candidate(M, c, nelim, u, small, &ct);
+            }
+            if ((tid & 63) == 0) { s_code[wv] = cd; s_t[wv] = ct; }
+            __syncthreads();
+#pragma unroll
+            for (int w = NW - 1; w >= 0; --w)
+                if (s_code[w] != TPP_NONE) { code = s_code[w]; p = base + w; t = s_t[w]; }
+            last_ok = s_ok != 0;
+            __syncthreads();
+            base += NW;
+            if (code != TPP_NONE || base >= n) break;
+        }
+        code = __builtin_amdgcn_readfirstlane(code);
+        p = __builtin_amdgcn_readfirstlane(p);
+        t = __builtin_amdgcn_readfirstlane(t);
+        if (code == TPP_ZERO) {
+            tpp_swap<NT>(M, lperm, p, nelim);
             set1(nelim, 0.0);
             ++n1;
-            for (int r = nelim + 1 + c.lane; r < c.m; r += NT) c.A[r + nelim * c.lda] = 0.0;
+            for (int r = nelim + 1 + tid; r < M.m; r += NT) M.A[r + nelim * M.ld] = 0.0;
             __syncthreads();
             nelim += 1;
-            continue;
-        }
-        bool found = false;
-        for (int p = nelim + 1; p < n; ++p) {
-            if (tpp_col_small(c, p, nelim, small)) {
-                tpp_swap(c, perm, p, nelim);
-                set1(nelim, 0.0);
-                ++n1;
-                for (int r = nelim + 1 + c.lane; r < c.m; r += NT) c.A[r + nelim * c.lda] = 0.0;
-                __syncthreads();
-                nelim += 1;
-                found = true;
-                break;
+        } else if (code == TPP_2X2) {
+            tpp_swap<NT>(M, lperm, t, nelim);
+            const int np = (p == nelim) ? t : p;
+            tpp_swap<NT>(M, lperm, np, nelim + 1);
+            if (tid == 0) {
+                gbl(F.dkind)[c0 + nelim] = 2; gbl(F.dkind)[c0 + nelim + 1] = 3;
+                gbl(F.ddiag)[c0 + nelim] = M.A[nelim + nelim * M.ld];
+                gbl(F.ddiag)[c0 + nelim + 1] = M.A[(nelim + 1) + (nelim + 1) * M.ld];
+                gbl(F.doff)[c0 + nelim] = M.A[(nelim + 1) + nelim * M.ld]; gbl(F.doff)[c0 + nelim + 1] = 0.0;
             }
-            const int t = tpp_row_abs_max(c, p, nelim, p);
-            const double maxt = tpp_rc_max_excl(c, t, nelim, p);
-            const double maxp = tpp_rc_max_excl(c, p, nelim, t);
-            if (tpp_test_2x2(c, t, p, maxt, maxp, u, small)) {
-                tpp_swap(c, perm, t, nelim);
-                const int np = (p == nelim) ? t : p;
-                tpp_swap(c, perm, np, nelim + 1);
-                const double d11 = c.A[nelim + nelim * c.lda];
-                const double d21 = c.A[(nelim + 1) + nelim * c.lda];
-                const double d22 = c.A[(nelim + 1) + (nelim + 1) * c.lda];
-                __syncthreads();
-                const double ml = tpp_apply_2x2<TJ>(c, nelim);
-                if (c.lane == 0) {
-                    gbl(F.dkind)[nelim] = 2; gbl(F.dkind)[nelim + 1] = 3;
-                    gbl(F.ddiag)[nelim] = d11; gbl(F.ddiag)[nelim + 1] = d22;
-                    gbl(F.doff)[nelim] = d21; gbl(F.doff)[nelim + 1] = 0.0;
-                }
-                ++n2;
-                maxl = fmax(maxl, ml);
-                nelim += 2;
-                found = true;
-                break;
+            ml = max_abs(ml, tpp_apply<NT, TJ, RB>(M, nelim, true));
+            ++n2;
+            nelim += 2;
+        } else {
+            if (code == TPP_NONE) {  // the 1x1 test of column nelim itself comes last
+                if (!last_ok) break;
+                p = nelim;
             }
-            const double maxpt = fmax(maxp, fabs(tpp_sym(c, p, t)));
-            if (fabs(c.A[p + p * c.lda]) >= u * maxpt) {
-                tpp_swap(c, perm, p, nelim);
-                const double ml = tpp_apply_1x1<TJ>(c, nelim);
-                set1(nelim, c.A[nelim + nelim * c.lda]);
-                ++n1;
-                maxl = fmax(maxl, ml);
-                nelim += 1;
-                found = true;
-                break;
-            }
-        }
-        if (!found) {
-            const double mp = tpp_rc_max_excl(c, nelim, nelim, -1);
-            if (fabs(c.A[nelim + nelim * c.lda]) >= u * mp) {
-                const double ml = tpp_apply_1x1<TJ>(c, nelim);
-                set1(nelim, c.A[nelim + nelim * c.lda]);
-                ++n1;
-                maxl = fmax(maxl, ml);
-                nelim += 1;
-            } else {
-                break;
-            }
+            tpp_swap<NT>(M, lperm, p, nelim);
+            set1(nelim, M.A[nelim + nelim * M.ld]);
+            ml = max_abs(ml, tpp_apply<NT, TJ, RB>(M, nelim, false));
+            ++n1;
+            nelim += 1;
         }
     }
+    ml = wave_max_abs(ml);
+    if ((tid & 63) == 0) s_ml[wv] = ml;
     __syncthreads();
-    if (c.lane == 0) {
-        F.ne = nelim;
+    if (tid == 0) {
+        for (int w = 1; w < NW; ++w) ml = max_abs(ml, s_ml[w]);
+        F.ne = c0 + nelim;
         F.n1 += n1;
         F.n2 += n2;
-        atomic_max_nonneg(&F.max_l_bits, maxl);
+        atomic_max_nonneg(&F.max_l_bits, ml);
     }
+    return nelim;
 }
 
-// One wavefront per front, factored in place.  (Staging a front's first k columns in LDS was
-// measured slower on the leaf levels: the LDS per workgroup cut the wavefronts per CU more than the
-// shorter latency gained.)  TJ = 2 keeps three wavefronts per SIMD (levels with more fronts than
-// SIMDs); TJ = 8 takes a quarter of the update round trips (levels of few, larger fronts).
-template <int TJ, int NT>
+// LDS of a staged front: its trapezoid's columns with an odd leading dimension (rows and columns
+// are read without bank conflicts), and the row order.
+__host__ __device__ __forceinline__ size_t tpp_lds_bytes(int m, int n) {
+    return ((size_t)(m | 1) * n * 8 + (size_t)n * 4 + 15) / 16 * 16;
+}
+constexpr size_t TPP_LDS_MAX = 158 * 1024;  // beside the workgroup's static LDS
+constexpr size_t TPP_LDS_SMALL = 38 * 1024;  // four workgroups per CU
+
+// One workgroup per front: mode 0 the whole front, mode 1 the columns APTP left (from F.ne).  A
+// pivot step is a serial chain of scans, so its memory round trips decide: the columns still to
+// eliminate are staged in LDS where they fit (lds bytes; all but the widest fronts), otherwise the
+// front is worked on in place.  Rows of earlier columns follow the row order at the end.
+// KKT of side 16 (fronts up to 131 x 131): TPPA us a step, 26 us with every scan through L2 and a
+// workgroup reduction of its own.
+template <int NT, int TJ>
 __global__ __launch_bounds__(NT) void k_tpp(FrontDev *__restrict__ fr, const int *__restrict__ flist,
-                                            int mode, double u, double small) {
+                                            int mode, double u, double small, unsigned lds) {
+    extern __shared__ __align__(16) double dyn[];
     FrontDev &F = fr[flist[blockIdx.x]];
-    const int n = F.k, m = F.m;
-    const int nelim = (mode == 0) ? 0 : F.ne;
-    if (nelim >= n) return;
-    tpp_run<TJ>(TppCtx<gdouble *, NT>{gbl(F.F), (size_t)m, m, n, (int)threadIdx.x}, F, nelim, u, small);
+    const int c0 = (mode == 0) ? 0 : F.ne;
+    const int n = F.k - c0, m = F.m - c0;
+    if (n <= 0) return;
+    const size_t lda = F.m;
+    gdouble *G = gbl(F.F) + c0 + c0 * lda;
+    const int tid = threadIdx.x;
+    int *lperm;
+    if (tpp_lds_bytes(m, n) <= lds) {
+        const size_t ld = m | 1;
+        lperm = (int *)(dyn + ld * n);
+        for (int j0 = tid >> 6; j0 < n; j0 += NT / 64 * 4)
+            for (int i = (tid & 63); i < m; i += 64) {
+                double v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] = G[i + (size_t)min(j0 + q * (NT / 64), n - 1) * lda];
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (j0 + q * (NT / 64) < n) dyn[i + (j0 + q * (NT / 64)) * ld] = v[q];
+            }
+        __syncthreads();
+        tpp_run<NT, TJ, 2>(TppMat<double *>{dyn, ld, m, n}, F, c0, lperm, u, small);
+        for (int j = tid >> 6; j < n; j += NT / 64)
+            for (int i = j + (tid & 63); i < m; i += 64) G[i + (size_t)j * lda] = dyn[i + j * ld];
+    } else {
+        lperm = F.sidx + c0;  // (written by k_collect after the factorization)
+        tpp_run<NT, TJ, 4>(TppMat<gdouble *>{G, lda, m, n}, F, c0, lperm, u, small);
+    }
+    __syncthreads();
+    // perm and the earlier columns' rows [c0, c0 + n) in the new order, columns dealt to the wavefronts
+    // (one register per lane and 64 rows; every load of a column before its stores)
+    gint *perm = gbl(F.perm) + c0;
+    constexpr int RB = 16;
+    if (n <= 64 * RB) {
+        for (int q = (tid >> 6) - 1; q < c0; q += NT / 64) {
+            gdouble *col = gbl(F.F) + c0 + (size_t)max(q, 0) * lda;
+            double v[RB];
+            int pv[RB];
+#pragma unroll
+            for (int r = 0; r < RB; ++r) {
+                const int i = (tid & 63) + 64 * r;
+                if (i >= n) continue;
+                if (q < 0) pv[r] = perm[lperm[i]];
+                else v[r] = col[lperm[i]];
+            }
+            __builtin_amdgcn_s_waitcnt(0);
+#pragma unroll
+            for (int r = 0; r < RB; ++r) {
+                const int i = (tid & 63) + 64 * r;
+                if (i >= n) continue;
+                if (q < 0) perm[i] = pv[r];
+                else col[i] = v[r];
+            }
+        }
+    } else {
+        // more columns left over: one column per thread, cycle by cycle (from each cycle's smallest row)
+        for (int q = tid - 1; q < c0; q += NT) {
+            gdouble *col = gbl(F.F) + c0 + (size_t)max(q, 0) * lda;
+            for (int i = 0; i < n; ++i) {
+                int a = lperm[i];
+                while (a > i) a = lperm[a];
+                if (a < i || lperm[i] == i) continue;
+                const double v = col[i];
+                const int pv = q < 0 ? perm[i] : 0;
+                a = i;
+                for (int b; (b = lperm[a]) != i; a = b) {
+                    if (q < 0) perm[a] = perm[b];
+                    else col[a] = col[b];
+                }
+                if (q < 0) perm[a] = pv;
+                else col[a] = v;
+            }
+        }
+    }
 }
 
 // ===========================================================================
@@ -4573,6 +4570,17 @@ void NumericGPU::plan_level(int lv, bool reset_arena) {
     L.o_sch = stage_push(stg, sch.data(), sch.size());
     L.nsch = sch.size();
     const size_t o_maps = stage_push(stg, maps.data(), maps.size());
+    // (small: staged in LDS with four workgroups per CU)
+    auto tpp_need = [&](int s) { return tpp_lds_bytes(m_[s], k_[s]); };
+    const auto tpp_mid = std::stable_partition(tpp_list.begin(), tpp_list.end(),
+                                               [&](int s) { return tpp_need(s) <= TPP_LDS_SMALL; });
+    L.ntpp_small = tpp_mid - tpp_list.begin();
+    L.tpp_lds[0] = L.tpp_lds[1] = 0;
+    for (size_t i = 0; i < tpp_list.size(); ++i)
+        if (tpp_need(tpp_list[i]) <= TPP_LDS_MAX) {
+            size_t &b = L.tpp_lds[i < L.ntpp_small ? 0 : 1];
+            b = std::max(b, tpp_need(tpp_list[i]));
+        }
     L.o_tpp = stage_push(stg, tpp_list.data(), tpp_list.size());
     L.ntpp = tpp_list.size();
     L.o_aptp = stage_push(stg, aptp_list.data(), aptp_list.size());
@@ -4901,10 +4909,15 @@ void NumericGPU::enqueue_level(int lv, const double *d_val, const double *d_scal
                                (const EaItem *)D(L.o_ea[r]));
     // ---- TPP fronts ----
     if (L.ntpp) {
-        // a level of more fronts than SIMDs: one wavefront per front; otherwise a workgroup of four
-        const bool wide = L.ntpp > 1024;
-        hipLaunchKernelGGL((wide ? k_tpp<2, 64> : k_tpp<8, 256>), dim3((unsigned)L.ntpp), dim3(wide ? 64 : 256), 0,
-                           stream_, d_fr_, (const int *)D(L.o_tpp), 0, o_.threshold, o_.small);
+        // fronts whose staged columns leave room for several workgroups per CU first, then the rest
+        // (so that one wide front does not take the other fronts' residency)
+        for (int c = 0; c < 2; ++c) {
+            const size_t n = c ? L.ntpp - L.ntpp_small : L.ntpp_small;
+            if (!n) continue;
+            hipLaunchKernelGGL((k_tpp<256, 4>), dim3((unsigned)n), dim3(256), L.tpp_lds[c], stream_, d_fr_,
+                               (const int *)D(L.o_tpp) + (c ? L.ntpp_small : 0), 0, o_.threshold, o_.small,
+                               (unsigned)L.tpp_lds[c]);
+        }
     }
     // ---- APTP fronts ----
     if (na > 0) {
@@ -4990,7 +5003,8 @@ void NumericGPU::enqueue_level(int lv, const double *d_val, const double *d_scal
             la_pending = false;
         }
         if (o_.failed_pivot_tpp)
-            hipLaunchKernelGGL((k_tpp<8, 256>), dim3(na), dim3(256), 0, stream_, d_fr_, dl, 1, o_.threshold, o_.small);
+            hipLaunchKernelGGL((k_tpp<1024, 4>), dim3(na), dim3(1024), TPP_LDS_MAX, stream_, d_fr_, dl, 1, o_.threshold,
+                               o_.small, (unsigned)TPP_LDS_MAX);
     }
     // ---- kept factor columns of the pooled fronts: final from here on, read beside the
     // contribution GEMMs (which only read them) on stream2_, joined after the collect (measured
