@@ -1014,66 +1014,211 @@ __global__ __launch_bounds__(256) void k_block_apply(FrontDev *__restrict__ fr,
     RV_PHASE(0, 5);
 }
 
+__device__ __forceinline__ double co_ld(const gdouble *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void co_st(gdouble *p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int co_ldi(const int *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void co_sti(int *p, int v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Bulk device-coherent loads: a plain buffer load carrying the same sc1 cache-policy bit as a
+// device-scope atomic load, which the compiler batches like any other load (atomic loads are
+// issued one round trip at a time).  The base is wavefront-uniform, the byte offset per lane; the
+// resource's range turns an offset past it into zero.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t co_rsrc(const gdouble *base) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>((const double *)base), (short)0, 0x7FFFFFF0,
+                                             0x00020000);
+}
+__device__ __forceinline__ double co_ldb(__amdgpu_buffer_rsrc_t r, size_t off) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)(off * sizeof(double)), 0, 16));
+}
+// The same with the front's own end as the range (rows past a panel's last column would leave
+// it); co_stb drops a store whose offset lies past the range.
+constexpr unsigned CO_OOB = 0x7FFFFFF8u;  // (a column offset added to it stays past the range)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t co_rsrc_front(const gdouble *A, size_t lda, size_t off) {
+    const size_t left = (lda * lda - off) * sizeof(double);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>((const double *)(A + off)), (short)0,
+                                             (int)(left < 0x7FFFFFF0 ? left : 0x7FFFFFF0), 0x00020000);
+}
+__device__ __forceinline__ double co_ldo(__amdgpu_buffer_rsrc_t r, unsigned off) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 16));
+}
+__device__ __forceinline__ void co_stb(__amdgpu_buffer_rsrc_t r, unsigned off, double v) {
+    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, (int)off, 0, 16);
+}
+__device__ __forceinline__ double co_ldd(const double *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void co_std(double *p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// every thread's stores complete, then the workgroup barrier
+__device__ __forceinline__ void stores_done_barrier() {
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+}
+
 // ===========================================================================
-// Symmetric line permutation for a sequence of swap_symmetric calls (factor.rs:452-505):
-// the composite is a symmetric permutation touching at most 2*ib lines; the touched lines
-// are snapshot and rewritten from the snapshot.
+// Symmetric line permutation for a sequence of at most MAX_IB swap_symmetric calls (factor.rs:452-505):
+// the composite touches at most 2 MAX_IB lines U.  Outside U x U every other line q is independent:
+// a thread loads its q's entries of up to 32 touched lines (whole cycles of the permutation, all
+// loads of a round in flight) and stores them to the lines' new places; the U x U entries go
+// through S.swapbuf.  CO: device-scope accesses to the front (inside the persistent launch).
+// Out of line: its registers stay out of the callers' common path.  Snapshotting whole lines to
+// memory one element and round trip at a time took a quarter of the factorization of a KKT system
+// with many delays (side 45: 28.4 ms, 21.9 so).
 // ===========================================================================
-__device__ void apply_swaps(FrontDev &F, AptpState &S, const int *sa, const int *sb, int nsw,
-                            int *U, int *src, int *cnt, int *ptmp) {
-    const int tid = threadIdx.x;
+struct SwapLds {
+    int U[2 * MAX_IB];     // touched lines
+    int from[2 * MAX_IB];  // line i receives line from[i] (indices into U)
+    int ptmp[2 * MAX_IB];
+    int mv[2 * MAX_IB];    // moved lines cycle by cycle: destination index, + 64 where a cycle ends
+    int gend[2 * MAX_IB];  // rounds of at most MAX_IB moves (whole cycles): end in mv
+    int n, nmv, ng;        // (ng = 0: a cycle of more than MAX_IB lines)
+};
+template <bool CO>
+__device__ __attribute__((noinline)) void apply_swaps(FrontDev &F, AptpState &S, const int *sa, const int *sb, int nsw,
+                                                      SwapLds &W) {
+    static_assert(MAX_IB == 32, "a touched line per lane");
+    constexpr int AUX = CO ? 16 : 0;
+    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+    const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int m = F.m;
     const size_t lda = m;
     gdouble *A = gbl(F.F);
-    if (tid == 0) {
-        int nU = 0;
+    if (wv == 0) {
+        // lane i: touched line i and the line whose content it ends with
+        int line = -1, from = lane, nU = 0;
+        const int la = lane < nsw ? sa[lane] : 0, lb = lane < nsw ? sb[lane] : 0;
         for (int s = 0; s < nsw; ++s) {
-            const int x = sa[s], y = sb[s];
-            int ix = -1, iy = -1;
-            for (int u = 0; u < nU; ++u) {
-                if (U[u] == x) ix = u;
-                if (U[u] == y) iy = u;
+            const int x = __builtin_amdgcn_readlane(la, s), y = __builtin_amdgcn_readlane(lb, s);
+            auto find = [&](int v) {
+                const unsigned long long hit = __ballot(lane < nU && line == v);
+                if (hit) return (int)__builtin_ctzll(hit);
+                line = (lane == nU) ? v : line;
+                return nU++;
+            };
+            const int ix = find(x), iy = find(y);
+            const int fx = __builtin_amdgcn_readlane(from, ix), fy = __builtin_amdgcn_readlane(from, iy);
+            from = (lane == ix) ? fy : (lane == iy) ? fx : from;
+        }
+        W.U[lane] = line;
+        W.from[lane] = from;
+        // the cycles, dealt to rounds
+        unsigned long long left = __ballot(from != lane);
+        int k = 0, g0 = 0, ng = 0;
+        bool longc = false;
+        while (left) {
+            const int first = __builtin_ctzll(left), k0 = k;
+            int c = first;
+            do {
+                left &= ~(1ull << c);
+                const int nx = __builtin_amdgcn_readlane(from, c);
+                if (lane == 0) W.mv[k] = c + (nx == first ? 64 : 0);
+                ++k;
+                c = nx;
+            } while (c != first);
+            longc |= k - k0 > MAX_IB;
+            if (k - g0 > MAX_IB) {
+                if (lane == 0) W.gend[ng] = k0;
+                ++ng;
+                g0 = k0;
             }
-            if (ix < 0) { U[nU] = x; src[nU] = x; ix = nU++; }
-            if (iy < 0) { U[nU] = y; src[nU] = y; iy = nU++; }
-            const int t = src[ix]; src[ix] = src[iy]; src[iy] = t;
         }
-        *cnt = nU;
+        if (lane == 0) {
+            W.gend[ng] = k;
+            W.n = nU;
+            W.nmv = k;
+            W.ng = longc ? 0 : ng + 1;
+        }
     }
     __syncthreads();
-    const int nU = *cnt;
-    if (nU == 0) return;
-    gint *mark = gbl(S.mark);
+    const int nU = __builtin_amdgcn_readfirstlane(W.n), nmv = __builtin_amdgcn_readfirstlane(W.nmv);
+    if (nmv == 0) return;
     gdouble *buf = gbl(S.swapbuf);
-    for (int u = tid; u < nU; u += blockDim.x) mark[U[u]] = u + 1;
-    for (int e = tid; e < nU * m; e += blockDim.x) {
-        const int ui = e / m, q = e % m;
-        const int u = U[ui];
-        buf[e] = (u >= q) ? A[u + q * lda] : A[q + u * lda];
+    const bool near = (size_t)m * m < (1u << 27);  // the front's offsets fit a buffer resource
+    const __amdgpu_buffer_rsrc_t ra = co_rsrc(A);
+    for (int e0 = tid; e0 < nU * nU; e0 += nt * 8) {
+        double v[8];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const int e = e0 + nt * r, x = e < nU * nU ? e / nU : 0, y = e < nU * nU ? e % nU : 0;
+            const size_t off = W.U[x] + (size_t)W.U[y] * lda;
+            const bool ok = e < nU * nU && W.U[x] >= W.U[y];
+            if (near)
+                v[r] = __builtin_bit_cast(
+                    double, __builtin_amdgcn_raw_buffer_load_b64(ra, (int)(ok ? (unsigned)off * 8u : CO_OOB), 0, AUX));
+            else
+                v[r] = ok ? co_ld(A + off) : 0.0;
+        }
+#pragma unroll
+        for (int r = 0; r < 8; ++r)
+            if (e0 + nt * r < nU * nU) buf[e0 + nt * r] = v[r];
     }
-    if (tid < nU) ptmp[tid] = gbl(F.perm)[U[tid]];
+    if (tid < nU) W.ptmp[tid] = gbl(F.perm)[W.U[tid]];
     __syncthreads();
-    for (int pi = 0; pi < nU; ++pi) {
-        const int p = U[pi];
-        const int sp = src[pi];
-        if (sp == p) continue;
-        const int sidx = mark[sp] - 1;
-        const gdouble *line = buf + (size_t)sidx * m;
-        for (int q = tid; q < m; q += blockDim.x) {
-            const int mq = mark[q];
-            const int qs = mq ? src[mq - 1] : q;
-            const double v = line[qs];
-            if (p >= q) A[p + q * lda] = v; else A[q + p * lda] = v;
+    const int ul = W.U[lane], fl = W.from[lane], ml = W.mv[lane] & 63;
+    const int ng = near ? __builtin_amdgcn_readfirstlane(W.ng) : 0;
+    // (every lane stays active: the lines are read across the lanes)
+    for (int q0 = 64 * wv; q0 < m; q0 += nt) {
+        const int q = q0 + lane;
+        bool in = q < m;
+        for (int s = 0; s < nU; ++s) in = in && q != __builtin_amdgcn_readlane(ul, s);
+        int g0 = 0;
+        for (int g = 0; g < ng; ++g) {
+            const int g1 = __builtin_amdgcn_readfirstlane(W.gend[g]), n = g1 - g0;
+            double v[MAX_IB];
+#pragma unroll
+            for (int s = 0; s < MAX_IB; ++s)
+                if (s < n) {
+                    const int u = __builtin_amdgcn_readlane(ul, __builtin_amdgcn_readlane(fl, __builtin_amdgcn_readlane(ml, g0 + s)));
+                    const unsigned off = in ? 8u * ((unsigned)max(q, u) + (unsigned)min(q, u) * (unsigned)m) : CO_OOB;
+                    v[s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(ra, (int)off, 0, AUX));
+                }
+#pragma unroll
+            for (int s = 0; s < MAX_IB; ++s)
+                if (s < n) {
+                    const int u = __builtin_amdgcn_readlane(ul, __builtin_amdgcn_readlane(ml, g0 + s));
+                    const unsigned off = in ? 8u * ((unsigned)max(q, u) + (unsigned)min(q, u) * (unsigned)m) : CO_OOB;
+                    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v[s]), ra, (int)off, 0, AUX);
+                }
+            g0 = g1;
+        }
+        if (ng == 0 && in) {
+            // a long cycle, or a front past 8 GB: along each cycle, the first entry kept aside
+            double first = 0.0;
+            bool start = true;
+            for (int s = 0; s < nmv; ++s) {
+                const int w = W.mv[s], i = w & 63, u = W.U[i], f = W.U[W.from[i]];
+                gdouble *pu = A + max(q, u) + (size_t)min(q, u) * lda, *pf = A + max(q, f) + (size_t)min(q, f) * lda;
+                if (start) first = CO ? co_ld(pu) : *pu;
+                const double x = (w & 64) ? first : CO ? co_ld(pf) : *pf;
+                if (CO) co_st(pu, x);
+                else *pu = x;
+                start = (w & 64) != 0;
+            }
         }
     }
-    if (tid < nU) {
-        // new perm[p] = old perm[src[p]]
-        const int sp = src[tid];
-        gbl(F.perm)[U[tid]] = ptmp[mark[sp] - 1];
+    for (int e = tid; e < nU * nU; e += nt) {
+        const int x = e / nU, y = e % nU;
+        const int p = W.U[x], r = W.U[y];
+        if (p < r) continue;
+        const int fx = W.from[x], fy = W.from[y];
+        const double v = buf[W.U[fx] >= W.U[fy] ? fx * nU + fy : fy * nU + fx];
+        if (CO) co_st(A + p + (size_t)r * lda, v);
+        else A[p + (size_t)r * lda] = v;
     }
-    __syncthreads();
-    for (int u = tid; u < nU; u += blockDim.x) mark[U[u]] = 0;
-    __syncthreads();
+    if (tid < nU) gbl(F.perm)[W.U[tid]] = W.ptmp[W.from[tid]];
+    if (CO) stores_done_barrier();
+    else __syncthreads();
 }
 
 // Diagonal tile of the next inner block after this block's update, formed in LDS with the
@@ -1457,8 +1602,9 @@ __global__ __launch_bounds__(256) void k_block_finish(FrontDev *__restrict__ fr,
     const int k = S.kpos, bs = S.bs;
     const int nelim = (bn > 0) ? effective_nelim(S) : 0;
     const int nxv = S.nx_valid;
-    __shared__ int sa[MAX_IB], sb[MAX_IB], U[2 * MAX_IB], src[2 * MAX_IB], ptmp[2 * MAX_IB];
-    __shared__ int nsw, cnt, s_end;
+    __shared__ int sa[MAX_IB], sb[MAX_IB];
+    __shared__ SwapLds sw;
+    __shared__ int nsw, s_end;
     int is1 = 0, is2 = 0;
     if (tid < nelim) {
         const int kd = S.bkind[tid];
@@ -1496,7 +1642,7 @@ __global__ __launch_bounds__(256) void k_block_finish(FrontDev *__restrict__ fr,
         s_end = end_pos;
     }
     __syncthreads();
-    apply_swaps(F, S, sa, sb, nsw, U, src, &cnt, ptmp);
+    apply_swaps<false>(F, S, sa, sb, nsw, sw);
     if (tid == 0) {
         S.kpos = k + nelim;
         S.end_pos = s_end;
@@ -1593,57 +1739,6 @@ __device__ __forceinline__ void chain_reset(ChainSync &C) {
         C.updated[i].v = 0;
         C.early[i].v = 0;
     }
-}
-
-__device__ __forceinline__ double co_ld(const gdouble *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void co_st(gdouble *p, double v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ int co_ldi(const int *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void co_sti(int *p, int v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Bulk device-coherent loads: a plain buffer load carrying the same sc1 cache-policy bit as a
-// device-scope atomic load, which the compiler batches like any other load (atomic loads are
-// issued one round trip at a time).  The base is wavefront-uniform, the byte offset per lane; the
-// resource's range turns an offset past it into zero.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t co_rsrc(const gdouble *base) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>((const double *)base), (short)0, 0x7FFFFFF0,
-                                             0x00020000);
-}
-__device__ __forceinline__ double co_ldb(__amdgpu_buffer_rsrc_t r, size_t off) {
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)(off * sizeof(double)), 0, 16));
-}
-// The same with the front's own end as the range (rows past a panel's last column would leave
-// it); co_stb drops a store whose offset lies past the range.
-constexpr unsigned CO_OOB = 0x7FFFFFF8u;  // (a column offset added to it stays past the range)
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t co_rsrc_front(const gdouble *A, size_t lda, size_t off) {
-    const size_t left = (lda * lda - off) * sizeof(double);
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>((const double *)(A + off)), (short)0,
-                                             (int)(left < 0x7FFFFFF0 ? left : 0x7FFFFFF0), 0x00020000);
-}
-__device__ __forceinline__ double co_ldo(__amdgpu_buffer_rsrc_t r, unsigned off) {
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 16));
-}
-__device__ __forceinline__ void co_stb(__amdgpu_buffer_rsrc_t r, unsigned off, double v) {
-    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, (int)off, 0, 16);
-}
-__device__ __forceinline__ double co_ldd(const double *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void co_std(double *p, double v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// every thread's stores complete, then the workgroup barrier
-__device__ __forceinline__ void stores_done_barrier() {
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
 }
 
 // All threads: wait until *p >= target (thread 0 spins).  False when the front's wait ran out
@@ -1852,63 +1947,6 @@ __device__ __forceinline__ void quad_ld(const double (&y)[8], const PivotCoef &P
     }
 }
 
-// Symmetric line permutation (apply_swaps) with device-scope accesses to the front.
-__device__ __forceinline__ void apply_swaps_co(FrontDev &F, AptpState &S, const int *sa, const int *sb, int nsw, int *U, int *src,
-                               int *cnt, int *ptmp) {
-    const int tid = threadIdx.x;
-    const int m = F.m;
-    const size_t lda = m;
-    gdouble *A = gbl(F.F);
-    if (tid == 0) {
-        int nU = 0;
-        for (int s = 0; s < nsw; ++s) {
-            const int x = sa[s], y = sb[s];
-            int ix = -1, iy = -1;
-            for (int u = 0; u < nU; ++u) {
-                if (U[u] == x) ix = u;
-                if (U[u] == y) iy = u;
-            }
-            if (ix < 0) { U[nU] = x; src[nU] = x; ix = nU++; }
-            if (iy < 0) { U[nU] = y; src[nU] = y; iy = nU++; }
-            const int t = src[ix]; src[ix] = src[iy]; src[iy] = t;
-        }
-        *cnt = nU;
-    }
-    __syncthreads();
-    const int nU = *cnt;
-    if (nU == 0) return;
-    gint *mark = gbl(S.mark);
-    gdouble *buf = gbl(S.swapbuf);
-    for (int u = tid; u < nU; u += blockDim.x) mark[U[u]] = u + 1;
-    for (int e = tid; e < nU * m; e += blockDim.x) {
-        const int ui = e / m, q = e % m;
-        const int u = U[ui];
-        buf[e] = (u >= q) ? co_ld(A + u + q * lda) : co_ld(A + q + u * lda);
-    }
-    if (tid < nU) ptmp[tid] = gbl(F.perm)[U[tid]];
-    __syncthreads();
-    for (int pi = 0; pi < nU; ++pi) {
-        const int p = U[pi];
-        const int sp = src[pi];
-        if (sp == p) continue;
-        const int sidx = mark[sp] - 1;
-        const gdouble *line = buf + (size_t)sidx * m;
-        for (int q = tid; q < m; q += blockDim.x) {
-            const int mq = mark[q];
-            const int qs = mq ? src[mq - 1] : q;
-            const double v = line[qs];
-            if (p >= q) co_st(A + p + q * lda, v); else co_st(A + q + p * lda, v);
-        }
-    }
-    if (tid < nU) {
-        const int sp = src[tid];
-        gbl(F.perm)[U[tid]] = ptmp[mark[sp] - 1];
-    }
-    __syncthreads();
-    for (int u = tid; u < nU; u += blockDim.x) mark[U[u]] = 0;
-    stores_done_barrier();
-}
-
 struct ChainLeaderLds {
     double blk[MAX_IB][MAX_IB + 1];      // the current block, factored (L11)
     double Ct[MAX_IB][MAX_IB + 1];       // the next block's tile, factored ahead
@@ -1922,8 +1960,9 @@ struct ChainLeaderLds {
     PivotCoef pc;
     double wbv[1];
     int wbp[1];
-    int sa[MAX_IB], sb[MAX_IB], U[2 * MAX_IB], src[2 * MAX_IB], ptmp[2 * MAX_IB];
-    int nsw, cnt, s_end, s_fail, s_upd, s_pf, s_err;
+    int sa[MAX_IB], sb[MAX_IB];
+    SwapLds sw;
+    int nsw, s_end, s_fail, s_upd, s_pf, s_err;
 };
 constexpr int CHAIN_LC_COLS = 128;  // trailing columns per round of the panel update
 struct ChainPanelLds {
@@ -2214,7 +2253,7 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
                 }
                 __syncthreads();
                 end_pos = L.s_end;
-                apply_swaps_co(F, S, L.sa, L.sb, L.nsw, L.U, L.src, &L.cnt, L.ptmp);
+                apply_swaps<true>(F, S, L.sa, L.sb, L.nsw, L.sw);
             }
             k += nelim;
         }
@@ -2708,9 +2747,9 @@ __device__ bool outer_end(FrontDev &F, AptpState &S, int ob, int nb, int la) {
     const bool two = p > nb;
     const int nouter = two ? (p + nb - 1) / nb : 1;
     if (ob >= nouter) return false;
-    __shared__ int sa[MAX_IB * 8], sb[MAX_IB * 8];
-    __shared__ int U[2 * MAX_IB], src[2 * MAX_IB], ptmp[2 * MAX_IB];
-    __shared__ int nsw, cnt;
+    __shared__ int sa[MAX_IB], sb[MAX_IB];
+    __shared__ SwapLds sw;
+    __shared__ int nsw;
     const int tid = threadIdx.x;
     if (!two) {
         if (tid == 0) F.ne = S.kpos;
@@ -2744,7 +2783,7 @@ __device__ bool outer_end(FrontDev &F, AptpState &S, int ob, int nb, int la) {
             nsw = n;
         }
         __syncthreads();
-        apply_swaps(F, S, sa, sb, nsw, U, src, &cnt, ptmp);
+        apply_swaps<false>(F, S, sa, sb, nsw, sw);
         done += cnt_sw;
     }
     __syncthreads();
@@ -2757,8 +2796,7 @@ __device__ bool outer_end(FrontDev &F, AptpState &S, int ob, int nb, int la) {
 }
 
 // The first outer block of every front of a level: the APTP state is installed from its staged
-// initial value (scratch pointers, fail_min = INT_MAX, the rest zero) and the front's swap marks
-// are cleared, then outer block 0 starts.
+// initial value (scratch pointers, fail_min = INT_MAX, the rest zero), then outer block 0 starts.
 __global__ __launch_bounds__(256) void k_outer_first(FrontDev *__restrict__ fr,
                                                      AptpState *__restrict__ st,
                                                      const AptpState *__restrict__ init,
@@ -2772,8 +2810,6 @@ __global__ __launch_bounds__(256) void k_outer_first(FrontDev *__restrict__ fr,
     const int *src = (const int *)&I;
     int *dst = (int *)&S;
     for (int i = threadIdx.x; i < (int)(sizeof(AptpState) / sizeof(int)); i += blockDim.x) dst[i] = src[i];
-    gint *mark = gbl(I.mark);
-    for (int i = threadIdx.x; i < F.m; i += blockDim.x) mark[i] = 0;
     __syncthreads();
     outer_begin(F, S, 0, nb, ib);
 }
@@ -3145,7 +3181,7 @@ constexpr size_t TPP_LDS_SMALL = 38 * 1024;  // four workgroups per CU
 // pivot step is a serial chain of scans, so its memory round trips decide: the columns still to
 // eliminate are staged in LDS where they fit (lds bytes; all but the widest fronts), otherwise the
 // front is worked on in place.  Rows of earlier columns follow the row order at the end.
-// KKT of side 16 (fronts up to 131 x 131): TPPA us a step, 26 us with every scan through L2 and a
+// KKT of side 16 (fronts up to 131 x 131): about 5 us a step, 26 us with every scan through L2 and a
 // workgroup reduction of its own.
 template <int NT, int TJ>
 __global__ __launch_bounds__(NT) void k_tpp(FrontDev *__restrict__ fr, const int *__restrict__ flist,
@@ -4770,10 +4806,9 @@ void NumericGPU::plan_level(int lv, bool reset_arena) {
     L.doffs.assign(nf + 1, 0);
     for (int li = 0; li < nf; ++li) L.doffs[li + 1] = L.doffs[li] + std::max(k_[fronts[li]], 1);
     L.o_doffs = stage_push(stg, L.doffs.data(), L.doffs.size());
-    // APTP state and scratch: backup (m x ib), swap lines (2 ib x m), line marks (m)
+    // APTP state and scratch: backup (m x ib), touched lines' crossings of a permutation
     if (na > 0) {
         std::vector<AptpState> hs(na);
-        size_t markbytes = 0;
         for (int li = 0; li < na; ++li) {
             AptpState &S = hs[li];
             std::memset(&S, 0, sizeof(S));
@@ -4781,15 +4816,7 @@ void NumericGPU::plan_level(int lv, bool reset_arena) {
             const int m = m_[aptp_list[li]];
             S.backup = (double *)scratch_.alloc((size_t)m * ib * sizeof(double));
             S.blkcopy = (double *)scratch_.alloc((size_t)MAX_IB * MAX_IB * sizeof(double));
-            S.swapbuf = (double *)scratch_.alloc((size_t)2 * MAX_IB * m * sizeof(double));
-            markbytes += ((size_t)m * sizeof(int) + 255) / 256 * 256;
-        }
-        L.mark_p = (char *)scratch_.alloc(markbytes);
-        L.mark_bytes = markbytes;
-        size_t mo = 0;
-        for (int li = 0; li < na; ++li) {
-            hs[li].mark = (int *)(L.mark_p + mo);
-            mo += ((size_t)m_[aptp_list[li]] * sizeof(int) + 255) / 256 * 256;
+            S.swapbuf = (double *)scratch_.alloc((size_t)4 * MAX_IB * MAX_IB * sizeof(double));
         }
         L.dS = (AptpState *)scratch_.alloc((size_t)na * sizeof(AptpState));
         L.dSnap[0] = (AptpState *)scratch_.alloc((size_t)na * sizeof(AptpState));

@@ -80,8 +80,7 @@ struct AptpState {
     double *blkcopy;  // the next inner block's lower ib x ib diagonal block (column-major,
                       // leading dimension MAX_IB), copied before k_block_apply writes the front
     double *backup;   // (m - kpos) x ib backup of the block column, lda = m
-    double *swapbuf;  // 2*ib lines of length m for symmetric line permutations
-    int *mark;        // length m, zero outside a permutation: 1 + index of a touched line
+    double *swapbuf;  // (2 MAX_IB)^2: crossings of the lines touched by a symmetric line permutation
 };
 
 // Work item of a tiled launch: front index plus tile coordinates.

@@ -187,8 +187,6 @@ private:
         size_t res_bytes = 0, res_del_off = 0;
         char *hres = nullptr;     // pinned copy of dres for the current run
         AptpState *dS = nullptr;
-        char *mark_p = nullptr;
-        size_t mark_bytes = 0;
         size_t o_ids = 0, o_lfr = 0, o_rows = 0, o_sch = 0, o_tpp = 0, o_aptp = 0, o_k2 = 0, o_k3 = 0,
                o_wp0 = 0, o_wp1 = 0, o_wp1b = 0, o_f0 = 0, o_f1 = 0, o_doffs = 0, o_hs = 0;
         // copies of the APTP states for outer updates run beside the next outer block (by
