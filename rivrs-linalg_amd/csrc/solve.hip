@@ -26,7 +26,11 @@
 //                        L[block C', block C]^T x_C' for the later blocks C' as they are
 //                        published, then the 128 x 128 transposed unit triangle.
 // A right-hand-side group of up to 8 columns shares every load of L.  All sums run in a fixed
-// order: results do not depend on scheduling.
+// order: results do not depend on scheduling, nor on the number of columns.
+//
+// A single right-hand side is bound by the chain of diagonal blocks (75 of them on the way to the
+// root of a Helmholtz 64^3 factor): a block's x is on its way to the next workgroup for about 2 us,
+// its products take half a microsecond and its triangles one.
 #pragma clang fp contract(off)
 
 #include <hip/hip_runtime.h>
@@ -45,7 +49,6 @@ namespace {
 
 constexpr int SB = 128;  // diagonal block of the blocked triangular solves (two 64-column halves)
 constexpr int GH = 256;  // L21 rows per backward column-chunk item
-constexpr int CW = 32;   // columns per streamed chunk of the forward row products (16 per half)
 constexpr long long SPIN_LIMIT = 1LL << 22;
 
 // Item kinds.  A front with one diagonal block and at most FUSE_R rows of L21 is one fused item
@@ -80,32 +83,24 @@ struct PlanDev {
     int nfront, nflag;
 };
 
-// Flags and counters, zeroed by k_solve_start; every array holds one slice per RHS group.
+// Counters, zeroed by k_solve_start; every array holds one slice per RHS group.
 struct SyncDev {
     int *tick;   // [2] ticket counters of the two sweeps
     int *err;    // [1] set when a wait exceeded its limit
-    int *fflag;  // forward: block solved
     int *fdone;  // forward: rows items of the front finished
-    int *bflag;  // backward: block solved
     int *bgc;    // backward: chunk items of the block finished
     int *bdone;  // backward: blocks of the front finished
 };
 
-__device__ __forceinline__ double readlane_f64(double v, int l) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)b, l);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
 // Data that one workgroup of a sweep writes and another reads within the same launch (x blocks,
 // Y, chunk partials) goes through device-coherent accesses: stores and loads with device scope
 // (they bypass the per-XCD L2, whose copies another XCD's writes would leave stale), so no cache
-// maintenance fence is needed.  A producer stores its data, waits until its stores have
-// completed (s_waitcnt), joins a workgroup barrier, and one thread then sets the flag or bumps the
-// counter with a device-scope atomic; a consumer's thread 0 spins on the flag with device-scope
-// loads, and after a workgroup barrier every thread reads the data with device-scope loads.
-// The factor L is never written during a solve and is read through the caches as usual.
+// maintenance fence is needed.  The blocks of x along the chain are polled themselves (UNSET,
+// below).  For the rest a producer stores its data, waits until its stores have completed
+// (s_waitcnt), joins a workgroup barrier, and one thread bumps a counter with a device-scope
+// atomic; a consumer's thread spins on the counter with device-scope loads, and after a workgroup
+// barrier every thread reads the data with device-scope loads.  The factor L is never written
+// during a solve and is read through the caches as usual.
 __device__ __forceinline__ double ld_co(const double *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -120,7 +115,7 @@ __device__ __forceinline__ void stores_done_barrier() {
     __syncthreads();
 }
 
-// Thread 0 waits until *p >= target; the caller follows with a workgroup barrier.
+// A thread waits until *p >= target; the caller follows with a workgroup barrier.
 __device__ __forceinline__ void wait_at_least(const int *p, int target, int *err) {
     long long it = 0;
     while (__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
@@ -134,12 +129,21 @@ __device__ __forceinline__ void wait_at_least(const int *p, int target, int *err
 }
 
 // after stores_done_barrier(), by one thread
-__device__ __forceinline__ void publish_set(int *p) {
-    __hip_atomic_store(p, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 __device__ __forceinline__ void publish_add(int *p) {
     __hip_atomic_fetch_add(p, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Blocks of x pass between workgroups without a flag: W and Xb start a solve filled with UNSET,
+// a signalling NaN that no arithmetic returns, and a reader polls the words it needs until none
+// is UNSET.  A flag costs the writer the wait for its stores and the reader a second trip.
+constexpr unsigned long long UNSET = 0x7FF4A5A55A5A5A4Aull;
+__device__ __forceinline__ unsigned long long ld_bits(const double *p) {
+    return __hip_atomic_load((const unsigned long long *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void publish_value(double *p, double v) {
+    unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    if (b == UNSET) b = 0x7FF8000000000000ull;  // (an input's own NaN)
+    __hip_atomic_store((unsigned long long *)p, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __device__ __forceinline__ int take_ticket(int *tick) {
@@ -149,45 +153,61 @@ __device__ __forceinline__ int take_ticket(int *tick) {
     return s_t;
 }
 
+// A solve's vectors hold group g of right-hand sides (nq columns from q0 = g wq on) in nq
+// consecutive entries per index, group after group: column q of index i is at
+// q0 total + i nq + (q - q0), and a gather of an index serves the whole group.
+
 // Start of a solve: x_perm[i] = rhs[perm_fwd[i]] (* s[i]) (solver.rs:396-410) for every RHS
-// column, and the sweeps' flags and counters cleared.
+// column, the sweeps' counters cleared, and the published vectors (W and Xb, nfill entries from
+// fill on) set to UNSET.
 __global__ void k_solve_start(const double *__restrict__ rhs, long long ld, double *__restrict__ xp, long long n,
-                              int nrhs, const int *__restrict__ pf, const double *__restrict__ s,
-                              int *__restrict__ sync, long long nsync) {
+                              int nrhs, int wq, const int *__restrict__ pf, const double *__restrict__ s,
+                              int *__restrict__ sync, long long nsync, unsigned long long *__restrict__ fill,
+                              long long nfill) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nsync) sync[i] = 0;
+    const int q0 = blockIdx.y * wq, nq = min(wq, nrhs - q0);
+    const long long step = (long long)gridDim.x * blockDim.x;
+    if (blockIdx.y == 0)
+        for (long long e = i; e < nsync; e += step) sync[e] = 0;
+    for (long long e = blockIdx.y * step + i; e < nfill; e += step * gridDim.y) fill[e] = UNSET;
     if (i >= n) return;
     const int p = pf[i];
     const double si = s ? s[i] : 1.0;
-    for (int q = 0; q < nrhs; ++q) {
-        double v = rhs[p + q * ld];
+#pragma unroll 4
+    for (int q = 0; q < nq; ++q) {
+        double v = rhs[p + (q0 + q) * ld];
         if (s) v *= si;
-        xp[i + q * n] = v;
+        xp[q0 * n + i * nq + q] = v;
     }
 }
 
 // rhs[perm_fwd[i]] = x_perm[i] (* s[i])  (solver.rs:416-425)
-__global__ void k_perm_out(double *__restrict__ rhs, long long ld, const double *__restrict__ xp,
-                           long long n, const int *__restrict__ pf, const double *__restrict__ s) {
+__global__ void k_perm_out(double *__restrict__ rhs, long long ld, const double *__restrict__ xp, long long n,
+                           int nrhs, int wq, const int *__restrict__ pf, const double *__restrict__ s) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int q = blockIdx.y;
+    const int q0 = blockIdx.y * wq, nq = min(wq, nrhs - q0);
     if (i >= n) return;
-    double v = xp[i + q * n];
-    if (s) v *= s[i];
-    rhs[pf[i] + q * ld] = v;
+    const int p = pf[i];
+    const double si = s ? s[i] : 1.0;
+#pragma unroll 4
+    for (int q = 0; q < nq; ++q) {
+        double v = xp[q0 * n + i * nq + q];
+        if (s) v *= si;
+        rhs[p + (q0 + q) * ld] = v;
+    }
 }
 
 // Pull of columns that no front eliminated (unresolved delays at the roots).
 __global__ void k_pull_rows(const int *__restrict__ rows, int nrows, const int *__restrict__ ptr,
                             const long long *__restrict__ ent, const double *__restrict__ Y,
-                            long long ytotal, double *__restrict__ x, long long n) {
+                            long long ytotal, double *__restrict__ x, long long n, int nrhs, int wq) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int q = blockIdx.y;
+    const int q0 = blockIdx.y / wq * wq, nq = min(wq, nrhs - q0), q = blockIdx.y - q0;
     if (i >= nrows) return;
     const int t = rows[i];
-    double v = x[t + q * n];
-    for (int e = ptr[t]; e < ptr[t + 1]; ++e) v -= Y[q * ytotal + ent[e]];
-    x[t + q * n] = v;
+    double v = x[q0 * n + (long long)t * nq + q];
+    for (int e = ptr[t]; e < ptr[t + 1]; ++e) v -= Y[q0 * ytotal + ent[e] * nq + q];
+    x[q0 * n + (long long)t * nq + q] = v;
 }
 
 // Inverses of the diagonal triangles.  Every 64 x 64 unit lower triangle T of L11 the solve
@@ -286,712 +306,781 @@ __global__ __launch_bounds__(64) void k_diag_inverse(const SolveFront *__restric
     invert_unit_lower<S>(Tt, rb, lda, n);
 }
 
-// The diagonal block [jb, jb + SB) in LDS: the inverses X_A, X_B of its two 64 x 64 unit lower
-// triangles (rows and columns jb..jb+63 and jb+64..jb+127) as compact strictly-lower triangles
-// (entry (r, c), c < r, at r (r - 1) / 2 + c), read from the block's upper triangle, and the tile
-// C = L[jb+64 : jb+128, jb : jb+64] between them (64 x 65, padded).  Thread (lane, quarter
-// q = tid >> 6) loads X entries (q + 4u, lane) and C entries (lane, q + 4u): lanes over
-// consecutive front rows in both (coalesced); the loads are issued at the start of an item, off
-// the chain.
-constexpr int TRI = 64 * 63 / 2;
-struct DiagLds {
-    double *tA, *tB;
-    double (*C)[65];
+// ---------------------------------------------------------------------------
+// Products on the matrix cores.  A workgroup serves W = 4 or 8 right-hand sides (nq <= W of them in
+// use); a wavefront owns 16-row tiles of the result.  The four blocks of v_mfma_f64_4x4x4 take 16
+// rows of L as one fragment -- lane l holds L(row l & 15, k = l >> 4) -- and four columns of x,
+// the same for all blocks; its four products are four FMAs in the order k = 0, 1, 2, 3, so a
+// column's result does not depend on W or on its neighbours.  One fragment of L serves all W
+// columns; on the VALU every product took an LDS read of x.
+// Why not v_mfma_f64_16x16x4 and 16 columns: a sweep is bound by its chain of diagonal blocks, and a
+// step of the chain takes as long as the products of one workgroup.  Helmholtz 40^3, both sweeps:
+// 8 right-hand sides 2.0 ms on the VALU, 1.37 on the wide instruction, 0.66 in groups of 4.
+// Element e of lane l is row tile_row(l) of the tile, column tile_col(l) + e: a lane's columns are
+// adjacent and come with one read.
+// ---------------------------------------------------------------------------
+template <int W>
+struct Tile {
+    double e[W / 4];
+};
+template <int W>
+__device__ __forceinline__ Tile<W> tile_zero() {
+    Tile<W> t;
+#pragma unroll
+    for (int e = 0; e < W / 4; ++e) t.e[e] = 0.0;
+    return t;
+}
+template <int W>
+__device__ __forceinline__ int tile_col(int lane) { return W / 4 * (lane & 3); }
+__device__ __forceinline__ int tile_row(int lane) { return 4 * ((lane >> 2) & 3) + (lane >> 4); }
+template <int W>
+__device__ __forceinline__ Tile<W> operator+(const Tile<W> &a, const Tile<W> &b) {
+    Tile<W> t;
+#pragma unroll
+    for (int e = 0; e < W / 4; ++e) t.e[e] = a.e[e] + b.e[e];
+    return t;
+}
+template <int W>
+__device__ __forceinline__ Tile<W> operator-(const Tile<W> &a, const Tile<W> &b) {
+    Tile<W> t;
+#pragma unroll
+    for (int e = 0; e < W / 4; ++e) t.e[e] = a.e[e] - b.e[e];
+    return t;
+}
+// x: the lane's first entry of the fragment's row
+template <int W>
+__device__ __forceinline__ void mma(double a, const double *x, Tile<W> &c) {
+#pragma unroll
+    for (int e = 0; e < W / 4; ++e) c.e[e] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, x[e], c.e[e], 0, 0, 0);
+}
+// a tile to and from W-wide rows
+template <int W>
+__device__ __forceinline__ void tile_store(double *rows, const Tile<W> &t) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int e = 0; e < W / 4; ++e) rows[tile_row(lane) * W + tile_col<W>(lane) + e] = t.e[e];
+}
+template <int W>
+__device__ __forceinline__ Tile<W> tile_load(const double *rows) {
+    const int lane = threadIdx.x & 63;
+    Tile<W> t;
+#pragma unroll
+    for (int e = 0; e < W / 4; ++e) t.e[e] = rows[tile_row(lane) * W + tile_col<W>(lane) + e];
+    return t;
+}
+
+// Loads of L go through buffer resources based at a block of columns and ending after its last
+// valid column: columns past the end and masked lanes (offset OUT) read zero, without a branch.
+constexpr unsigned OUT = 0x7FFFFFF8u;  // (column offsets added to it stay past every range)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t cols_rsrc(const gdouble *L, size_t lda, size_t c0, int ncols) {
+    const size_t bytes = (size_t)ncols * lda * sizeof(double);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>((const double *)(L + c0 * lda)), (short)0,
+                                             (int)(bytes < 0x7FFFFFF0 ? bytes : 0x7FFFFFF0), 0x00020000);
+}
+__device__ __forceinline__ double buf_ld(__amdgpu_buffer_rsrc_t r, unsigned off) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0));
+}
+
+// Row order of x for the transposed products (see TCols)
+__device__ __forceinline__ int tcol_pos(int row) { return (row & ~7) | ((row & 1) << 2) | ((row >> 1) & 3); }
+
+// A block's n rows of x (row stride nq) on their way to LDS.  ask loads the words without waiting
+// for them (AHEAD: while the block before is used, so that a block published long ago costs a reader
+// behind the chain no trip of its own); take polls until all are set and stores them to xb (row stride W, zeros for rows and columns that
+// do not exist; TCOL: rows in the order of tcol_pos), ending with the barrier.  near: the block is
+// one of the reader's last NEAR steps of the chain and is polled by every thread; otherwise a
+// wavefront waits for one word of it first, a trip more.
+constexpr int NEAR = 3;
+template <int W, bool TCOL = false>
+struct XBlock {
+    static constexpr int NI = SB * W / 256;
+    static constexpr bool AHEAD = W == 4;  // (wider, the registers are short)
+    const double *src;
+    int n, nq;
+    unsigned long long v[NI];
+    __device__ __forceinline__ void ask(const double *src_, int n_, int nq_) {
+        src = src_, n = n_, nq = nq_;
+        reload();
+    }
+    __device__ __forceinline__ void reload() {
+        const int tid = threadIdx.x;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int e = tid + 256 * i, row = e / W, q = e % W;
+            v[i] = (row < n && q < nq) ? ld_bits(src + (size_t)row * nq + q) : 0ull;
+        }
+    }
+    __device__ __forceinline__ void take(bool near, double *xb, int *err) {
+        const int tid = threadIdx.x;
+        int spins = 0;
+        auto pause = [&]() {  // false: give up
+            if ((++spins & 63) == 0 &&
+                (spins > SPIN_LIMIT || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+                atomicOr(err, 1);
+                return false;
+            }
+            __builtin_amdgcn_s_sleep(1);
+            return true;
+        };
+        for (;;) {
+            bool bad = false;
+#pragma unroll
+            for (int i = 0; i < NI; ++i) bad |= v[i] == UNSET;
+            if (!__any(bad)) break;
+            if (!near) {
+                const double *last = src + (size_t)n * nq - 1;
+                while (ld_bits(last) == UNSET)
+                    if (!pause()) break;
+            }
+            if (!pause()) break;
+            reload();
+        }
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int e = tid + 256 * i;
+            xb[TCOL ? tcol_pos(e / W) * W + e % W : e] = __longlong_as_double((long long)v[i]);
+        }
+        __syncthreads();
+    }
 };
 
-__device__ __forceinline__ void load_diag_block(const DiagLds &d, const gdouble *L, size_t lda, int jb, int n1,
-                                                int n2) {
-    const int l = threadIdx.x & 63, q = threadIdx.x >> 6;
-    double a[16], b[16], c[16];
+// Rows of a front times a chunk of 32 columns: two sums of 16 products, added and subtracted from
+// acc (columns ascending).  a[t][s]: fragment of tile t, columns 4s .. 4s + 3; xb: the chunk's x.
+template <int W>
+__device__ __forceinline__ void fwd_chunk(const double (&a)[2][8], const double *xb, Tile<W> (&acc)[2]) {
+    const int lane = threadIdx.x & 63, b0 = (lane >> 4) * W + tile_col<W>(lane);
+    Tile<W> p[2][2];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-        const int i = q + 4 * u;  // X row, C column
-        a[u] = (i < n1 && l < i) ? L[(jb + l) + (size_t)(jb + i) * lda] : 0.0;
-        b[u] = (i < n2 && l < i) ? L[(jb + 64 + l) + (size_t)(jb + 64 + i) * lda] : 0.0;
-        c[u] = (l < n2) ? L[(jb + 64 + l) + (size_t)(jb + i) * lda] : 0.0;
+    for (int t = 0; t < 2; ++t) p[t][0] = p[t][1] = tile_zero<W>();
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        const double *x0 = xb + 4 * s * W + b0, *x1 = x0 + 16 * W;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            mma<W>(a[t][s], x0, p[t][0]);
+            mma<W>(a[t][4 + s], x1, p[t][1]);
+        }
     }
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-        const int i = q + 4 * u;
-        if (l < i) {
-            d.tA[i * (i - 1) / 2 + l] = a[u];
-            d.tB[i * (i - 1) / 2 + l] = b[u];
+    for (int t = 0; t < 2; ++t) acc[t] = acc[t] - (p[t][0] + p[t][1]);
+}
+
+// acc -= L[r0 : r0 + nr, 0 : ncols] x, wavefront w forming rows 32w .. 32w + 31.  WAIT: x comes
+// block by block from src as it is published; else (ncols <= SB) the caller has filled xs.  A whole
+// block of L is in flight ahead of the products: when a block's x arrives, which ends a step of the
+// chain, only products remain.  (With one chunk in flight a workgroup took 6 us a block and fell
+// behind the chain, whose step is 3 to 5 us.)
+template <int W, bool WAIT>
+__device__ __forceinline__ void fwd_rows(const gdouble *L, size_t lda, int r0, int nr, int ncols, const double *src,
+                                         int nq, Tile<W> (&acc)[2], double *xs, int *err) {
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool act = 32 * wv < nr;  // (the wavefront has rows)
+    const int nblk = (ncols + SB - 1) / SB;
+    const unsigned col = 8u * (unsigned)lda;
+    unsigned off[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int row = 32 * wv + 16 * t + (lane & 15);
+        off[t] = row < nr ? 8u * (unsigned)(r0 + row) + (unsigned)(lane >> 4) * col : OUT;
+    }
+    auto load = [&](int blk, int ch, double (&v)[2][8]) {
+        const __amdgpu_buffer_rsrc_t r = cols_rsrc(L, lda, (size_t)blk * SB, min(SB, ncols - blk * SB));
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int s = 0; s < 8; ++s) v[t][s] = buf_ld(r, off[t] + (unsigned)(32 * ch + 4 * s) * col);
+    };
+    // chunk ch of the current block in a[ch]; once used, its registers take the next block's
+    double a[4][2][8];
+    if (act) {
+#pragma unroll
+        for (int ch = 0; ch < 4; ++ch)
+            if (32 * ch < ncols) load(0, ch, a[ch]);
+    }
+    XBlock<W> X;
+    if (WAIT && X.AHEAD) X.ask(src, min(SB, ncols), nq);
+    for (int blk = 0; blk < nblk; ++blk) {
+        const int n = min(SB, ncols - blk * SB), next = ncols - (blk + 1) * SB;
+        double *xb = xs + (blk & 1) * (SB * W);
+        if (WAIT && !X.AHEAD) X.ask(src + (size_t)blk * SB * nq, n, nq);
+        if (WAIT) X.take(blk + NEAR >= nblk, xb, err);
+        if (WAIT && X.AHEAD && next > 0) X.ask(src + (size_t)(blk + 1) * SB * nq, min(SB, next), nq);
+        if (!act) continue;
+#pragma unroll
+        for (int ch = 0; ch < 4; ++ch) {
+            if (32 * ch < n) fwd_chunk<W>(a[ch], xb + 32 * ch * W, acc);
+            if (32 * ch < next) load(blk + 1, ch, a[ch]);
         }
-        d.C[l][i] = c[u];
     }
 }
 
-// x = X w for a 64 x 64 unit lower triangle's inverse X (compact): wavefront w takes right-hand
-// sides w, w + 4, ...; lane i forms x_i = w_i + sum_{j<i} X(i, j) w_j with its row of X in
-// registers and w_j by readlane, the sum in four interleaved partial sums combined in a fixed
-// order.  ws[q * SB + off + i] holds w on entry and x on return; rows >= nn take no part.
-// part (may be null): four column-quarter sums per right-hand side, part[(4q + k) * 64 + i], taken
-// off w first as ((p0 + p1) + p2) + p3 (the update by the tile before the triangle, folded into
-// the read so that it needs no barrier of its own).
-__device__ __forceinline__ void tri_fwd(const double *X, double *ws, int off, int nn, int nq,
-                                        const double *part = nullptr) {
-    const int lane = threadIdx.x & 63;
-    if ((threadIdx.x >> 6) >= nq) return;
-    const int rb = lane * (lane - 1) / 2;
-    double row[64];
+// The diagonal block [jb, jb + nb): fragments of the inverses of its two unit triangles (kept by
+// k_diag_inverse in the block's upper triangle) in LDS, each read only by the wavefront that
+// stored it, and of the tile C = L[jb + 64 : jb + 128, jb : jb + 64] between them in registers.
+// Wavefront w forms rows 16w .. 16w + 15 of both halves; a product with a triangle is four sums,
+// over the columns 16r .. 16r + 15 (r = 0 .. 3), of which those on the other side of the diagonal
+// are empty and not stored: 40 fragments a triangle.  C_EARLY: C is loaded with the triangles;
+// otherwise, where its registers are needed until then, after the block's other products
+// (load_c), and its lines only touched here.
+constexpr int TFRAG = 40 * 64;
+template <bool FWD, bool C_EARLY>
+struct Diag {
+    double c[16];
+    double *tri;  // the wavefront's fragments of triangle A; B's TFRAG later
+    int n1, n2;
+    static __device__ __forceinline__ bool has(int r, int w) { return FWD ? r <= w : r >= w; }
+    __device__ __forceinline__ void load(const gdouble *L, size_t lda, int jb, int nb, double *frags) {
+        const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const int i = 16 * w + (lane & 15), k = lane >> 4;
+        n1 = min(64, nb), n2 = nb - n1;
+        tri = frags + (FWD ? 2 * w * (w + 1) : 16 * w - 2 * w * (w - 1)) * 64 + lane;
+        const __amdgpu_buffer_rsrc_t ra = cols_rsrc(L, lda, jb, nb);
+        const unsigned col = 8u * (unsigned)lda;
+        auto half = [&](int h, int n, double (&v)[16]) {
 #pragma unroll
-    for (int j = 0; j < 63; ++j) row[j] = (j < lane) ? X[rb + j] : 0.0;
-    row[63] = 0.0;
-    for (int q = threadIdx.x >> 6; q < nq; q += 4) {
-        double wi = (lane < nn) ? ws[q * SB + off + lane] : 0.0;
-        if (part && lane < nn)
-            wi -= ((part[(q * 4) * 64 + lane] + part[(q * 4 + 1) * 64 + lane]) + part[(q * 4 + 2) * 64 + lane]) +
-                  part[(q * 4 + 3) * 64 + lane];
-        double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+            for (int r = 0; r < 4; ++r)
+                if (has(r, w)) {
 #pragma unroll
-        for (int j = 0; j < 64; j += 4) {
-            a0 += row[j] * readlane_f64(wi, j);
-            a1 += row[j + 1] * readlane_f64(wi, j + 1);
-            a2 += row[j + 2] * readlane_f64(wi, j + 2);
-            a3 += row[j + 3] * readlane_f64(wi, j + 3);
+                    for (int s = 0; s < 4; ++s) {
+                        const int j = 16 * r + 4 * s + k;
+                        const int x = FWD ? i : j, y = FWD ? j : i;  // inverse entry (x, y), kept at (y, x)
+                        v[4 * r + s] = buf_ld(ra, y < x && x < n ? 8u * (unsigned)(jb + h + y) + (unsigned)(h + x) * col : OUT);
+                    }
+                }
+        };
+        double a[16], b[16], touch = 0.0;
+        half(0, n1, a);
+        if (n2 > 0) {
+            half(64, n2, b);
+            if (C_EARLY) load_c(L, lda, jb);
+            else touch = buf_ld(ra, 16 * k < n2 ? 8u * (unsigned)(jb + 64 + 16 * k) + (unsigned)i * col : OUT);
         }
-        if (lane < nn) ws[q * SB + off + lane] = wi + ((a0 + a1) + (a2 + a3));
+        double *t = tri;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (has(r, w)) {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    t[0] = a[4 * r + s];
+                    if (n2 > 0) t[TFRAG] = b[4 * r + s];
+                    t += 64;
+                }
+            }
+        if (!C_EARLY) asm volatile("" ::"v"(touch));
     }
-}
-
-// x = X^T w: lane i forms x_i = w_i + sum_{j>i} X(j, i) w_j with column i of X in registers;
-// part (may be null): part[q * 64 + i] is taken off w first.
-__device__ __forceinline__ void tri_bwd(const double *X, double *ws, int off, int nn, int nq,
-                                        const double *part = nullptr) {
-    const int lane = threadIdx.x & 63;
-    if ((threadIdx.x >> 6) >= nq) return;
-    double col[64];
-    col[0] = 0.0;
+    __device__ __forceinline__ void load_c(const gdouble *L, size_t lda, int jb) {
+        const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const int i = 16 * w + (lane & 15), k = lane >> 4;
+        const __amdgpu_buffer_rsrc_t ra = cols_rsrc(L, lda, jb, min(SB, n1 + n2));
 #pragma unroll
-    for (int j = 1; j < 64; ++j) col[j] = (j > lane) ? X[j * (j - 1) / 2 + lane] : 0.0;
-    for (int q = threadIdx.x >> 6; q < nq; q += 4) {
-        double wi = (lane < nn) ? ws[q * SB + off + lane] : 0.0;
-        if (part && lane < nn) wi -= part[q * 64 + lane];
-        double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-#pragma unroll
-        for (int j = 0; j < 64; j += 4) {
-            a0 += col[j] * readlane_f64(wi, j);
-            a1 += col[j + 1] * readlane_f64(wi, j + 1);
-            a2 += col[j + 2] * readlane_f64(wi, j + 2);
-            a3 += col[j + 3] * readlane_f64(wi, j + 3);
+        for (int s = 0; s < 16; ++s) {
+            const int x = FWD ? i : 4 * s + k, y = FWD ? 4 * s + k : i;  // C(x, y)
+            c[s] = buf_ld(ra, x < n2 ? 8u * (unsigned)(jb + 64 + x) + 8u * (unsigned)y * (unsigned)lda : OUT);
         }
-        if (lane < nn) ws[q * SB + off + lane] = wi + ((a0 + a1) + (a2 + a3));
     }
-}
-
-// Forward substitution of one diagonal block for nq right-hand sides (all threads of the
-// workgroup): ws[q * SB + i] holds the block's w on entry and its x on return.
-template <int NR>
-__device__ __forceinline__ void fwd_block(const DiagLds &d, double *ws, double *part, int n1, int n2, int nq) {
-    const int tid = threadIdx.x, i = tid & 63, jq = tid >> 6;
-    tri_fwd(d.tA, ws, 0, n1, nq);
-    __syncthreads();
-    if (n2 > 0) {
-        // C x_A: column quarters combined in a fixed order
+    // sum_j X(i, j) w_j (j != i) of half h, w in LDS (row stride W)
+    template <int W>
+    __device__ __forceinline__ Tile<W> tri_sum(int h, const double *ws) const {
+        const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const double *t = tri + h * TFRAG;
+        const double *x = ws + (64 * h + (lane >> 4)) * W + tile_col<W>(lane);
+        Tile<W> a[4];
 #pragma unroll
-        for (int q = 0; q < NR; ++q) {
-            if (q < nq) {
-                double s = 0.0;
+        for (int r = 0; r < 4; ++r) {
+            a[r] = tile_zero<W>();
+            if (has(r, w)) {
 #pragma unroll
-                for (int u = 0; u < 16; ++u) s += d.C[i][jq + 4 * u] * ws[q * SB + jq + 4 * u];
-                part[(q * 4 + jq) * 64 + i] = s;
+                for (int s = 0; s < 4; ++s) mma<W>(t[64 * s], x + (16 * r + 4 * s) * W, a[r]);
+                t += 256;
             }
         }
-        __syncthreads();
-        tri_fwd(d.tB, ws, 64, n2, nq, part);  // w_B - C x_A, then the triangle
-        __syncthreads();
+        return (a[0] + a[1]) + (a[2] + a[3]);
+    }
+};
+
+// Sum of leaf(r0) .. leaf(r0 + N - 1) as a binary tree
+template <int N, class T, class F>
+__device__ __forceinline__ T tree_sum(int r0, F &&leaf) {
+    if constexpr (N == 1) {
+        return leaf(r0);
+    } else {
+        const T x = tree_sum<N / 2, T>(r0, leaf);
+        const T y = tree_sum<N / 2, T>(r0 + N / 2, leaf);
+        return x + y;
     }
 }
-
-// Cross-lane moves for the butterflies, all on the VALU (no LDS round trip): the 32- and 16-lane
-// exchanges by v_permlane32_swap / v_permlane16_swap, the 8-lane one by a DPP rotation within rows
-// of 16, the 2- and 1-lane ones by DPP quad permutations.
-template <bool D32>
-__device__ __forceinline__ void perm_swap(double &a, double &b) {
-    const unsigned long long x = (unsigned long long)__double_as_longlong(a);
-    const unsigned long long y = (unsigned long long)__double_as_longlong(b);
-    const unsigned xl = (unsigned)x, xh = (unsigned)(x >> 32), yl = (unsigned)y, yh = (unsigned)(y >> 32);
-    auto lo = D32 ? __builtin_amdgcn_permlane32_swap(xl, yl, false, false) : __builtin_amdgcn_permlane16_swap(xl, yl, false, false);
-    auto hi = D32 ? __builtin_amdgcn_permlane32_swap(xh, yh, false, false) : __builtin_amdgcn_permlane16_swap(xh, yh, false, false);
-    a = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
-    b = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+template <int W>
+struct Tile2 {
+    Tile<W> t[2];
+};
+template <int W>
+__device__ __forceinline__ Tile2<W> operator+(const Tile2<W> &a, const Tile2<W> &b) {
+    return Tile2<W>{{a.t[0] + b.t[0], a.t[1] + b.t[1]}};
 }
 
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xF, 0xF, true);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, true);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
-// Column sums over the 64 lanes of a wavefront for 8 columns at once, a fixed order: a
-// reduce-scatter butterfly over lane bits 5, 4, 3 (8 -> 1 values per lane), then sums over lane
-// bits 2, 1, 0; at every stage the lower lane of a pair contributes first.  p[c] is the lane's
-// partial of column c; on return every lane holds the sum of column ((lane >> 3) & 7) in p[0].
-__device__ __forceinline__ void wave_colsum8(double (&p)[8]) {
-    const int lane = threadIdx.x & 63;
-    // bit 5: after the swap a holds (own, partner's) p[i] on lower lanes and (partner's, own)
-    // p[i + 4] on upper lanes, paired with b: a + b is (keep + received) resp. (received + keep)
+// Transposed products: rows r0 .. r0 + nr - 1 (nr <= 128, r0 > 0) times columns c0 .. c0 + ncols - 1
+// (at most 128; wavefront w forms columns 32w .. 32w + 31), x of the rows in xs.  A 16-byte load
+// takes 64 bytes of each of 16 columns: rows 8s + 2k and 8s + 2k + 1 in lane group k, so the four
+// even and the four odd rows of eight are a fragment each, and xs holds its rows in that order
+// (tcol_pos).  Every fragment's sum is a leaf; the 32 leaves are added as a binary tree.
+template <int W>
+struct TCols {
+    unsigned off[2];
+    int nr, row0;
+    __amdgpu_buffer_rsrc_t rs;
+    double a[4][8][2];  // leaves 8g .. 8g + 7 in a[g]
+    __device__ __forceinline__ void at(const gdouble *L, size_t lda, int r0, int nr_, int c0, int ncols) {
+        const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        rs = cols_rsrc(L, lda, c0, ncols);
+        nr = nr_;
+        row0 = 2 * (lane >> 4);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        double a = p[i], b = p[i + 4];
-        perm_swap<true>(a, b);
-        p[i] = a + b;
+        for (int t = 0; t < 2; ++t)
+            off[t] = 8u * (unsigned)(r0 + row0) + (unsigned)(32 * wv + 16 * t + (lane & 15)) * 8u * (unsigned)lda;
     }
+    __device__ __forceinline__ void load(int g) {
+        typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+        typedef double f64x2 __attribute__((ext_vector_type(2)));
+        auto pair = [&](unsigned o) { return __builtin_bit_cast(f64x2, __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)o, 0, 0))); };
+        if (32 * g + 32 <= nr) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        double a = p[i], b = p[i + 2];
-        perm_swap<false>(a, b);
-        p[i] = a + b;
-    }
-    {
-        const bool hi = (lane & 8) != 0;
-        const double keep = hi ? p[1] : p[0];
-        const double send = hi ? p[0] : p[1];
-        const double recv = dpp_f64<0x128>(send);  // row_ror:8 = lane ^ 8 within rows of 16
-        p[0] = hi ? recv + keep : keep + recv;
-    }
-    {
-        const double other = __shfl_xor(p[0], 4);
-        p[0] = (lane & 4) ? other + p[0] : p[0] + other;
-    }
-    {
-        const double other = dpp_f64<0x4E>(p[0]);  // quad_perm [2,3,0,1]
-        p[0] = (lane & 2) ? other + p[0] : p[0] + other;
-    }
-    {
-        const double other = dpp_f64<0xB1>(p[0]);  // quad_perm [1,0,3,2]
-        p[0] = (lane & 1) ? other + p[0] : p[0] + other;
-    }
-}
-
-// Backward substitution of one diagonal block with L11^T (all threads): ws holds the block's
-// right-hand side, from which every later block and L21 have been removed, and its x on return.
-// C^T x_B: wavefront jq sums its sixteen columns jq + 4u over the 64 rows with the butterfly.
-template <int NR>
-__device__ __forceinline__ void bwd_block(const DiagLds &d, double *ws, double *part, int n1, int n2, int nq) {
-    const int tid = threadIdx.x, i = tid & 63, jq = tid >> 6;
-    if (n2 > 0) {
-        tri_bwd(d.tB, ws, 64, n2, nq);
-        __syncthreads();
+            for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int q = 0; q < NR; ++q) {
-            if (q < nq) {
-                const double xb = (i < n2) ? ws[q * SB + 64 + i] : 0.0;
+                for (int t = 0; t < 2; ++t) {
+                    const f64x2 v = pair(off[t] + 8u * (unsigned)(32 * g + 8 * s));
+                    a[g][2 * s][t] = v[0];
+                    a[g][2 * s + 1][t] = v[1];
+                }
+        } else {
+            // a last odd row comes as the second of the pair before it
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    double p[8];
+            for (int s = 0; s < 4; ++s) {
+                const int row = 32 * g + 8 * s + row0;
+                const bool in0 = row < nr, in1 = row + 1 < nr;
 #pragma unroll
-                    for (int u = 0; u < 8; ++u) p[u] = d.C[i][jq + 4 * (8 * h + u)] * xb;
-                    wave_colsum8(p);
-                    if ((i & 7) == 0) part[q * 64 + jq + 4 * (8 * h + ((i >> 3) & 7))] = p[0];
+                for (int t = 0; t < 2; ++t) {
+                    const f64x2 v = pair(in0 ? off[t] + 8u * (unsigned)(32 * g + 8 * s) - (in1 ? 0u : 8u) : OUT);
+                    a[g][2 * s][t] = in1 ? v[0] : v[1];
+                    a[g][2 * s + 1][t] = in1 ? v[1] : 0.0;
                 }
             }
         }
-        __syncthreads();
     }
-    tri_bwd(d.tA, ws, 0, n1, nq, n2 > 0 ? part : nullptr);  // w_A - C^T x_B, then the triangle
-    __syncthreads();
-}
-
-// Pull of the descendants' updates into column i of a front: x[t] - sum of the Y entries of
-// global index t = sidx[i], in list order (postorder of the fronts that produced them).
-__device__ __forceinline__ double pull_column(int t, const int *__restrict__ ptr, const long long *__restrict__ ent,
-                                              const double *__restrict__ Yq, const double *__restrict__ xq) {
-    const int e1 = ptr[t + 1];
-    int e = ptr[t];
-    double acc = 0.0;
-    for (; e + 4 <= e1; e += 4) {
-        const long long a0 = ent[e], a1 = ent[e + 1], a2 = ent[e + 2], a3 = ent[e + 3];
-        const double y0 = ld_co(Yq + a0), y1 = ld_co(Yq + a1), y2 = ld_co(Yq + a2), y3 = ld_co(Yq + a3);
-        acc = (((acc + y0) + y1) + y2) + y3;
+    __device__ __forceinline__ void load_all() {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            if (32 * g < nr) load(g);
     }
-    for (; e < e1; ++e) acc += ld_co(Yq + ent[e]);
-    return xq[t] - acc;
-}
-
-// Row products of the forward sweep: acc[q] (thread tid < 128, row r0 + tid) -= L[r0 + tid, 0:ncols] x,
-// the columns streamed in chunks of CW (thread (row ri, half ch) holds 16 columns of a chunk,
-// the next chunk's loads in flight during the current products), each 128-column block's x
-// read from W once its flag is set -- or, with flags == nullptr (ncols <= SB), taken from xs as
-// the caller filled it (zeros beyond ncols).  Per chunk the two halves' sums are subtracted in
-// order, the same arithmetic either way.
-template <int NR>
-__device__ __forceinline__ void fwd_chunk(const double (&v)[16], int k, int nq, double (&acc)[NR], const double *xs,
-                                          double *ps) {
-    const int tid = threadIdx.x, ri = tid & 127, ch = tid >> 7;
-    const int xo = (k * CW) % SB + 16 * ch;
-    double *pk = ps + (k & 1) * (NR * 256);
-#pragma unroll
-    for (int q = 0; q < NR; ++q) {
-        if (q < nq) {
-            double s = 0.0;
-#pragma unroll
-            for (int u = 0; u < 16; ++u) s += v[u] * xs[q * SB + xo + u];
-            pk[q * 256 + ch * 128 + ri] = s;
-        }
+    __device__ __forceinline__ Tile<W> sum(int g, int t, const double *xs) const {
+        const int lane = threadIdx.x & 63;
+        const double *x = xs + (lane >> 4) * W + tile_col<W>(lane);
+        return tree_sum<8, Tile<W>>(0, [&](int r) {
+            Tile<W> p = tile_zero<W>();
+            mma<W>(a[g][r][t], x + 4 * (8 * g + r) * W, p);
+            return p;
+        });
     }
-    __syncthreads();
-    if (tid < 128) {
+    // the sum over the rows; with a next tile (rows nr1 > 0 from r1, same columns), each group's
+    // registers take its leaves once they are used
+    __device__ __forceinline__ Tile2<W> step(const double *xs, int dr, int nr1) {
+        Tile2<W> s[4];
+        const int n = nr;
 #pragma unroll
-        for (int q = 0; q < NR; ++q)
-            if (q < nq) acc[q] -= pk[q * 256 + tid] + pk[q * 256 + 128 + tid];
-    }
-}
-
-// The four chunks of one block at once (the last block, whose loads were all issued before its
-// flag): the four partial sums per thread into four slices of ps, one barrier, then the chunks'
-// sums subtracted in chunk order -- the arithmetic of four fwd_chunk calls.
-template <int NR>
-__device__ __forceinline__ void fwd_chunk4(const double (&v0)[16], const double (&v1)[16], const double (&v2)[16],
-                                           const double (&v3)[16], int k, int nq, double (&acc)[NR],
-                                           const double *xs, double *ps) {
-    const int tid = threadIdx.x, ri = tid & 127, ch = tid >> 7;
-    auto part = [&](const double (&v)[16], int kk, int slot) {
-        const int xo = (kk * CW) % SB + 16 * ch;
-        double *pk = ps + slot * (NR * 256);
+        for (int t = 0; t < 2; ++t) off[t] += 8u * (unsigned)dr;
+        nr = nr1;
 #pragma unroll
-        for (int q = 0; q < NR; ++q) {
-            if (q < nq) {
-                double s = 0.0;
+        for (int g = 0; g < 4; ++g) {
 #pragma unroll
-                for (int u = 0; u < 16; ++u) s += v[u] * xs[q * SB + xo + u];
-                pk[q * 256 + ch * 128 + ri] = s;
+            for (int t = 0; t < 2; ++t) {
+                s[g].t[t] = tile_zero<W>();
+                if (32 * g < n) s[g].t[t] = sum(g, t, xs);
+                __builtin_amdgcn_sched_barrier(0);
             }
+            if (32 * g < nr1) load(g);
+            if (g & 1) s[g - 1] = s[g - 1] + s[g];
         }
-    };
-    part(v0, k, 0);
-    part(v1, k + 1, 1);
-    part(v2, k + 2, 2);
-    part(v3, k + 3, 3);
-    __syncthreads();
-    if (tid < 128) {
-#pragma unroll
-        for (int slot = 0; slot < 4; ++slot) {
-            const double *pk = ps + slot * (NR * 256);
-#pragma unroll
-            for (int q = 0; q < NR; ++q)
-                if (q < nq) acc[q] -= pk[q * 256 + tid] + pk[q * 256 + 128 + tid];
-        }
+        return s[0] + s[2];
     }
-}
+};
 
-template <int NR, bool FLAGS>
-__device__ __forceinline__ void fwd_rows_product(const gdouble *L, size_t lda, int r0, int nr, int ncols,
-                                                 const int *flags, int *err, const double *Wf, long long wtotal,
-                                                 int nq, double (&acc)[NR], double *xs, double *ps) {
-    const int tid = threadIdx.x, ri = tid & 127, ch = tid >> 7;
-    const bool rin = ri < nr;
-    const int nchunk = (ncols + CW - 1) / CW;
-    const gdouble *Lr = L + (r0 + ri);
-    auto load = [&](int k, double (&v)[16]) {
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const int col = k * CW + 16 * ch + u;
-            v[u] = (rin && col < ncols) ? Lr[(size_t)col * lda] : 0.0;
-        }
-    };
-    auto take_block = [&](int blk) {  // wait for block blk's x and stage it in xs
-        __syncthreads();  // the previous block's x is no longer read
-        if (tid == 0) wait_at_least(flags + blk, 1, err);
-        __syncthreads();
-        for (int e = tid; e < nq * SB; e += 256) {
-            const int q = e / SB, j = e % SB, col = blk * SB + j;
-            xs[e] = (col < ncols) ? ld_co(Wf + q * wtotal + col) : 0.0;
-        }
-        __syncthreads();
-    };
-    // the last block's chunks are all loaded before its flag is awaited: that wait ends the chain
-    // step of the block before, and only the products remain after it
-    const int klast = FLAGS ? ((ncols + SB - 1) / SB - 1) * (SB / CW) : nchunk;
-    double cur[16], nxt[16];
-    if (nchunk > 0) load(0, cur);
-    for (int k = 0; k < nchunk; ++k) {
-        if (FLAGS && k == klast) {
-            static_assert(SB / CW == 4, "four chunks per block");
-            double c1[16], c2[16], c3[16];
-            load(k + 1, c1);
-            load(k + 2, c2);
-            load(k + 3, c3);
-            take_block(k / (SB / CW));
-            fwd_chunk4<NR>(cur, c1, c2, c3, k, nq, acc, xs, ps);
-            break;
-        }
-        if (FLAGS && (k * CW) % SB == 0) take_block(k / (SB / CW));
-        if (k + 1 < nchunk) load(k + 1, nxt);
-        fwd_chunk<NR>(cur, k, nq, acc, xs, ps);
-#pragma unroll
-        for (int u = 0; u < 16; ++u) cur[u] = nxt[u];
-    }
-}
-
-// Transposed products for up to 128 columns [c0, c0 + ncols): out[q * SB + j] = sum over rows
-// i in [r0, r0 + nr) of L[i, c0 + j] * x(q, i).  Wavefront w takes columns 32w .. 32w + 31 in
-// four batches of 8; lanes take rows r0 + lane + 64u (u < RPL), xv[q][u] being the lane's x of
-// that row.  Every load of L serves all nq right-hand sides.
-template <int NR, int RPL>
-__device__ __forceinline__ void tcol_product(const gdouble *L, size_t lda, int r0, int nr, int c0, int ncols,
-                                             const double (&xv)[NR][RPL], int nq, double *out) {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll 1
-    for (int cb = 32 * wv; cb < 32 * wv + 32; cb += 8) {
-        if (cb >= ncols) break;
-        double lv[RPL][8];
-#pragma unroll
-        for (int u = 0; u < RPL; ++u) {
-            const int i = lane + 64 * u;
-#pragma unroll
-            for (int c = 0; c < 8; ++c)
-                lv[u][c] = (i < nr && cb + c < ncols) ? L[(size_t)(r0 + i) + (size_t)(c0 + cb + c) * lda] : 0.0;
-        }
-#pragma unroll
-        for (int q = 0; q < NR; ++q) {
-            if (q < nq) {
-                double p[8];
-#pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    double s = 0.0;
-#pragma unroll
-                    for (int u = 0; u < RPL; ++u) s += lv[u][c] * xv[q][u];
-                    p[c] = s;
-                }
-                wave_colsum8(p);
-                const int col = cb + ((lane >> 3) & 7);
-                if ((lane & 7) == 0 && col < ncols) out[q * SB + col] = p[0];
-            }
-        }
-    }
-}
-
-// A transposed tile of at most 128 rows [r0, r0 + nr) x 128 columns [c0, c0 + ncols) wholly in
-// registers (wavefront w: columns 32w .. 32w + 31 in four batches of 8; lanes: rows lane, lane + 64),
-// so it can be loaded before the x it multiplies is available.
-__device__ __forceinline__ void tcol_load2(const gdouble *L, size_t lda, int r0, int nr, int c0, int ncols,
-                                           double (&lv)[4][2][8]) {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int i = lane + 64 * u;
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const int col = 32 * wv + 8 * b + c;
-                lv[b][u][c] = (i < nr && col < ncols) ? L[(size_t)(r0 + i) + (size_t)(c0 + col) * lda] : 0.0;
-            }
-        }
-}
-
-// out[q * SB + j] = sum over the tile's rows of tile(i, j) x(q, i), the arithmetic of tcol_product
-template <int NR>
-__device__ __forceinline__ void tcol_compute2(const double (&lv)[4][2][8], const double (&xv)[NR][2], int nq,
-                                              int ncols, double *out) {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        const int cb = 32 * wv + 8 * b;
-        if (cb >= ncols) break;
-#pragma unroll
-        for (int q = 0; q < NR; ++q) {
-            if (q < nq) {
-                double p[8];
-#pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    double sum = 0.0;
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) sum += lv[b][u][c] * xv[q][u];
-                    p[c] = sum;
-                }
-                wave_colsum8(p);
-                const int col = cb + ((lane >> 3) & 7);
-                if ((lane & 7) == 0 && col < ncols) out[q * SB + col] = p[0];
-            }
-        }
-    }
-}
 
 // ===========================================================================
 // Forward sweep (one launch): ticket order = item order.
 // ===========================================================================
-template <int NR>
+template <int W>
 __global__ __launch_bounds__(256, 2) void k_fwd_sweep(PlanDev P, const int4 *__restrict__ items, int nwork, int ngrp,
-                                                   int nrhs, double *__restrict__ x, long long n,
-                                                   double *__restrict__ W, long long wtotal, double *__restrict__ Y,
-                                                   long long ytotal, SyncDev S) {
+                                                      int nrhs, int wq, const double *__restrict__ x, long long n,
+                                                      double *__restrict__ Wx, long long wtotal,
+                                                      double *__restrict__ Y, long long ytotal, SyncDev S) {
+    constexpr int NE = W / 4, NP = 2 * NE, NU = 16 / NP;
     const int t = take_ticket(S.tick);
     if (t >= nwork) return;
     const int4 it = items[t / ngrp];
-    const int grp = t % ngrp;
-    const int q0 = grp * NR, nq = min(NR, nrhs - q0);
+    const int grp = t % ngrp, q0 = grp * wq, nq = min(wq, nrhs - q0);
     const int li = it.x;
     const SolveFront &Fr = P.sf[li];
     const int ne = Fr.ne, m = Fr.m;
     const size_t lda = (size_t)m;
     const gdouble *L = gbl(Fr.F);
-    const int tid = threadIdx.x;
-    const int *flags = S.fflag + (size_t)grp * P.nflag + Fr.fbase;
-    const double *Wf = W + (size_t)q0 * wtotal + Fr.wbase;
-    __shared__ double xs[NR * SB];
-    __shared__ double ps[4 * NR * 256];  // chunk partials (two slices in turn, four for a block)
-    __shared__ double tri[2 * TRI];
-    __shared__ double cti[64][65];
-    __shared__ double ws[NR * SB];
-    const DiagLds dl{tri, tri + TRI, cti};
-    double acc[NR];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int trow = tile_row(lane), qc = tile_col<W>(lane);
+    double *Wf = Wx + (size_t)q0 * wtotal + (size_t)Fr.wbase * nq;
+    double *Yg = Y + (size_t)q0 * ytotal;
+    __shared__ __align__(16) double xs[2 * SB * W];
+    __shared__ double frags[2 * TFRAG];
+    Tile<W> acc[2] = {tile_zero<W>(), tile_zero<W>()};
+    auto store_rows = [&](const Tile<W> (&a)[2], int r0, int nr) {  // Y of 128 rows of L21
 #pragma unroll
-    for (int q = 0; q < NR; ++q) acc[q] = 0.0;
-    if (it.y == IT_FDIAG || it.y == IT_FSMALL) {
-        const int c = it.z, j0 = c * SB;
-        const int nb = min(SB, ne - j0), n1 = min(64, nb), n2 = nb - n1;
-        load_diag_block(dl, L, lda, j0, n1, n2);
-        // the descendants' Y vectors are complete once the effective children are
-        if (tid == 0) {
-            for (int e = Fr.ech0; e < Fr.ech1; ++e) {
-                const int2 ch = P.ech[e];
-                wait_at_least(S.fdone + (size_t)grp * P.nfront + ch.x, ch.y, S.err);
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int e = 0; e < NE; ++e) {
+                const int row = 32 * wv + 16 * tt + trow, q = qc + e;
+                if (row < nr && q < nq) st_co(Yg + (size_t)(Fr.ybase + (r0 - ne) + row) * nq + q, -a[tt].e[e]);
             }
-        }
-        __syncthreads();
-        if (tid < nb) {
-            const int tg = gbl(Fr.sidx)[j0 + tid];
-            if ((unsigned)tg < (unsigned)n) {
-#pragma unroll
-                for (int q = 0; q < NR; ++q)
-                    if (q < nq)
-                        acc[q] = pull_column(tg, P.ptr, P.ent, Y + (size_t)(q0 + q) * ytotal, x + (size_t)(q0 + q) * n);
-            } else {
-                atomicOr(S.err, 2);  // an index outside the system: the solve plan does not fit the fronts
-            }
-        }
-        if (it.y == IT_FDIAG) fwd_rows_product<NR, true>(L, lda, j0, nb, j0, flags, S.err, Wf, wtotal, nq, acc, xs, ps);
-        if (tid < nb) {
-#pragma unroll
-            for (int q = 0; q < NR; ++q) ws[q * SB + tid] = acc[q];
-        }
-        __syncthreads();
-        fwd_block<NR>(dl, ws, ps, n1, n2, nq);
-        if (it.y == IT_FDIAG) {
-            // later blocks and the rows items of this front read x_c
-            if (tid < nb) {
-#pragma unroll
-                for (int q = 0; q < NR; ++q)
-                    if (q < nq) st_co(W + (size_t)(q0 + q) * wtotal + Fr.wbase + j0 + tid, ws[q * SB + tid]);
-            }
-            stores_done_barrier();
-            if (tid == 0) publish_set(S.fflag + (size_t)grp * P.nflag + Fr.fbase + c);
-            return;
-        }
-        // fused front: x stays in LDS for its own rows (W is read by the next launch only)
-        for (int e = tid; e < nq * SB; e += 256) {
-            const int q = e / SB, j = e % SB;
-            const double v = (j < nb) ? ws[e] : 0.0;
-            xs[e] = v;
-            if (j < nb) W[(size_t)(q0 + q) * wtotal + Fr.wbase + j] = v;
-        }
-        __syncthreads();
-        for (int r0 = ne; r0 < m; r0 += SB) {
-            const int nr = min(SB, m - r0);
-            double a2[NR];
-#pragma unroll
-            for (int q = 0; q < NR; ++q) a2[q] = 0.0;
-            fwd_rows_product<NR, false>(L, lda, r0, nr, ne, nullptr, S.err, Wf, wtotal, nq, a2, xs, ps);
-            if (tid < nr) {
-#pragma unroll
-                for (int q = 0; q < NR; ++q)
-                    if (q < nq) st_co(Y + (size_t)(q0 + q) * ytotal + Fr.ybase + (r0 - ne) + tid, -a2[q]);
-            }
-            __syncthreads();  // ps of this row block is read before the next one writes it
-        }
+    };
+    if (it.y == IT_FROWS) {  // 128 rows of L21
+        const int r0 = ne + it.z * SB, nr = min(SB, m - r0);
+        fwd_rows<W, true>(L, lda, r0, nr, ne, Wf, nq, acc, xs, S.err);
+        store_rows(acc, r0, nr);
         stores_done_barrier();
         if (tid == 0) publish_add(S.fdone + (size_t)grp * P.nfront + li);
         return;
     }
-    // IT_FROWS: 128 rows of L21
-    const int r0 = ne + it.z * SB, nr = min(SB, m - r0);
-    fwd_rows_product<NR, true>(L, lda, r0, nr, ne, flags, S.err, Wf, wtotal, nq, acc, xs, ps);
-    if (tid < nr) {
+    const int j0 = it.z * SB, nb = min(SB, ne - j0);
+    // The lists to pull, and what does not depend on the children, ahead of the wait for them
+    int e0[NP], e1[NP];
+    long long ent[NP][NU];
+    double xv[NP];
 #pragma unroll
-        for (int q = 0; q < NR; ++q)
-            if (q < nq) st_co(Y + (size_t)(q0 + q) * ytotal + Fr.ybase + (r0 - ne) + tid, -acc[q]);
+    for (int p = 0; p < NP; ++p) {
+        const int row = 32 * wv + 16 * (p / NE) + trow, q = qc + p % NE;
+        e0[p] = e1[p] = 0;
+        xv[p] = 0.0;
+        if (row < nb && q < nq) {
+            const int tg = gbl(Fr.sidx)[j0 + row];
+            if ((unsigned)tg < (unsigned)n) {
+                e0[p] = P.ptr[tg];
+                e1[p] = P.ptr[tg + 1];
+                xv[p] = x[(size_t)q0 * n + (size_t)tg * nq + q];
+            } else {
+                atomicOr(S.err, 2);  // an index outside the system: the solve plan does not fit the fronts
+            }
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int u = 0; u < NU; ++u) ent[p][u] = e0[p] + u < e1[p] ? P.ent[e0[p] + u] : 0;
+    Diag<true, W == 4> dg;
+    dg.load(L, lda, j0, nb, frags);
+    // the descendants' Y vectors are complete once the effective children are
+    if (wv == 0) {
+        for (int e = Fr.ech0 + lane; e < Fr.ech1; e += 64) {
+            const int2 ch = P.ech[e];
+            wait_at_least(S.fdone + (size_t)grp * P.nfront + ch.x, ch.y, S.err);
+        }
+    }
+    __syncthreads();
+    // pull of the descendants' updates: x[t] - sum of the Y entries of global index t = sidx[i], in
+    // list order (postorder of the fronts that produced them), a lane's rows in step
+    {
+        double sum[NP];
+#pragma unroll
+        for (int p = 0; p < NP; ++p) sum[p] = 0.0;
+        for (;;) {
+            bool more = false;
+            double y[NP][NU];
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+#pragma unroll
+                for (int u = 0; u < NU; ++u) {
+                    y[p][u] = e0[p] + u < e1[p] ? ld_co(Yg + (size_t)ent[p][u] * nq + qc + p % NE) : 0.0;
+                    // the next round's
+                    ent[p][u] = e0[p] + NU + u < e1[p] ? P.ent[e0[p] + NU + u] : 0;
+                }
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+#pragma unroll
+                for (int u = 0; u < NU; ++u)
+                    if (e0[p] + u < e1[p]) sum[p] += y[p][u];
+                e0[p] += NU;
+                more |= e0[p] < e1[p];
+            }
+            if (!__any(more)) break;
+        }
+#pragma unroll
+        for (int p = 0; p < NP; ++p) acc[p / NE].e[p % NE] = xv[p] - sum[p];
+    }
+    if (it.y == IT_FDIAG && j0 > 0) fwd_rows<W, true>(L, lda, j0, nb, j0, Wf, nq, acc, xs, S.err);
+    if (W != 4 && dg.n2 > 0) dg.load_c(L, lda, j0);
+    // The block's w, then its x.  The half of xs that the last block of x did not use is free.
+    const int lastb = max(j0 / SB - 1, 0);
+    double *ws = xs + ((lastb + 1) & 1) * (SB * W), *xo = xs + (lastb & 1) * (SB * W);
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) tile_store<W>(ws + (32 * wv + 16 * tt) * W, acc[tt]);
+    __syncthreads();
+    // later blocks and the rows items of this front read a published x; a fused front's x stays in
+    // LDS for its own rows, and W is read by the next launch
+    auto finish = [&](int h, int nn, const Tile<W> &v) {
+        tile_store<W>(xo + (64 * h + 16 * wv) * W, v);
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+            const int row = 16 * wv + trow, q = qc + e;
+            if (row < nn && q < nq) {
+                double *p = Wf + (size_t)(j0 + 64 * h + row) * nq + q;
+                if (it.y == IT_FDIAG) publish_value(p, v.e[e]);
+                else *p = v.e[e];
+            }
+        }
+    };
+    auto own = [&](int h) { return tile_load<W>(ws + (64 * h + 16 * wv) * W); };
+    finish(0, dg.n1, own(0) + dg.template tri_sum<W>(0, ws));
+    if (dg.n2 > 0) {
+        __syncthreads();
+        Tile<W> p[4];
+        const double *xa = xo + (lane >> 4) * W + qc;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            p[r] = tile_zero<W>();
+#pragma unroll
+            for (int s = 0; s < 4; ++s) mma<W>(dg.c[4 * r + s], xa + (16 * r + 4 * s) * W, p[r]);
+        }
+        const Tile<W> wb = own(1) - (((p[0] + p[1]) + p[2]) + p[3]);
+        tile_store<W>(ws + (64 + 16 * wv) * W, wb);
+        __syncthreads();
+        finish(1, dg.n2, wb + dg.template tri_sum<W>(1, ws));
+    } else if (it.y == IT_FSMALL) {
+        tile_store<W>(xo + (64 + 16 * wv) * W, tile_zero<W>());
+    }
+    if (it.y == IT_FDIAG) return;
+    __syncthreads();
+    for (int r0 = ne; r0 < m; r0 += SB) {
+        const int nr = min(SB, m - r0);
+        acc[0] = acc[1] = tile_zero<W>();
+        fwd_rows<W, false>(L, lda, r0, nr, ne, nullptr, nq, acc, xo, S.err);
+        store_rows(acc, r0, nr);
     }
     stores_done_barrier();
     if (tid == 0) publish_add(S.fdone + (size_t)grp * P.nfront + li);
 }
 
 // z = D^-1 y for column jj of a front (MixedDiagonal::solve_in_place, diagonal.rs:312-365):
-// 1x1 -> y / d (0 for a zero pivot); a 2x2 by Cramer's rule (0 for a singular block).
-__device__ __forceinline__ double dsolve_col(const SolveFront &F, int jj, const double *__restrict__ y) {
+// 1x1 -> y / d (0 for a zero pivot); a 2x2 by Cramer's rule (0 for a singular block).  y has row
+// stride nq.
+__device__ __forceinline__ double dsolve_col(const SolveFront &F, int jj, const double *__restrict__ y, int nq) {
     const int kd = gbl(F.dkind)[jj];
     if (kd == 1) {
         const double d = gbl(F.ddiag)[jj];
-        return (d == 0.0) ? 0.0 : y[jj] / d;
+        return (d == 0.0) ? 0.0 : y[(size_t)jj * nq] / d;
     }
     const int f = (kd == 2) ? jj : jj - 1;  // first column of the 2x2
     const double a = gbl(F.ddiag)[f], b = gbl(F.doff)[f], cc = gbl(F.ddiag)[f + 1];
     const double det = a * cc - b * b;
     if (det == 0.0) return 0.0;
-    const double r1 = y[f], r2 = y[f + 1];
+    const double r1 = y[(size_t)f * nq], r2 = y[(size_t)(f + 1) * nq];
     return (kd == 2) ? (cc * r1 - b * r2) / det : (a * r2 - b * r1) / det;
-}
-
-// x of the L21 rows [ne + rb, ne + rb + nr) of a front, lane rows rb + lane + 64u, for the chunk
-// products of the backward sweep (device-coherent: ancestors write them in the same launch)
-template <int NR>
-__device__ __forceinline__ void gather_rows_x(const SolveFront &Fr, int rb, int nr, const double *__restrict__ x,
-                                              long long n, int q0, int nq, double (&xv)[NR][GH / 64], int *err) {
-    const int lane = threadIdx.x & 63;
-    const gint *ri = gbl(Fr.sidx) + Fr.ne + rb;
-#pragma unroll
-    for (int u = 0; u < GH / 64; ++u) {
-        const int i = lane + 64 * u;
-        int g = (i < nr) ? ri[i] : -1;
-        if (g >= n) {
-            atomicOr(err, 2);  // an index outside the system: the solve plan does not fit the fronts
-            g = -1;
-        }
-#pragma unroll
-        for (int q = 0; q < NR; ++q) xv[q][u] = (g >= 0 && q < nq) ? ld_co(x + (size_t)(q0 + q) * n + g) : 0.0;
-    }
 }
 
 // ===========================================================================
 // Backward sweep (one launch).
 // ===========================================================================
-template <int NR>
+template <int W>
 __global__ __launch_bounds__(256, 2) void k_bwd_sweep(PlanDev P, const int4 *__restrict__ items, int nwork, int ngrp,
-                                                   int nrhs, double *__restrict__ x, long long n,
-                                                   const double *__restrict__ W, double *__restrict__ Xb,
-                                                   long long wtotal, double *__restrict__ Pp, long long ptotal,
-                                                   SyncDev S) {
+                                                      int nrhs, int wq, double *__restrict__ x, long long n,
+                                                      const double *__restrict__ Wx, double *__restrict__ Xb,
+                                                      long long wtotal, double *__restrict__ Pp, long long ptotal,
+                                                      SyncDev S) {
+    constexpr int NE = W / 4;
     const int t = take_ticket(S.tick + 1);
     if (t >= nwork) return;
     const int4 it = items[t / ngrp];
-    const int grp = t % ngrp;
-    const int q0 = grp * NR, nq = min(NR, nrhs - q0);
+    const int grp = t % ngrp, q0 = grp * wq, nq = min(wq, nrhs - q0);
     const int li = it.x;
     const SolveFront &Fr = P.sf[li];
     const int ne = Fr.ne, m = Fr.m, r = m - ne;
     const size_t lda = (size_t)m;
     const gdouble *L = gbl(Fr.F);
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int trow = tile_row(lane), qc = tile_col<W>(lane);
     const int nblk = (ne + SB - 1) / SB;
     const int fb = grp * P.nflag + Fr.fbase;
     const int nch = Fr.nchk;
-    __shared__ double cs[NR * SB];
-    __shared__ double tri[2 * TRI];
-    __shared__ double cti[64][65];
-    __shared__ double ws[NR * SB];
-    __shared__ double part[NR * 4 * 64];
-    const DiagLds dl{tri, tri + TRI, cti};
+    double *xg = x + (size_t)q0 * n;
+    double *Pg = Pp + (size_t)q0 * ptotal;
+    __shared__ __align__(16) double xs[2 * SB * W];
+    __shared__ double frags[2 * TFRAG];
+    static_assert(GH == 2 * SB, "a chunk's rows fill xs");
+    // x of the L21 rows ne + rb .. ne + rb + nr - 1 into xs, zeros beyond (device-coherent:
+    // ancestors write them in the same launch)
+    auto gather = [&](int rb, int nr) {
+        const gint *ri = gbl(Fr.sidx) + ne + rb;
+        constexpr int NI = GH * W / 256;
+        int g[NI];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int e = tid + 256 * i, row = e / W;
+            g[i] = (row < nr && e % W < nq) ? ri[row] : -1;
+            if (g[i] >= n) {
+                atomicOr(S.err, 2);  // an index outside the system: the solve plan does not fit the fronts
+                g[i] = -1;
+            }
+        }
+        double v[NI];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) v[i] = g[i] >= 0 ? ld_co(xg + (size_t)g[i] * nq + (tid + 256 * i) % W) : 0.0;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int e = tid + 256 * i;
+            xs[tcol_pos(e / W) * W + e % W] = v[i];
+        }
+    };
+    TCols<W> T;
+    // a chunk's first 128 rows ...
+    auto chunk_start = [&](int rb, int nr, int c0, int ncols) {
+        T.at(L, lda, ne + rb, min(SB, nr), c0, ncols);
+        if (32 * wv < ncols) T.load_all();
+    };
+    // ... and the sum over the chunk for this wavefront's 32 columns
+    auto chunk_sum = [&](int rb, int nr, int ncols) {
+        Tile2<W> v{{tile_zero<W>(), tile_zero<W>()}};
+        gather(rb, nr);
+        __syncthreads();
+        if (32 * wv < ncols) {
+            v = T.step(xs, SB, max(nr - SB, 0));
+            if (nr > SB) v = v + T.step(xs + SB * W, 0, 0);
+        }
+        return v;
+    };
     // chunk items and fused fronts read the x of L21 rows: every ancestor has finished
-    if (it.y != IT_BDIAG) {
+    auto wait_parent = [&]() {
         if (tid == 0 && Fr.epar >= 0)
             wait_at_least(S.bdone + (size_t)grp * P.nfront + Fr.epar, Fr.epar_nblk, S.err);
         __syncthreads();
-    }
+    };
     if (it.y == IT_BCHUNK) {
         const int C = it.z / nch, h = it.z % nch;
         const int c0 = C * SB, ncols = min(SB, ne - c0);
         const int rb = h * GH, nr = min(GH, r - rb);
-        double xv[NR][GH / 64];
-        gather_rows_x<NR>(Fr, rb, nr, x, n, q0, nq, xv, S.err);
-        tcol_product<NR, GH / 64>(L, lda, ne + rb, nr, c0, ncols, xv, nq, cs);
-        __syncthreads();
-        for (int e = tid; e < nq * SB; e += 256) {
-            const int q = e / SB, j = e % SB;
-            if (j < ncols) st_co(Pp + (size_t)(q0 + q) * ptotal + Fr.pbase + ((size_t)C * nch + h) * SB + j, cs[e]);
-        }
+        chunk_start(rb, nr, c0, ncols);
+        wait_parent();
+        const Tile2<W> v = chunk_sum(rb, nr, ncols);
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int e = 0; e < NE; ++e) {
+                const int j = 32 * wv + 16 * tt + trow, q = qc + e;
+                if (j < ncols && q < nq)
+                    st_co(Pg + (size_t)(Fr.pbase + ((long long)C * nch + h) * SB + j) * nq + q, v.t[tt].e[e]);
+            }
         stores_done_barrier();
         if (tid == 0) publish_add(S.bgc + fb + C);
         return;
     }
     // IT_BDIAG (column block C) or IT_BSMALL (the whole front, C = 0)
     const int C = it.z, j0 = C * SB;
-    const int nb = min(SB, ne - j0), n1 = min(64, nb), n2 = nb - n1;
-    // a fused front loads its diagonal block after the chunk products (fewer registers live
-    // across them); a diagonal item loads it first, its loads in flight during the waits
-    if (it.y == IT_BDIAG) load_diag_block(dl, L, lda, j0, n1, n2);
-    double acc[NR];
-    const int st = (tid < nb) ? gbl(Fr.sidx)[j0 + tid] : 0;
+    const int nb = min(SB, ne - j0);
+    Diag<false, W == 4> dg;
+    dg.load(L, lda, j0, nb, frags);
+    int st[2];  // global indices of the rows this lane finishes
+    Tile<W> acc[2];
 #pragma unroll
-    for (int q = 0; q < NR; ++q)
-        acc[q] = (tid < nb && q < nq) ? dsolve_col(Fr, j0 + tid, W + (size_t)(q0 + q) * wtotal + Fr.wbase) : 0.0;
+    for (int h = 0; h < 2; ++h) {
+        const int row = 64 * h + 16 * wv + trow;
+        st[h] = row < nb ? gbl(Fr.sidx)[j0 + row] : 0;
+        const int col = 32 * wv + 16 * h + trow;
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+            const int q = qc + e;
+            acc[h].e[e] = (col < nb && q < nq)
+                              ? dsolve_col(Fr, j0 + col, Wx + (size_t)q0 * wtotal + (size_t)Fr.wbase * nq + q, nq)
+                              : 0.0;
+        }
+    }
+    auto take_off = [&](const Tile2<W> &v) {
+        acc[0] = acc[0] - v.t[0];
+        acc[1] = acc[1] - v.t[1];
+    };
     if (it.y == IT_BSMALL) {
+        if (nch > 0) chunk_start(0, min(GH, r), 0, ne);
+        wait_parent();
         // L21^T x_rows chunk by chunk, subtracted in chunk order (as the chunk partials are)
         for (int h = 0; h < nch; ++h) {
             const int rb = h * GH, nr = min(GH, r - rb);
-            double xv[NR][GH / 64];
-            gather_rows_x<NR>(Fr, rb, nr, x, n, q0, nq, xv, S.err);
-            tcol_product<NR, GH / 64>(L, lda, ne + rb, nr, 0, ne, xv, nq, cs);
-            __syncthreads();
-            if (tid < nb) {
-#pragma unroll
-                for (int q = 0; q < NR; ++q)
-                    if (q < nq) acc[q] -= cs[q * SB + tid];
-            }
+            if (h > 0) chunk_start(rb, nr, 0, ne);
+            take_off(chunk_sum(rb, nr, ne));
             __syncthreads();
         }
-        load_diag_block(dl, L, lda, j0, n1, n2);
     } else if (r > 0) {
         if (tid == 0) wait_at_least(S.bgc + fb + C, nch, S.err);
         __syncthreads();
-        if (tid < nb) {
-            for (int h = 0; h < nch; ++h) {
+        for (int h = 0; h < nch; ++h) {
 #pragma unroll
-                for (int q = 0; q < NR; ++q)
-                    if (q < nq) acc[q] -= ld_co(Pp + (size_t)(q0 + q) * ptotal + Fr.pbase + ((size_t)C * nch + h) * SB + tid);
-            }
+            for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                for (int e = 0; e < NE; ++e) {
+                    const int j = 32 * wv + 16 * tt + trow, q = qc + e;
+                    if (j < nb && q < nq)
+                        acc[tt].e[e] -= ld_co(Pg + (size_t)(Fr.pbase + ((long long)C * nch + h) * SB + j) * nq + q);
+                }
         }
     }
-    // later blocks of the same front, as they are published (descending)
-    for (int Cp = nblk - 1; Cp > C; --Cp) {
-        const int i0 = Cp * SB, nr = min(SB, ne - i0);
-        // the tile is loaded before block Cp's flag is awaited (for Cp = C + 1 that wait ends the
-        // previous chain step; only the products remain after it)
-        double lv[4][2][8];
-        tcol_load2(L, lda, i0, nr, j0, nb, lv);
-        double xv[NR][2];
-        __syncthreads();  // cs of the previous block consumed
-        if (tid == 0) wait_at_least(S.bflag + fb + Cp, 1, S.err);
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int i = lane + 64 * u;
-#pragma unroll
-            for (int q = 0; q < NR; ++q)
-                xv[q][u] = (i < nr && q < nq) ? ld_co(Xb + (size_t)(q0 + q) * wtotal + Fr.wbase + i0 + i) : 0.0;
-        }
-        tcol_compute2<NR>(lv, xv, nq, nb, cs);
-        __syncthreads();
-        if (tid < nb) {
-#pragma unroll
-            for (int q = 0; q < NR; ++q)
-                if (q < nq) acc[q] -= cs[q * SB + tid];
+    // later blocks of the same front, as they are published (descending), a whole tile of L in
+    // flight ahead of the products
+    if (nblk - 1 > C) {
+        const double *Xf = Xb + (size_t)q0 * wtotal + (size_t)Fr.wbase * nq;
+        const bool act = 32 * wv < nb;
+        const int nr = ne - (nblk - 1) * SB;
+        T.at(L, lda, (nblk - 1) * SB, nr, j0, nb);
+        if (act) T.load_all();
+        XBlock<W, true> X;
+        if (X.AHEAD) X.ask(Xf + (size_t)(nblk - 1) * SB * nq, nr, nq);
+        for (int Cp = nblk - 1; Cp > C; --Cp) {
+            double *xb = xs + (Cp & 1) * (SB * W);
+            if (!X.AHEAD) X.ask(Xf + (size_t)Cp * SB * nq, Cp == nblk - 1 ? nr : SB, nq);
+            X.take(Cp <= C + NEAR, xb, S.err);
+            if (X.AHEAD && Cp > C + 1) X.ask(Xf + (size_t)(Cp - 1) * SB * nq, SB, nq);
+            if (act) take_off(T.step(xb, -SB, Cp > C + 1 ? SB : 0));
         }
     }
-    if (tid < nb) {
+    if (W != 4 && dg.n2 > 0) dg.load_c(L, lda, j0);
+    // The block's right-hand side, from which every later block and L21 have been removed, then its
+    // x with L11^T.  The half of xs that the last block of x did not use is free.
+    double *ws = xs + (C & 1) * (SB * W), *xo = xs + ((C + 1) & 1) * (SB * W);
 #pragma unroll
-        for (int q = 0; q < NR; ++q) ws[q * SB + tid] = acc[q];
-    }
+    for (int tt = 0; tt < 2; ++tt) tile_store<W>(ws + (32 * wv + 16 * tt) * W, acc[tt]);
     __syncthreads();
-    bwd_block<NR>(dl, ws, part, n1, n2, nq);
-    if (tid < nb) {
+    auto finish = [&](int h, int nn, const Tile<W> &v) {
 #pragma unroll
-        for (int q = 0; q < NR; ++q) {
-            if (q < nq) {
-                const double v = ws[q * SB + tid];
-                if (nblk > 1) st_co(Xb + (size_t)(q0 + q) * wtotal + Fr.wbase + j0 + tid, v);
-                if ((unsigned)st < (unsigned)n) st_co(x + (size_t)(q0 + q) * n + st, v);
+        for (int e = 0; e < NE; ++e) {
+            const int row = 16 * wv + trow, q = qc + e;
+            if (row < nn && q < nq) {
+                if (nblk > 1)
+                    publish_value(Xb + (size_t)q0 * wtotal + (size_t)(Fr.wbase + j0 + 64 * h + row) * nq + q, v.e[e]);
+                if ((unsigned)st[h] < (unsigned)n) st_co(xg + (size_t)st[h] * nq + q, v.e[e]);
                 else atomicOr(S.err, 2);
             }
         }
+    };
+    auto own = [&](int h) { return tile_load<W>(ws + (64 * h + 16 * wv) * W); };
+    Tile<W> wa = own(0);
+    if (dg.n2 > 0) {
+        const Tile<W> xb = own(1) + dg.template tri_sum<W>(1, ws);
+        tile_store<W>(xo + 16 * wv * W, xb);
+        finish(1, dg.n2, xb);
+        __syncthreads();
+        // C^T x_B: 16 sums over four rows, added as a binary tree
+        const double *xr = xo + (lane >> 4) * W + qc;
+        wa = wa - tree_sum<16, Tile<W>>(0, [&](int s) {
+                 Tile<W> p = tile_zero<W>();
+                 mma<W>(dg.c[s], xr + 4 * s * W, p);
+                 return p;
+             });
+        tile_store<W>(ws + 16 * wv * W, wa);
+        __syncthreads();
     }
+    finish(0, dg.n1, wa + dg.template tri_sum<W>(0, ws));
     stores_done_barrier();
-    if (tid == 0) {
-        if (nblk > 1) publish_set(S.bflag + fb + C);
-        publish_add(S.bdone + (size_t)grp * P.nfront + li);
-    }
+    if (tid == 0) publish_add(S.bdone + (size_t)grp * P.nfront + li);
 }
 
 }  // namespace
@@ -1197,16 +1286,23 @@ void NumericGPU::prepare_solve() {
     solve_ready_ = true;
 }
 
+// Columns per group of right-hand sides, dealt evenly to groups of at most 4 or, past 32 columns,
+// 8.  Groups of 4 have the shorter chain step, groups of 8 read the factor half as often, which
+// counts once the groups fill the chip.  Helmholtz 40^3, both sweeps, groups of 4 / of 8: 8 columns
+// 657 / 870 us, 16: 828 / 964, 32: 1190 / 1210, 64: 1985 / 1635.
+int NumericGPU::solve_group_width(int nrhs) {
+    if (nrhs <= 0) return 1;
+    const int most = nrhs <= 32 ? 4 : 8;
+    const int ngrp = (nrhs + most - 1) / most;
+    return (nrhs + ngrp - 1) / ngrp;
+}
+
 long long NumericGPU::solve_scratch_bytes(int nrhs) const {
     const int nr = solve_group_width(nrhs);
     const long long ngrp = nrhs > 0 ? (nrhs + nr - 1) / nr : 0;
-    const long long nsync = 2 + 1 + ngrp * (3LL * sm_.nflag + 2LL * sm_.nfront);
+    const long long nsync = 2 + 1 + ngrp * (1LL * sm_.nflag + 2LL * sm_.nfront);
     const long long doubles = ((long long)prep_->n + 2 * sm_.wtotal + sm_.ytotal + sm_.ptotal) * nrhs;
     return ((doubles * 8 + 255) / 256) * 256 + ((nsync * 4 + 255) / 256) * 256;
-}
-
-int NumericGPU::solve_group_width(int nrhs) {
-    return nrhs >= 8 ? 8 : nrhs >= 4 ? 4 : nrhs >= 2 ? 2 : 1;
 }
 
 void NumericGPU::solve(double *d_rhs, i64 ldrhs, int nrhs, const double *d_scaling) {
@@ -1227,8 +1323,8 @@ void NumericGPU::solve(double *d_rhs, i64 ldrhs, int nrhs, const double *d_scali
 void NumericGPU::solve_with(double *d_rhs, i64 ldrhs, int nrhs, const double *d_scaling, void *work) {
     const Prepared &P = *prep_;
     const i64 n = P.n;
-    const int NRW = solve_group_width(nrhs);
-    const int ngrp = (nrhs + NRW - 1) / NRW;
+    const int wq = solve_group_width(nrhs);
+    const int ngrp = (nrhs + wq - 1) / wq;
     const long long wt = sm_.wtotal, yt = sm_.ytotal, pt = sm_.ptotal, nn = n;
     double *xp = (double *)work;
     double *W = xp + (size_t)n * nrhs;
@@ -1237,13 +1333,11 @@ void NumericGPU::solve_with(double *d_rhs, i64 ldrhs, int nrhs, const double *d_
     double *Pp = Y + (size_t)yt * nrhs;
     const long long doubles = ((long long)n + 2 * wt + yt + pt) * nrhs;
     int *sync = (int *)((char *)work + ((doubles * 8 + 255) / 256) * 256);
-    const long long nsync = 3 + (long long)ngrp * (3LL * sm_.nflag + 2LL * sm_.nfront);
+    const long long nsync = 3 + (long long)ngrp * (1LL * sm_.nflag + 2LL * sm_.nfront);
     SyncDev S;
     S.tick = sync;
     S.err = sync + 2;
-    S.fflag = sync + 3;
-    S.bflag = S.fflag + (size_t)ngrp * sm_.nflag;
-    S.bgc = S.bflag + (size_t)ngrp * sm_.nflag;
+    S.bgc = sync + 3;
     S.fdone = S.bgc + (size_t)ngrp * sm_.nflag;
     S.bdone = S.fdone + (size_t)ngrp * sm_.nfront;
     sol_err_ = S.err;
@@ -1270,34 +1364,22 @@ void NumericGPU::solve_with(double *d_rhs, i64 ldrhs, int nrhs, const double *d_
                                (const SolveFront *)sm_.fronts, tp);
         inv_valid_ = true;
     }
-    const long long nstart = std::max<long long>(n, nsync);
-    hipLaunchKernelGGL(k_solve_start, dim3((unsigned)((nstart + 255) / 256)), dim3(256), 0, stream_, d_rhs,
-                       (long long)ldrhs, xp, nn, nrhs, P.d_perm_fwd, d_scaling, sync, nsync);
+    const dim3 gn((unsigned)((n + 255) / 256), (unsigned)ngrp);
+    hipLaunchKernelGGL(k_solve_start, gn, dim3(256), 0, stream_, d_rhs, (long long)ldrhs, xp, nn, nrhs, wq,
+                       P.d_perm_fwd, d_scaling, sync, nsync, (unsigned long long *)W, 2 * wt * nrhs);
     const int nfw = sm_.nfitems * ngrp, nbw = sm_.nbitems * ngrp;
-#define RV_SWEEPS(NRV)                                                                                        \
-    do {                                                                                                      \
-        if (nfw > 0)                                                                                          \
-            hipLaunchKernelGGL(k_fwd_sweep<NRV>, dim3((unsigned)nfw), dim3(256), 0, stream_, D, sm_.fitems,   \
-                               nfw, ngrp, nrhs, xp, nn, W, wt, Y, yt, S);                                     \
-        if (sm_.nunres > 0)                                                                                   \
-            hipLaunchKernelGGL(k_pull_rows, dim3((sm_.nunres + 255) / 256, nrhs), dim3(256), 0, stream_,       \
-                               sm_.unres, sm_.nunres, sm_.ptr, sm_.ent, (const double *)Y, yt, xp, nn);       \
-        if (nbw > 0)                                                                                          \
-            hipLaunchKernelGGL(k_bwd_sweep<NRV>, dim3((unsigned)nbw), dim3(256), 0, stream_, D, sm_.bitems,   \
-                               nbw, ngrp, nrhs, xp, nn, (const double *)W, Xb, wt, Pp, pt, S);                \
-    } while (0)
-    switch (NRW) {
-        case 8: RV_SWEEPS(8); break;
-        case 4: RV_SWEEPS(4); break;
-        case 2: RV_SWEEPS(2); break;
-        default: RV_SWEEPS(1); break;
-    }
-#undef RV_SWEEPS
-    const dim3 gp((unsigned)((n + 255) / 256), nrhs);
-    hipLaunchKernelGGL(k_perm_out, gp, dim3(256), 0, stream_, d_rhs, (long long)ldrhs, (const double *)xp, nn,
-                       P.d_perm_fwd, d_scaling);
+    if (nfw > 0)
+        hipLaunchKernelGGL((wq <= 4 ? k_fwd_sweep<4> : k_fwd_sweep<8>), dim3((unsigned)nfw), dim3(256), 0, stream_, D,
+                           sm_.fitems, nfw, ngrp, nrhs, wq, (const double *)xp, nn, W, wt, Y, yt, S);
+    if (sm_.nunres > 0)
+        hipLaunchKernelGGL(k_pull_rows, dim3((sm_.nunres + 255) / 256, nrhs), dim3(256), 0, stream_, sm_.unres,
+                           sm_.nunres, sm_.ptr, sm_.ent, (const double *)Y, yt, xp, nn, nrhs, wq);
+    if (nbw > 0)
+        hipLaunchKernelGGL((wq <= 4 ? k_bwd_sweep<4> : k_bwd_sweep<8>), dim3((unsigned)nbw), dim3(256), 0, stream_, D,
+                           sm_.bitems, nbw, ngrp, nrhs, wq, xp, nn, (const double *)W, Xb, wt, Pp, pt, S);
+    hipLaunchKernelGGL(k_perm_out, gn, dim3(256), 0, stream_, d_rhs, (long long)ldrhs, (const double *)xp, nn, nrhs,
+                       wq, P.d_perm_fwd, d_scaling);
 }
-
 
 // ===========================================================================
 // Fixed workspace of the allocation-free solve entry point: one array per GPU, held until the
