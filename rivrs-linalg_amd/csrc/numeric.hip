@@ -1071,10 +1071,12 @@ __device__ __forceinline__ void stores_done_barrier() {
 // the composite touches at most 2 MAX_IB lines U.  Outside U x U every other line q is independent:
 // a thread loads its q's entries of up to 32 touched lines (whole cycles of the permutation, all
 // loads of a round in flight) and stores them to the lines' new places; the U x U entries go
-// through S.swapbuf.  CO: device-scope accesses to the front (inside the persistent launch).
+// through S.swapbuf.  CO: device-scope accesses to the front (inside the persistent launch, where
+// the panels share the other lines).
 // Out of line: its registers stay out of the callers' common path.  Snapshotting whole lines to
 // memory one element and round trip at a time took a quarter of the factorization of a KKT system
-// with many delays (side 45: 28.4 ms, 21.9 so).
+// with many delays (side 45: 28.4 ms, 21.9 so); by the leader of the persistent launch alone the
+// lines still took 88 us a block, shared between its workgroups the step went from 17.9 to 13.6 ms.
 // ===========================================================================
 struct SwapLds {
     int U[2 * MAX_IB];     // touched lines
@@ -1084,18 +1086,11 @@ struct SwapLds {
     int gend[2 * MAX_IB];  // rounds of at most MAX_IB moves (whole cycles): end in mv
     int n, nmv, ng;        // (ng = 0: a cycle of more than MAX_IB lines)
 };
-template <bool CO>
-__device__ __attribute__((noinline)) void apply_swaps(FrontDev &F, AptpState &S, const int *sa, const int *sb, int nsw,
-                                                      SwapLds &W) {
+// The plan of a sequence of nsw swaps (all threads; ends with the barrier).
+__device__ __forceinline__ void swap_plan(SwapLds &W, const int *sa, const int *sb, int nsw) {
     static_assert(MAX_IB == 32, "a touched line per lane");
-    constexpr int AUX = CO ? 16 : 0;
-    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-    const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int m = F.m;
-    const size_t lda = m;
-    gdouble *A = gbl(F.F);
-    if (wv == 0) {
+    const int lane = threadIdx.x & 63;
+    if (threadIdx.x < 64) {
         // lane i: touched line i and the line whose content it ends with
         int line = -1, from = lane, nU = 0;
         const int la = lane < nsw ? sa[lane] : 0, lb = lane < nsw ? sb[lane] : 0;
@@ -1142,8 +1137,74 @@ __device__ __attribute__((noinline)) void apply_swaps(FrontDev &F, AptpState &S,
         }
     }
     __syncthreads();
+}
+
+// The touched lines' crossings with the lines [q_begin, q_end) outside U; a wavefront takes 64 of
+// these and one round.
+template <bool CO>
+__device__ __forceinline__ void swap_lines(FrontDev &F, const SwapLds &W, int q_begin, int q_end) {
+    constexpr int AUX = CO ? 16 : 0;
+    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+    const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m = F.m;
+    const size_t lda = m;
+    gdouble *A = gbl(F.F);
     const int nU = __builtin_amdgcn_readfirstlane(W.n), nmv = __builtin_amdgcn_readfirstlane(W.nmv);
-    if (nmv == 0) return;
+    const bool near = (size_t)m * m < (1u << 27);  // the front's offsets fit a buffer resource
+    const __amdgpu_buffer_rsrc_t ra = co_rsrc(A);
+    const int ul = W.U[lane], fl = W.from[lane], ml = W.mv[lane] & 63;
+    const int ng = near ? __builtin_amdgcn_readfirstlane(W.ng) : 0, ngx = max(ng, 1);
+    const int ntask = (q_end - q_begin + 63) / 64 * ngx;
+    // (every lane stays active: the lines are read across the lanes)
+    for (int task = wv; task < ntask; task += nw) {
+        const int g = task % ngx, q = q_begin + task / ngx * 64 + lane;
+        bool in = q < q_end;
+        for (int s = 0; s < nU; ++s) in = in && q != __builtin_amdgcn_readlane(ul, s);
+        if (ng > 0) {
+            const int g0 = g > 0 ? __builtin_amdgcn_readfirstlane(W.gend[g > 0 ? g - 1 : 0]) : 0;
+            const int n = __builtin_amdgcn_readfirstlane(W.gend[g]) - g0;
+            double v[MAX_IB];
+#pragma unroll
+            for (int s = 0; s < MAX_IB; ++s)
+                if (s < n) {
+                    const int u = __builtin_amdgcn_readlane(ul, __builtin_amdgcn_readlane(fl, __builtin_amdgcn_readlane(ml, g0 + s)));
+                    const unsigned off = in ? 8u * ((unsigned)max(q, u) + (unsigned)min(q, u) * (unsigned)m) : CO_OOB;
+                    v[s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(ra, (int)off, 0, AUX));
+                }
+#pragma unroll
+            for (int s = 0; s < MAX_IB; ++s)
+                if (s < n) {
+                    const int u = __builtin_amdgcn_readlane(ul, __builtin_amdgcn_readlane(ml, g0 + s));
+                    const unsigned off = in ? 8u * ((unsigned)max(q, u) + (unsigned)min(q, u) * (unsigned)m) : CO_OOB;
+                    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v[s]), ra, (int)off, 0, AUX);
+                }
+        } else if (in) {
+            // a long cycle, or a front past 8 GB: along each cycle, the first entry kept aside
+            double first = 0.0;
+            bool start = true;
+            for (int s = 0; s < nmv; ++s) {
+                const int w = W.mv[s], i = w & 63, u = W.U[i], f = W.U[W.from[i]];
+                gdouble *pu = A + max(q, u) + (size_t)min(q, u) * lda, *pf = A + max(q, f) + (size_t)min(q, f) * lda;
+                if (start) first = CO ? co_ld(pu) : *pu;
+                const double x = (w & 64) ? first : CO ? co_ld(pf) : *pf;
+                if (CO) co_st(pu, x);
+                else *pu = x;
+                start = (w & 64) != 0;
+            }
+        }
+    }
+}
+
+// The touched lines' crossings with each other (through S.swapbuf) and the row order.
+template <bool CO>
+__device__ __forceinline__ void swap_cross(FrontDev &F, AptpState &S, SwapLds &W) {
+    constexpr int AUX = CO ? 16 : 0;
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const int m = F.m;
+    const size_t lda = m;
+    gdouble *A = gbl(F.F);
+    const int nU = __builtin_amdgcn_readfirstlane(W.n);
     gdouble *buf = gbl(S.swapbuf);
     const bool near = (size_t)m * m < (1u << 27);  // the front's offsets fit a buffer resource
     const __amdgpu_buffer_rsrc_t ra = co_rsrc(A);
@@ -1166,48 +1227,6 @@ __device__ __attribute__((noinline)) void apply_swaps(FrontDev &F, AptpState &S,
     }
     if (tid < nU) W.ptmp[tid] = gbl(F.perm)[W.U[tid]];
     __syncthreads();
-    const int ul = W.U[lane], fl = W.from[lane], ml = W.mv[lane] & 63;
-    const int ng = near ? __builtin_amdgcn_readfirstlane(W.ng) : 0;
-    // (every lane stays active: the lines are read across the lanes)
-    for (int q0 = 64 * wv; q0 < m; q0 += nt) {
-        const int q = q0 + lane;
-        bool in = q < m;
-        for (int s = 0; s < nU; ++s) in = in && q != __builtin_amdgcn_readlane(ul, s);
-        int g0 = 0;
-        for (int g = 0; g < ng; ++g) {
-            const int g1 = __builtin_amdgcn_readfirstlane(W.gend[g]), n = g1 - g0;
-            double v[MAX_IB];
-#pragma unroll
-            for (int s = 0; s < MAX_IB; ++s)
-                if (s < n) {
-                    const int u = __builtin_amdgcn_readlane(ul, __builtin_amdgcn_readlane(fl, __builtin_amdgcn_readlane(ml, g0 + s)));
-                    const unsigned off = in ? 8u * ((unsigned)max(q, u) + (unsigned)min(q, u) * (unsigned)m) : CO_OOB;
-                    v[s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(ra, (int)off, 0, AUX));
-                }
-#pragma unroll
-            for (int s = 0; s < MAX_IB; ++s)
-                if (s < n) {
-                    const int u = __builtin_amdgcn_readlane(ul, __builtin_amdgcn_readlane(ml, g0 + s));
-                    const unsigned off = in ? 8u * ((unsigned)max(q, u) + (unsigned)min(q, u) * (unsigned)m) : CO_OOB;
-                    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v[s]), ra, (int)off, 0, AUX);
-                }
-            g0 = g1;
-        }
-        if (ng == 0 && in) {
-            // a long cycle, or a front past 8 GB: along each cycle, the first entry kept aside
-            double first = 0.0;
-            bool start = true;
-            for (int s = 0; s < nmv; ++s) {
-                const int w = W.mv[s], i = w & 63, u = W.U[i], f = W.U[W.from[i]];
-                gdouble *pu = A + max(q, u) + (size_t)min(q, u) * lda, *pf = A + max(q, f) + (size_t)min(q, f) * lda;
-                if (start) first = CO ? co_ld(pu) : *pu;
-                const double x = (w & 64) ? first : CO ? co_ld(pf) : *pf;
-                if (CO) co_st(pu, x);
-                else *pu = x;
-                start = (w & 64) != 0;
-            }
-        }
-    }
     for (int e = tid; e < nU * nU; e += nt) {
         const int x = e / nU, y = e % nU;
         const int p = W.U[x], r = W.U[y];
@@ -1218,8 +1237,52 @@ __device__ __attribute__((noinline)) void apply_swaps(FrontDev &F, AptpState &S,
         else A[p + (size_t)r * lda] = v;
     }
     if (tid < nU) gbl(F.perm)[W.U[tid]] = W.ptmp[W.from[tid]];
-    if (CO) stores_done_barrier();
-    else __syncthreads();
+}
+
+// The whole permutation by one workgroup.
+__device__ __attribute__((noinline)) void apply_swaps(FrontDev &F, AptpState &S, const int *sa, const int *sb, int nsw,
+                                                      SwapLds &W) {
+    swap_plan(W, sa, sb, nsw);
+    if (W.nmv > 0) {
+        swap_cross<false>(F, S, W);
+        swap_lines<false>(F, W, 0, F.m);
+    }
+    __syncthreads();
+}
+
+// Inside the persistent launch the permutation is shared: the leader's part (part < 0), and part of
+// np of the other lines.  Ends with the workgroup's stores complete.
+__device__ __forceinline__ void apply_swaps_shared(FrontDev &F, AptpState &S, const int *sa, const int *sb,
+                                                             int nsw, SwapLds &W, int part, int np) {
+    swap_plan(W, sa, sb, nsw);
+    if (W.nmv > 0) {
+        if (part < 0) {
+            swap_cross<true>(F, S, W);
+        } else {
+            const int per = (F.m + np - 1) / np;
+            swap_lines<true>(F, W, min(part * per, F.m), min((part + 1) * per, F.m));
+        }
+    }
+    stores_done_barrier();
+}
+
+// The swaps that move block [k, k + bs)'s failed columns (from nelim on; all with bn == 0) to the end
+// of the outer block: one thread; returns their number, end_pos is moved.
+__device__ __forceinline__ int failed_swaps(int k, int bs, int bn, int nelim, int &end_pos, int *sa, int *sb) {
+    int n = 0;
+    if (bn == 0) {
+        for (int off = 0; off < bs; ++off) {
+            end_pos -= 1;
+            if (k + off < end_pos) { sa[n] = k + off; sb[n] = end_pos; ++n; }
+        }
+    } else {
+        for (int i = bs - nelim - 1; i >= 0; --i) {
+            const int dp = k + nelim + i;
+            end_pos -= 1;
+            if (dp < end_pos) { sa[n] = dp; sb[n] = end_pos; ++n; }
+        }
+    }
+    return n;
 }
 
 // Diagonal tile of the next inner block after this block's update, formed in LDS with the
@@ -1626,24 +1689,11 @@ __global__ __launch_bounds__(256) void k_block_finish(FrontDev *__restrict__ fr,
         F.n1 += n1;
         F.n2 += n2;
         int end_pos = S.end_pos;
-        int n = 0;
-        if (bn == 0) {
-            for (int off = 0; off < bs; ++off) {
-                end_pos -= 1;
-                if (k + off < end_pos) { sa[n] = k + off; sb[n] = end_pos; ++n; }
-            }
-        } else {
-            for (int i = bs - nelim - 1; i >= 0; --i) {
-                const int dp = k + nelim + i;
-                end_pos -= 1;
-                if (dp < end_pos) { sa[n] = dp; sb[n] = end_pos; ++n; }
-            }
-        }
-        nsw = n;
+        nsw = failed_swaps(k, bs, bn, nelim, end_pos, sa, sb);
         s_end = end_pos;
     }
     __syncthreads();
-    apply_swaps<false>(F, S, sa, sb, nsw, sw);
+    apply_swaps(F, S, sa, sb, nsw, sw);
     if (tid == 0) {
         S.kpos = k + nelim;
         S.end_pos = s_end;
@@ -1728,6 +1778,7 @@ struct ChainSync {
     ChainCounter updated[CHAIN_MAX_IT];     // panels done with the updates of block it
     ChainCounter early[CHAIN_MAX_IT];       // panels that own rows of the block after the next and
                                             // have updated their first columns (no column failed)
+    ChainCounter swapped[CHAIN_MAX_IT];     // panels done with their share of the failed columns' swaps
     ChainRec recs[CHAIN_MAX_IT];
 };
 
@@ -1739,6 +1790,7 @@ __device__ __forceinline__ void chain_reset(ChainSync &C) {
         C.applied[i].aux = INT_MAX;
         C.updated[i].v = 0;
         C.early[i].v = 0;
+        C.swapped[i].v = 0;
     }
 }
 
@@ -1981,6 +2033,8 @@ struct ChainPanelLds {
     PivotCoef pc;
     int rec[4];
     int s_fail;
+    int sa[MAX_IB], sb[MAX_IB], nsw;     // (failed columns)
+    SwapLds sw;
 };
 union ChainLds {
     ChainLeaderLds ld;
@@ -2236,25 +2290,15 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
                 if (!upd_prev && !chain_wait(&C.updated[it].v, NP, &C.err.v)) return;
                 upd_prev = true;
                 if (tid == 0) {
-                    int n = 0;
-                    if (bn == 0) {
-                        for (int off = 0; off < bs; ++off) {
-                            end_pos -= 1;
-                            if (k + off < end_pos) { L.sa[n] = k + off; L.sb[n] = end_pos; ++n; }
-                        }
-                    } else {
-                        for (int i = bs - nelim - 1; i >= 0; --i) {
-                            const int dp = k + nelim + i;
-                            end_pos -= 1;
-                            if (dp < end_pos) { L.sa[n] = dp; L.sb[n] = end_pos; ++n; }
-                        }
-                    }
-                    L.nsw = n;
+                    L.nsw = failed_swaps(k, bs, bn, nelim, end_pos, L.sa, L.sb);
                     L.s_end = end_pos;
                 }
                 __syncthreads();
                 end_pos = L.s_end;
-                apply_swaps<true>(F, S, L.sa, L.sb, L.nsw, L.sw);
+                if (L.nsw > 0) {
+                    apply_swaps_shared(F, S, L.sa, L.sb, L.nsw, L.sw, -1, NP);
+                    if (!chain_wait(&C.swapped[it].v, NP, &C.err.v)) return;
+                }
             }
             k += nelim;
         }
@@ -2350,6 +2394,20 @@ __device__ __forceinline__ void cu_store(const double (&cv)[4][8], const double 
             co_stb(rc, ok ? (unsigned)(o + 128 * i) : CO_OOB, cv[i][q] - acc[i][q]);
         }
     }
+}
+
+// A block's failed columns move to the end of the outer block: the panel's share of the lines, after
+// every panel's restore and cross terms.  False when a wait ran out.
+__device__ __attribute__((noinline)) bool chain_panel_failed(FrontDev &F, AptpState &S, ChainSync &C, ChainPanelLds &L,
+                                                             int it, int k, int bs, int bn, int nelim, int end_pos,
+                                                             int pidx, int NP) {
+    if (threadIdx.x == 0) L.nsw = failed_swaps(k, bs, bn, nelim, end_pos, L.sa, L.sb);
+    __syncthreads();
+    if (L.nsw == 0) return true;
+    if (!chain_wait(&C.updated[it].v, NP, &C.err.v)) return false;
+    apply_swaps_shared(F, S, L.sa, L.sb, L.nsw, L.sw, pidx, NP);
+    if (threadIdx.x == 0) __hip_atomic_fetch_add(&C.swapped[it].v, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
 }
 
 // Panel rows of chunk c: [ob_start + c * CH, min(ob_start + (c + 1) * CH, m)).
@@ -2488,11 +2546,12 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
         __amdgpu_buffer_rsrc_t rc = co_rsrc_front(A, lda, (size_t)min(R0f, m - 1) + (size_t)min(be, m - 1) * lda);
         cu_load(cv, rc, lda, fast && be < obe);
         if (!chain_wait_aux(C.applied[it], NP + 2, &C.err.v, &L.s_fail)) return;
-        int permute_from = -1;
+        int permute_from = -1, nel = 0;
         if (bn > 0) {
             int nelim = min(L.s_fail, bn);
             if (nelim > 0 && L.bkind[nelim - 1] == 2) nelim -= 1;
             nelim = __builtin_amdgcn_readfirstlane(nelim);
+            nel = nelim;
             const int nbs = min(end_pos - be, ib);
             const bool ahead = nelim == bs && nbs > 0 && it + 1 < nit;
             const int lead = ahead ? be + nbs : be;
@@ -2689,6 +2748,10 @@ __device__ __forceinline__ void chain_panel(FrontDev &F, AptpState &S, ChainSync
         if (tid == 0) __hip_atomic_fetch_add(&C.updated[it].v, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // without failed columns nothing moves: the next block starts at be, its rows can come now
         pre_k = -1;
+        if (nel < bs) {
+            if (!chain_panel_failed(F, S, C, L, it, k, bs, bn, nel, end_pos, pidx, NP)) return;
+            continue;
+        }
         if (permute_from == 0 && single && pidx < nchunk && it + 1 < nit && end_pos > be) {
             pre_k = be;
             pre_bs = min(end_pos - be, ib);
@@ -2784,7 +2847,7 @@ __device__ bool outer_end(FrontDev &F, AptpState &S, int ob, int nb, int la) {
             nsw = n;
         }
         __syncthreads();
-        apply_swaps<false>(F, S, sa, sb, nsw, sw);
+        apply_swaps(F, S, sa, sb, nsw, sw);
         done += cnt_sw;
     }
     __syncthreads();
@@ -2824,7 +2887,7 @@ __global__ __launch_bounds__(256) void k_outer_end(FrontDev *__restrict__ fr,
 // The end of outer block ob and the start of ob + 1 in one launch (one workgroup per front).
 // la: block ob's trailing update runs beside this launch and block ob + 1 (planned without failed
 // columns in block ob).
-__global__ __launch_bounds__(256) void k_outer_next(FrontDev *__restrict__ fr,
+__global__ __launch_bounds__(512) void k_outer_next(FrontDev *__restrict__ fr,
                                                     AptpState *__restrict__ st,
                                                     const int *__restrict__ flist, int ob, int nb,
                                                     int ib, ChainSync *__restrict__ cs, int la) {
@@ -5012,7 +5075,7 @@ void NumericGPU::enqueue_level(int lv, const double *d_val, const double *d_scal
                 if (nhere) timed_outer(stream_, nhere, (const TileItem *)D(L.o_ot[ob][0]), dS, wpp);
             }
             if (ob + 1 < L.max_outer)
-                hipLaunchKernelGGL(k_outer_next, dim3(na), dim3(256), 0, stream_, d_fr_, dS, dl, ob, nb, ib, L.dC,
+                hipLaunchKernelGGL(k_outer_next, dim3(na), dim3(512), 0, stream_, d_fr_, dS, dl, ob, nb, ib, L.dC,
                                    la ? 1 : 0);
             else
                 hipLaunchKernelGGL(k_outer_end, dim3(na), dim3(256), 0, stream_, d_fr_, dS, dl, ob, nb);
