@@ -6,7 +6,7 @@
 //                    children without common rows, so a parent's entries sum their children in
 //                    reference order)
 //   2. dense factor  fronts with k < ib or inside a small-leaf subtree: k_tpp (threshold
-//                    partial pivoting, one wavefront per front);
+//                    partial pivoting, one workgroup per front);
 //                    other fronts: APTP with ib x ib complete pivoting blocks
 //                    (k_block_apply -> k_block_update -> k_block_finish per inner block, the
 //                    trailing update restricted to the outer block, and the rank-nb outer
@@ -189,15 +189,6 @@ __device__ __forceinline__ bool aptp_active(int p, int nb, int ib, int ob, int i
 __device__ __forceinline__ double wave_fmax(double v) {
     for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
     return v;
-}
-
-// larger value wins; equal values -> smaller index
-__device__ __forceinline__ void wave_argmax(double &v, int &idx) {
-    for (int o = 32; o > 0; o >>= 1) {
-        const double v2 = __shfl_xor(v, o);
-        const int i2 = __shfl_xor(idx, o);
-        if (v2 > v || (v2 == v && i2 < idx)) { v = v2; idx = i2; }
-    }
 }
 
 __device__ __forceinline__ int wave_min_int(int v) {
@@ -395,15 +386,6 @@ __device__ __forceinline__ double wave_max_dpp(double v) {
     v = fmax(v, dpp_f64<0x140>(v));  // row_mirror
     return fmax(fmax(readlane_f64(v, 0), readlane_f64(v, 16)),
                 fmax(readlane_f64(v, 32), readlane_f64(v, 48)));
-}
-
-// Position of the wavefront maximum: larger value wins, equal values -> smaller position.
-// vmax is the wavefront maximum of v; lanes without a candidate hold pos == INT_MAX.
-__device__ __forceinline__ int wave_argmax_pos(double v, int pos, double vmax) {
-    const unsigned long long mask = __ballot(pos != INT_MAX && v == vmax);
-    if (mask == 0) return INT_MAX;
-    if ((mask & (mask - 1)) == 0) return __builtin_amdgcn_readlane(pos, __ffsll((long long)mask) - 1);
-    return wave_min_int((v == vmax) ? pos : INT_MAX);
 }
 
 // Copy of the lower diagonal block [kpos, kpos + bs) of the next inner block (all threads of
@@ -698,10 +680,10 @@ __device__ __forceinline__ int block_pivots(const double (*blk)[MAX_IB + 1], dou
 }
 
 // All 256 threads: the block in blk (lower triangle) on entry; the factored block in position
-// order on return (D's off-diagonal of a 2x2 at (q + 1, q)).  blk2, lbuf, bp2: working LDS.
+// order on return (D's off-diagonal of a 2x2 at (q + 1, q)).  blk2, lbuf: working LDS.
 // Wavefronts 1 to 3 call `beside` while the first runs the pivot steps.
 template <class Beside>
-__device__ __forceinline__ int block_factor_wg(double (*blk)[MAX_IB + 1], double (*blk2)[MAX_IB + 1], int *bp, int *bp2,
+__device__ __forceinline__ int block_factor_wg(double (*blk)[MAX_IB + 1], double (*blk2)[MAX_IB + 1], int *bp,
                                                int8_t *bkind, double *bdiag, double *boff, int bs, double small,
                                                double *maxl, double *wbv, int *wbp, double (*lbuf)[MAX_IB + 1],
                                                Beside beside) {
@@ -875,7 +857,7 @@ __global__ __launch_bounds__(256) void k_block_apply(FrontDev *__restrict__ fr,
     __shared__ int8_t bkind[MAX_IB];
     __shared__ double bdiag[MAX_IB], boff[MAX_IB], dinv[MAX_IB];
     __shared__ double wbv[1];
-    __shared__ int wbp[1], bp2[MAX_IB];
+    __shared__ int wbp[1];
     __shared__ double lbuf[MAX_IB][MAX_IB + 1], blk2[MAX_IB][MAX_IB + 1];
     const int tid = threadIdx.x;
     const int r = be + chunk * 256 + tid;
@@ -947,7 +929,7 @@ __global__ __launch_bounds__(256) void k_block_apply(FrontDev *__restrict__ fr,
     lds_barrier();
     RV_PHASE(0, 1);
     double bml;
-    bn = block_factor_wg(blk, blk2, bp, bp2, bkind, bdiag, boff, bs, small, &bml, wbv, wbp, lbuf, [] {});
+    bn = block_factor_wg(blk, blk2, bp, bkind, bdiag, boff, bs, small, &bml, wbv, wbp, lbuf, [] {});
     RV_PHASE(0, 2);
     // D off-diagonals of 2x2 pivots read as zeros of L11 (factor.rs:1898-1912)
     if (tid < bn) {
@@ -1052,9 +1034,6 @@ __device__ __forceinline__ double co_ldo(__amdgpu_buffer_rsrc_t r, unsigned off)
 __device__ __forceinline__ void co_stb(__amdgpu_buffer_rsrc_t r, unsigned off, double v) {
     typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, (int)off, 0, 16);
-}
-__device__ __forceinline__ double co_ldd(const double *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void co_std(double *p, double v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1376,7 +1355,7 @@ __device__ void lookahead_factor(FrontDev &F, AptpState &S, double (*Wr)[MAX_IB 
     if (probe) { atomicAdd(&g_phase[1][6], clock64() - t_start); atomicAdd(&g_phase[1][5], 1ull); }
     const unsigned long long t0 = clock64();
 #endif
-    __shared__ int bp[MAX_IB], bp2[MAX_IB], operm[MAX_IB];
+    __shared__ int bp[MAX_IB], operm[MAX_IB];
     __shared__ int8_t bkind[MAX_IB];
     __shared__ double bdiag[MAX_IB], boff[MAX_IB];
     __shared__ double wbv[1];
@@ -1427,7 +1406,7 @@ __device__ void lookahead_factor(FrontDev &F, AptpState &S, double (*Wr)[MAX_IB 
 #ifdef RV_PHASE_TIMING
     if (probe) atomicAdd(&g_phase[1][2], clock64() - t0);
 #endif
-    const int bn = block_factor_wg(Ct, Wr, bp, bp2, bkind, bdiag, boff, nbs, small, &bml, wbv, wbp, Wr + MAX_IB,
+    const int bn = block_factor_wg(Ct, Wr, bp, bkind, bdiag, boff, nbs, small, &bml, wbv, wbp, Wr + MAX_IB,
                                    [] {});
 #ifdef RV_PHASE_TIMING
     if (probe) atomicAdd(&g_phase[1][3], clock64() - t0);
@@ -1729,12 +1708,15 @@ __global__ __launch_bounds__(256) void k_block_finish(FrontDev *__restrict__ fr,
 // on the device at once.  Per front one leader workgroup runs the pivot chain and NP panel
 // workgroups own chunks of CH rows from the outer block's first column down:
 //   leader, inner block it: factor the diagonal block (or take the one factored ahead), publish
-//     its pivots (record it); then, when the block eliminated every column, form the next
+//     its pivots and L11 (record it); then, when the block eliminated every column, form the next
 //     block's L rows itself (the panel substitution for those 32 rows), its diagonal tile after
-//     this block's update, and factor that tile ahead; once every panel has checked block it,
-//     keep the block factored ahead when no column failed (write it to the front, backup, column
-//     order) or, after failures, wait for the panels' restores, delay the failed columns to the
-//     end of the outer block (k_block_finish's swaps) and factor the next block afresh.
+//     this block's update, factor that tile ahead and write its record, unpublished; meanwhile two
+//     of its wavefronts store the current tile (they count among the NP + 2 of `applied`), and
+//     while one runs the pivots the others bring the operands of the block after it once the
+//     panels that own them report (`early`).  When every panel has checked block it, the next
+//     record is published if no column failed; after failures the panels' restores are awaited,
+//     the failed columns move to the end of the outer block (the panels swap the lines, `swapped`)
+//     and the next block is factored afresh.
 //   panel, inner block it: backup, column permutation, substitution and threshold check of its
 //     rows (k_block_apply), then, once every panel has checked, partial restore and cross terms,
 //     the update of the outer block's trailing columns in its rows (the tile factored ahead left
@@ -1876,7 +1858,7 @@ __device__ __forceinline__ bool wave_poll(ChainCounter &c, int target, int *err,
 // Substitution with L11 and D^-1 (factor.rs:1295-1408), four lanes per panel row: lane h of a
 // row's quad holds columns 4 t + h, t = 0 .. 7, so the serial chain of 496 multiply-subtract
 // pairs per row runs four columns wide and a panel's 64 rows fill the workgroup's four
-// wavefronts (one row per lane kept one wavefront busy: 4 us against 1).  Every column receives
+// wavefronts (one row per lane kept one wavefront of four busy).  Every column receives
 // its terms in ascending order, as the row form.
 template <int CTRL>
 __device__ __forceinline__ double quad_perm(double v) { return dpp_f64<CTRL>(v); }
@@ -2007,7 +1989,7 @@ struct ChainLeaderLds {
     double Wr[2 * MAX_IB][MAX_IB + 1];   // next block's L rows and W, then the factor's buffers
     double Yn[MAX_IB][MAX_IB + 1];       // next block's rows in the current block's columns
     double Cn[MAX_IB][MAX_IB + 1];       // next block's tile as it stands
-    int bp[MAX_IB], bp2[MAX_IB], nbp[MAX_IB], operm[MAX_IB], noperm[MAX_IB];
+    int bp[MAX_IB], nbp[MAX_IB], operm[MAX_IB], noperm[MAX_IB];
     int8_t bkind[MAX_IB], nbkind[MAX_IB];
     double bdiag[MAX_IB], boff[MAX_IB], nbdiag[MAX_IB], nboff[MAX_IB];
     PivotCoef pc;
@@ -2094,8 +2076,8 @@ __device__ __forceinline__ void load_operands(ChainLeaderLds &L, const gdouble *
 }
 
 // The pivot chain of a front's outer block.  Per inner block, once its record is out: substitution
-// of the next block's rows and its tile's update (4 + 2 of the 23 us), the next block's pivots on
-// the first wavefront, its record; when the panels' checks of the current block are in, the next
+// of the next block's rows and its tile's update (about 2 us each), the next block's pivots on the
+// first wavefront (14 to 20 us), its record; when the panels' checks of the current block are in, the next
 // record's flag goes up at once and the bookkeeping of the finished block follows.  Beside the
 // pivots the other wavefronts wait for the panels' updates of the current block and bring the
 // operands of the block after the next into LDS, and before them two wavefronts store the current
@@ -2147,7 +2129,7 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
             if (tid < MAX_IB) L.operm[tid] = (tid < bs) ? perm[k + tid] : 0;
             lds_barrier();
             double bml;
-            bn = block_factor_wg(L.blk, L.Wr, L.bp, L.bp2, L.bkind, L.bdiag, L.boff, bs, small, &bml, L.wbv, L.wbp,
+            bn = block_factor_wg(L.blk, L.Wr, L.bp, L.bkind, L.bdiag, L.boff, bs, small, &bml, L.wbv, L.wbp,
                                  L.Wr + MAX_IB, [] {});
             if (tid < bn && L.bkind[tid] == 2) L.blk[tid + 1][tid] = 0.0;
             if (tid < 64) pivot_coefs(L.bkind, L.bdiag, L.boff, bn, L.pc);
@@ -2209,7 +2191,7 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
 #pragma unroll
             for (int u = 0; u < MAX_IB / 8; ++u) L.Nv[ii][jg + 8 * u] = nv[u];
             const int be2 = be + nbs, nbs2 = min(end_pos - be2, ib);
-            bn2 = block_factor_wg(L.Ct, L.Wr, L.nbp, L.bp2, L.nbkind, L.nbdiag, L.nboff, nbs, small, &bml2, L.wbv,
+            bn2 = block_factor_wg(L.Ct, L.Wr, L.nbp, L.nbkind, L.nbdiag, L.nboff, nbs, small, &bml2, L.wbv,
                                   L.wbp, L.Wr + MAX_IB, [&] {
                 // with a failed column in the current block this block is discarded (and the panels
                 // have more to do): nothing to bring
