@@ -71,7 +71,7 @@ struct SolveFront {
     int nchk;            // backward: chunks per column block
     int ech0, ech1;      // effective children (nearest descendants with ne > 0) in ech
     int epar;            // effective parent or -1
-    int epar_nblk;       // its column blocks (backward done target)
+    int epar_nblk;       // its done target in the backward sweep (on top of the forward's)
 };
 
 // The solve plan as the kernels see it.
@@ -87,9 +87,8 @@ struct PlanDev {
 struct SyncDev {
     int *tick;   // [2] ticket counters of the two sweeps
     int *err;    // [1] set when a wait exceeded its limit
-    int *fdone;  // forward: rows items of the front finished
+    int *done;   // forward: rows items of the front finished; backward, counting on: its blocks
     int *bgc;    // backward: chunk items of the block finished
-    int *bdone;  // backward: blocks of the front finished
 };
 
 // Data that one workgroup of a sweep writes and another reads within the same launch (x blocks,
@@ -743,7 +742,7 @@ __global__ __launch_bounds__(256, 2) void k_fwd_sweep(PlanDev P, const int4 *__r
         fwd_rows<W, true>(L, lda, r0, nr, ne, Wf, nq, acc, xs, S.err);
         store_rows(acc, r0, nr);
         stores_done_barrier();
-        if (tid == 0) publish_add(S.fdone + (size_t)grp * P.nfront + li);
+        if (tid == 0) publish_add(S.done + (size_t)grp * P.nfront + li);
         return;
     }
     const int j0 = it.z * SB, nb = min(SB, ne - j0);
@@ -777,7 +776,7 @@ __global__ __launch_bounds__(256, 2) void k_fwd_sweep(PlanDev P, const int4 *__r
     if (wv == 0) {
         for (int e = Fr.ech0 + lane; e < Fr.ech1; e += 64) {
             const int2 ch = P.ech[e];
-            wait_at_least(S.fdone + (size_t)grp * P.nfront + ch.x, ch.y, S.err);
+            wait_at_least(S.done + (size_t)grp * P.nfront + ch.x, ch.y, S.err);
         }
     }
     __syncthreads();
@@ -861,7 +860,7 @@ __global__ __launch_bounds__(256, 2) void k_fwd_sweep(PlanDev P, const int4 *__r
         store_rows(acc, r0, nr);
     }
     stores_done_barrier();
-    if (tid == 0) publish_add(S.fdone + (size_t)grp * P.nfront + li);
+    if (tid == 0) publish_add(S.done + (size_t)grp * P.nfront + li);
 }
 
 // z = D^-1 y for column jj of a front (MixedDiagonal::solve_in_place, diagonal.rs:312-365):
@@ -954,7 +953,7 @@ __global__ __launch_bounds__(256, 2) void k_bwd_sweep(PlanDev P, const int4 *__r
     // chunk items and fused fronts read the x of L21 rows: every ancestor has finished
     auto wait_parent = [&]() {
         if (tid == 0 && Fr.epar >= 0)
-            wait_at_least(S.bdone + (size_t)grp * P.nfront + Fr.epar, Fr.epar_nblk, S.err);
+            wait_at_least(S.done + (size_t)grp * P.nfront + Fr.epar, Fr.epar_nblk, S.err);
         __syncthreads();
     };
     if (it.y == IT_BCHUNK) {
@@ -1080,7 +1079,7 @@ __global__ __launch_bounds__(256, 2) void k_bwd_sweep(PlanDev P, const int4 *__r
     }
     finish(0, dg.n1, wa + dg.template tri_sum<W>(0, ws));
     stores_done_barrier();
-    if (tid == 0) publish_add(S.bdone + (size_t)grp * P.nfront + li);
+    if (tid == 0) publish_add(S.done + (size_t)grp * P.nfront + li);
 }
 
 }  // namespace
@@ -1186,7 +1185,7 @@ void NumericGPU::prepare_solve() {
         f.ech0 = ech_ptr[li];
         f.ech1 = ech_ptr[li + 1];
         f.epar = epar[li];
-        f.epar_nblk = epar[li] >= 0 ? (ne_[flist[epar[li]]] + SB - 1) / SB : 0;
+        f.epar_nblk = epar[li] >= 0 ? ndone(epar[li]) + (ne_[flist[epar[li]]] + SB - 1) / SB : 0;
     }
     // items: forward by levels bottom-up, backward top-down.  Within a level: forward, the
     // diagonal (and fused) items by block step across fronts, then the rows items; backward, the
@@ -1300,7 +1299,7 @@ int NumericGPU::solve_group_width(int nrhs) {
 long long NumericGPU::solve_scratch_bytes(int nrhs) const {
     const int nr = solve_group_width(nrhs);
     const long long ngrp = nrhs > 0 ? (nrhs + nr - 1) / nr : 0;
-    const long long nsync = 2 + 1 + ngrp * (1LL * sm_.nflag + 2LL * sm_.nfront);
+    const long long nsync = 2 + 1 + ngrp * ((long long)sm_.nflag + sm_.nfront);
     const long long doubles = ((long long)prep_->n + 2 * sm_.wtotal + sm_.ytotal + sm_.ptotal) * nrhs;
     return ((doubles * 8 + 255) / 256) * 256 + ((nsync * 4 + 255) / 256) * 256;
 }
@@ -1333,13 +1332,12 @@ void NumericGPU::solve_with(double *d_rhs, i64 ldrhs, int nrhs, const double *d_
     double *Pp = Y + (size_t)yt * nrhs;
     const long long doubles = ((long long)n + 2 * wt + yt + pt) * nrhs;
     int *sync = (int *)((char *)work + ((doubles * 8 + 255) / 256) * 256);
-    const long long nsync = 3 + (long long)ngrp * (1LL * sm_.nflag + 2LL * sm_.nfront);
+    const long long nsync = 3 + (long long)ngrp * ((long long)sm_.nflag + sm_.nfront);
     SyncDev S;
     S.tick = sync;
     S.err = sync + 2;
     S.bgc = sync + 3;
-    S.fdone = S.bgc + (size_t)ngrp * sm_.nflag;
-    S.bdone = S.fdone + (size_t)ngrp * sm_.nfront;
+    S.done = S.bgc + (size_t)ngrp * sm_.nflag;
     sol_err_ = S.err;
     PlanDev D;
     D.sf = (const SolveFront *)sm_.fronts;
