@@ -3042,9 +3042,11 @@ __device__ __forceinline__ void tpp_swap(const TppMat<P> &M, int *lperm, int i, 
 }
 
 // Elimination of the 1x1 at ne (two = false) or the 2x2 at ne, ne + 1: the columns scaled to L, then
-// the fully-summed columns updated, TJ per wavefront and pass.  Returns the thread's largest |l|.
-template <int NT, int TJ, int RB, class P>
-__device__ __forceinline__ double tpp_apply(const TppMat<P> &M, int ne, bool two) {
+// the fully-summed columns updated, TJ per wavefront and pass.  LB: the new columns of L are also
+// kept in lb (LDS, 2 m doubles) and read from there, so that a pass over a front in memory waits
+// for its own entries only.  Returns the thread's largest |l|.
+template <int NT, int TJ, int RB, bool LB, class P>
+__device__ __forceinline__ double tpp_apply(const TppMat<P> &M, int ne, bool two, double *lb) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     P A = M.A;
     const size_t ld = M.ld;
@@ -3071,10 +3073,12 @@ __device__ __forceinline__ double tpp_apply(const TppMat<P> &M, int ne, bool two
                 const double l2 = (v2[t] * a11 - v1[t] * a21) * inv;
                 A[i + ne * ld] = l1;
                 A[i + (ne + 1) * ld] = l2;
+                if (LB) { lb[i] = l1; lb[M.m + i] = l2; }
                 ml = max_abs(max_abs(ml, l1), l2);
             } else {
                 const double l = v1[t] * inv;
                 A[i + ne * ld] = l;
+                if (LB) lb[i] = l;
                 ml = max_abs(ml, l);
             }
         }
@@ -3085,9 +3089,9 @@ __device__ __forceinline__ double tpp_apply(const TppMat<P> &M, int ne, bool two
 #pragma unroll
         for (int q = 0; q < TJ; ++q) {
             const int j = min(j0 + q, M.n - 1);
-            const double lj1 = A[j + ne * ld];
+            const double lj1 = LB ? lb[j] : A[j + ne * ld];
             if (two) {
-                const double lj2 = A[j + (ne + 1) * ld];
+                const double lj2 = LB ? lb[M.m + j] : A[j + (ne + 1) * ld];
                 w1[q] = lj1 * a11 + lj2 * a21;
                 w2[q] = lj1 * a21 + lj2 * a22;
             } else {
@@ -3101,8 +3105,8 @@ __device__ __forceinline__ double tpp_apply(const TppMat<P> &M, int ne, bool two
 #pragma unroll
             for (int r = 0; r < RB; ++r) {
                 const int i = min(i0 + 64 * r, M.m - 1);
-                l1[r] = A[i + ne * ld];
-                l2[r] = two ? A[i + (ne + 1) * ld] : 0.0;
+                l1[r] = LB ? lb[i] : A[i + ne * ld];
+                l2[r] = !two ? 0.0 : LB ? lb[M.m + i] : A[i + (ne + 1) * ld];
 #pragma unroll
                 for (int q = 0; q < TJ; ++q) c[q][r] = A[i + min(j0 + q, M.n - 1) * ld];
             }
@@ -3124,10 +3128,19 @@ __device__ __forceinline__ double tpp_apply(const TppMat<P> &M, int ne, bool two
     return ml;
 }
 
-// Threshold partial pivoting of a front's columns from c0 on.  Returns the columns eliminated; the
-// row order in lperm.
-template <int NT, int TJ, int RB, class P>
-__device__ __forceinline__ int tpp_run(const TppMat<P> &M, FrontDev &F, int c0, int *lperm, double u, double small) {
+// LDS of a staged front: its trapezoid's columns with an odd leading dimension (rows and columns
+// are read without bank conflicts), and the row order.
+__host__ __device__ __forceinline__ size_t tpp_lds_bytes(int m, int n) {
+    return ((size_t)(m | 1) * n * 8 + (size_t)n * 4 + 15) / 16 * 16;
+}
+constexpr size_t TPP_LDS_MAX = 158 * 1024;  // beside the workgroup's static LDS
+constexpr size_t TPP_LDS_SMALL = 38 * 1024;  // four workgroups per CU
+
+// Threshold partial pivoting of a front's columns from c0 on, until what is left fits in lds bytes
+// (0: to the end).  Returns the columns eliminated; the row order in lperm.
+template <int NT, int TJ, int RB, bool LB, class P>
+__device__ __forceinline__ int tpp_run(const TppMat<P> &M, FrontDev &F, int c0, int *lperm, double u, double small,
+                                       unsigned lds, double *lb) {
     constexpr int NW = NT / 64;
     __shared__ int s_code[NW], s_t[NW], s_ok;
     __shared__ double s_ml[NW];
@@ -3140,7 +3153,7 @@ __device__ __forceinline__ int tpp_run(const TppMat<P> &M, FrontDev &F, int c0, 
     auto set1 = [&](int col, double v) {
         if (tid == 0) { gbl(F.dkind)[c0 + col] = 1; gbl(F.ddiag)[c0 + col] = v; gbl(F.doff)[c0 + col] = 0.0; }
     };
-    while (nelim < n) {
+    while (nelim < n && !(lds && tpp_lds_bytes(M.m - nelim, n - nelim) <= lds)) {
         // rounds of candidates: in the first, wavefront 0 looks at column nelim itself
         int code = TPP_NONE, p = nelim, t = nelim;
         bool last_ok = false;
@@ -3187,7 +3200,7 @@ __device__ __forceinline__ int tpp_run(const TppMat<P> &M, FrontDev &F, int c0, 
                 gbl(F.ddiag)[c0 + nelim + 1] = M.A[(nelim + 1) + (nelim + 1) * M.ld];
                 gbl(F.doff)[c0 + nelim] = M.A[(nelim + 1) + nelim * M.ld]; gbl(F.doff)[c0 + nelim + 1] = 0.0;
             }
-            ml = max_abs(ml, tpp_apply<NT, TJ, RB>(M, nelim, true));
+            ml = max_abs(ml, tpp_apply<NT, TJ, RB, LB>(M, nelim, true, lb));
             ++n2;
             nelim += 2;
         } else {
@@ -3197,7 +3210,7 @@ __device__ __forceinline__ int tpp_run(const TppMat<P> &M, FrontDev &F, int c0, 
             }
             tpp_swap<NT>(M, lperm, p, nelim);
             set1(nelim, M.A[nelim + nelim * M.ld]);
-            ml = max_abs(ml, tpp_apply<NT, TJ, RB>(M, nelim, false));
+            ml = max_abs(ml, tpp_apply<NT, TJ, RB, LB>(M, nelim, false, lb));
             ++n1;
             nelim += 1;
         }
@@ -3215,97 +3228,103 @@ __device__ __forceinline__ int tpp_run(const TppMat<P> &M, FrontDev &F, int c0, 
     return nelim;
 }
 
-// LDS of a staged front: its trapezoid's columns with an odd leading dimension (rows and columns
-// are read without bank conflicts), and the row order.
-__host__ __device__ __forceinline__ size_t tpp_lds_bytes(int m, int n) {
-    return ((size_t)(m | 1) * n * 8 + (size_t)n * 4 + 15) / 16 * 16;
-}
-constexpr size_t TPP_LDS_MAX = 158 * 1024;  // beside the workgroup's static LDS
-constexpr size_t TPP_LDS_SMALL = 38 * 1024;  // four workgroups per CU
-
 // One workgroup per front: mode 0 the whole front, mode 1 the columns APTP left (from F.ne).  A
 // pivot step is a serial chain of scans, so its memory round trips decide: the columns still to
-// eliminate are staged in LDS where they fit (lds bytes; all but the widest fronts), otherwise the
-// front is worked on in place.  Rows of earlier columns follow the row order at the end.
+// eliminate are staged in LDS where they fit (lds bytes).  Wider remainders are worked on in place
+// until the rest fits, the step's new columns of L kept in LDS (mode 1; a wide front of mode 0 is
+// worked on in place throughout, its kernel keeps to few registers).  Rows of earlier columns follow
+// the row order at the end of either part.
 // KKT of side 16 (fronts up to 131 x 131): about 5 us a step, 26 us with every scan through L2 and a
-// workgroup reduction of its own.
+// workgroup reduction of its own.  422 left-over columns at the root of KKT 45: 5.3 ms in place
+// throughout on 1024 threads, 3.8 so on 512 (24 -> 15 us a step in memory, 4.7 staged).
 template <int NT, int TJ>
 __global__ __launch_bounds__(NT) void k_tpp(FrontDev *__restrict__ fr, const int *__restrict__ flist,
                                             int mode, double u, double small, unsigned lds) {
     extern __shared__ __align__(16) double dyn[];
     FrontDev &F = fr[flist[blockIdx.x]];
-    const int c0 = (mode == 0) ? 0 : F.ne;
-    const int n = F.k - c0, m = F.m - c0;
-    if (n <= 0) return;
     const size_t lda = F.m;
-    gdouble *G = gbl(F.F) + c0 + c0 * lda;
     const int tid = threadIdx.x;
-    int *lperm;
-    if (tpp_lds_bytes(m, n) <= lds) {
-        const size_t ld = m | 1;
-        lperm = (int *)(dyn + ld * n);
-        for (int j0 = tid >> 6; j0 < n; j0 += NT / 64 * 4)
-            for (int i = (tid & 63); i < m; i += 64) {
-                double v[4];
+    int c0 = (mode == 0) ? 0 : F.ne;
+    for (bool more = c0 < F.k; more;) {
+        const int n = F.k - c0, m = F.m - c0;
+        gdouble *G = gbl(F.F) + c0 + c0 * lda;
+        int *lperm;
+        int nelim = 0;
+        more = false;
+        if (tpp_lds_bytes(m, n) <= lds) {
+            const size_t ld = m | 1;
+            lperm = (int *)(dyn + ld * n);
+            for (int j0 = tid >> 6; j0 < n; j0 += NT / 64 * 4)
+                for (int i = (tid & 63); i < m; i += 64) {
+                    double v[4];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) v[q] = G[i + (size_t)min(j0 + q * (NT / 64), n - 1) * lda];
+                    for (int q = 0; q < 4; ++q) v[q] = G[i + (size_t)min(j0 + q * (NT / 64), n - 1) * lda];
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    if (j0 + q * (NT / 64) < n) dyn[i + (j0 + q * (NT / 64)) * ld] = v[q];
-            }
-        __syncthreads();
-        tpp_run<NT, TJ, 2>(TppMat<double *>{dyn, ld, m, n}, F, c0, lperm, u, small);
-        for (int j = tid >> 6; j < n; j += NT / 64)
-            for (int i = j + (tid & 63); i < m; i += 64) G[i + (size_t)j * lda] = dyn[i + j * ld];
-    } else {
-        lperm = F.sidx + c0;  // (written by k_collect after the factorization)
-        tpp_run<NT, TJ, 4>(TppMat<gdouble *>{G, lda, m, n}, F, c0, lperm, u, small);
-    }
-    __syncthreads();
-    // perm and the earlier columns' rows [c0, c0 + n) in the new order, columns dealt to the wavefronts
-    // (one register per lane and 64 rows; every load of a column before its stores)
-    gint *perm = gbl(F.perm) + c0;
-    constexpr int RB = 16;
-    if (n <= 64 * RB) {
-        for (int q = (tid >> 6) - 1; q < c0; q += NT / 64) {
-            gdouble *col = gbl(F.F) + c0 + (size_t)max(q, 0) * lda;
-            double v[RB];
-            int pv[RB];
-#pragma unroll
-            for (int r = 0; r < RB; ++r) {
-                const int i = (tid & 63) + 64 * r;
-                if (i >= n) continue;
-                if (q < 0) pv[r] = perm[lperm[i]];
-                else v[r] = col[lperm[i]];
-            }
-            __builtin_amdgcn_s_waitcnt(0);
-#pragma unroll
-            for (int r = 0; r < RB; ++r) {
-                const int i = (tid & 63) + 64 * r;
-                if (i >= n) continue;
-                if (q < 0) perm[i] = pv[r];
-                else col[i] = v[r];
-            }
-        }
-    } else {
-        // more columns left over: one column per thread, cycle by cycle (from each cycle's smallest row)
-        for (int q = tid - 1; q < c0; q += NT) {
-            gdouble *col = gbl(F.F) + c0 + (size_t)max(q, 0) * lda;
-            for (int i = 0; i < n; ++i) {
-                int a = lperm[i];
-                while (a > i) a = lperm[a];
-                if (a < i || lperm[i] == i) continue;
-                const double v = col[i];
-                const int pv = q < 0 ? perm[i] : 0;
-                a = i;
-                for (int b; (b = lperm[a]) != i; a = b) {
-                    if (q < 0) perm[a] = perm[b];
-                    else col[a] = col[b];
+                    for (int q = 0; q < 4; ++q)
+                        if (j0 + q * (NT / 64) < n) dyn[i + (j0 + q * (NT / 64)) * ld] = v[q];
                 }
-                if (q < 0) perm[a] = pv;
-                else col[a] = v;
+            __syncthreads();
+            tpp_run<NT, TJ, 2, false>(TppMat<double *>{dyn, ld, m, n}, F, c0, lperm, u, small, 0, nullptr);
+            for (int j = tid >> 6; j < n; j += NT / 64)
+                for (int i = j + (tid & 63); i < m; i += 64) G[i + (size_t)j * lda] = dyn[i + j * ld];
+        } else {
+            lperm = F.sidx + c0;  // (written by k_collect after the factorization)
+            const TppMat<gdouble *> M{G, lda, m, n};
+            if (NT > 256 && (size_t)m * 16 <= lds) {
+                nelim = tpp_run<NT, TJ, 4, true>(M, F, c0, lperm, u, small, lds, dyn);
+                more = nelim < n && tpp_lds_bytes(m - nelim, n - nelim) <= lds;
+            } else {
+                tpp_run<NT, TJ, 4, false>(M, F, c0, lperm, u, small, 0, nullptr);
             }
         }
+        __syncthreads();
+        // perm and the earlier columns' rows [c0, c0 + n) in the new order, columns dealt to the wavefronts
+        // (one register per lane and 64 rows; every load of a column before its stores)
+        gint *perm = gbl(F.perm) + c0;
+        constexpr int RB = 16;
+        if (n <= 64 * RB) {
+            for (int q = (tid >> 6) - 1; q < c0; q += NT / 64) {
+                gdouble *col = gbl(F.F) + c0 + (size_t)max(q, 0) * lda;
+                double v[RB];
+                int pv[RB];
+#pragma unroll
+                for (int r = 0; r < RB; ++r) {
+                    const int i = (tid & 63) + 64 * r;
+                    if (i >= n) continue;
+                    if (q < 0) pv[r] = perm[lperm[i]];
+                    else v[r] = col[lperm[i]];
+                }
+                __builtin_amdgcn_s_waitcnt(0);
+#pragma unroll
+                for (int r = 0; r < RB; ++r) {
+                    const int i = (tid & 63) + 64 * r;
+                    if (i >= n) continue;
+                    if (q < 0) perm[i] = pv[r];
+                    else col[i] = v[r];
+                }
+            }
+        } else {
+            // more columns left over: one column per thread, cycle by cycle (from each cycle's smallest row)
+            for (int q = tid - 1; q < c0; q += NT) {
+                gdouble *col = gbl(F.F) + c0 + (size_t)max(q, 0) * lda;
+                for (int i = 0; i < n; ++i) {
+                    int a = lperm[i];
+                    while (a > i) a = lperm[a];
+                    if (a < i || lperm[i] == i) continue;
+                    const double v = col[i];
+                    const int pv = q < 0 ? perm[i] : 0;
+                    a = i;
+                    for (int b; (b = lperm[a]) != i; a = b) {
+                        if (q < 0) perm[a] = perm[b];
+                        else col[a] = col[b];
+                    }
+                    if (q < 0) perm[a] = pv;
+                    else col[a] = v;
+                }
+            }
+        }
+        c0 += nelim;
+        __syncthreads();
     }
 }
 
@@ -5083,7 +5102,7 @@ void NumericGPU::enqueue_level(int lv, const double *d_val, const double *d_scal
             la_pending = false;
         }
         if (o_.failed_pivot_tpp)
-            hipLaunchKernelGGL((k_tpp<1024, 4>), dim3(na), dim3(1024), TPP_LDS_MAX, stream_, d_fr_, dl, 1, o_.threshold,
+            hipLaunchKernelGGL((k_tpp<512, 4>), dim3(na), dim3(512), TPP_LDS_MAX, stream_, d_fr_, dl, 1, o_.threshold,
                                o_.small, (unsigned)TPP_LDS_MAX);
     }
     // ---- kept factor columns of the pooled fronts: final from here on, read beside the

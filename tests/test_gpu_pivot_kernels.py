@@ -57,6 +57,16 @@ def test_swapped_columns_match_oracle(m, p, kind):
     _same(_matrix(m, 300 + m + p, kind), p)
 
 
+# A root whose columns mostly fail: threshold pivoting takes them in memory until the rest fits in
+# LDS (140 square), then there; a remainder that fits from the start, one just above, wide ones.
+@pytest.mark.parametrize("m", [150, 180, 300, 420])
+@pytest.mark.parametrize("kind", ["delays", "pairs"])
+def test_left_over_columns_match_oracle(m, kind):
+    print("left-over columns m=%d %s" % (m, kind), flush=True)
+    ref = _same(_matrix(m, 400 + m, kind), m)
+    assert ref["num_eliminated"] == m
+
+
 def _matrix(m, seed, kind):
     rng = np.random.default_rng(seed)
     if kind == "ties":
@@ -65,6 +75,11 @@ def _matrix(m, seed, kind):
     a = gen.deterministic_indefinite_matrix(m, seed, 0.1)
     if kind == "delays":
         return gen.cause_delays(a, seed, 1000.0)
+    if kind == "pairs":  # large couplings between the halves: no block of 32 has an acceptable pivot
+        d = rng.permutation(m // 2)
+        a[m - m // 2 + np.arange(m // 2), d] += 1e4
+        a[d, m - m // 2 + np.arange(m // 2)] += 1e4
+        return a
     if kind == "saddle":
         a[np.arange(m), np.arange(m)] = np.where(rng.random(m) < 0.5, 0.0, np.diag(a))
         return a
