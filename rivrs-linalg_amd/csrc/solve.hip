@@ -28,7 +28,7 @@
 // A right-hand-side group of up to 8 columns shares every load of L.  All sums run in a fixed
 // order: results do not depend on scheduling, nor on the number of columns.
 //
-// A single right-hand side is bound by the chain of diagonal blocks (75 of them on the way to the
+// A single right-hand side is bound by the chain of diagonal blocks (97 of them on the way to the
 // root of a Helmholtz 64^3 factor): a block's x is on its way to the next workgroup for about 2 us,
 // its products take half a microsecond and its triangles one.
 #pragma clang fp contract(off)
@@ -314,7 +314,8 @@ __global__ __launch_bounds__(64) void k_diag_inverse(const SolveFront *__restric
 // columns; on the VALU every product took an LDS read of x.
 // Why not v_mfma_f64_16x16x4 and 16 columns: a sweep is bound by its chain of diagonal blocks, and a
 // step of the chain takes as long as the products of one workgroup.  Helmholtz 40^3, both sweeps:
-// 8 right-hand sides 2.0 ms on the VALU, 1.37 on the wide instruction, 0.66 in groups of 4.
+// 8 right-hand sides 2.58 ms on the VALU, 1.37 on the wide instruction, 0.66 in groups of 4 (one
+// column 0.87 on the VALU, 0.58 now; 64 columns 5.39 and 1.63).
 // Element e of lane l is row tile_row(l) of the tile, column tile_col(l) + e: a lane's columns are
 // adjacent and come with one read.
 // ---------------------------------------------------------------------------
