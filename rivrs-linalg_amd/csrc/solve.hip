@@ -42,6 +42,7 @@
 
 #include "../../include/rivrs_ldlt.h"
 #include "rv_numeric.h"
+#include "rv_poll.h"
 
 namespace rv {
 
@@ -49,7 +50,7 @@ namespace {
 
 constexpr int SB = 128;  // diagonal block of the blocked triangular solves (two 64-column halves)
 constexpr int GH = 256;  // L21 rows per backward column-chunk item
-constexpr long long SPIN_LIMIT = 1LL << 22;
+constexpr int SPIN_LIMIT = 1 << 22;
 
 // Item kinds.  A front with one diagonal block and at most FUSE_R rows of L21 is one fused item
 // per sweep; larger fronts split into diagonal, rows and chunk items.
@@ -412,29 +413,24 @@ struct XBlock {
     }
     __device__ __forceinline__ void take(bool near, double *xb, int *err) {
         const int tid = threadIdx.x;
-        int spins = 0;
-        auto pause = [&]() {  // false: give up
-            if ((++spins & 63) == 0 &&
-                (spins > SPIN_LIMIT || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
-                atomicOr(err, 1);
-                return false;
-            }
-            __builtin_amdgcn_s_sleep(1);
-            return true;
-        };
-        for (;;) {
-            bool bad = false;
+        SpinBudget budget{SPIN_LIMIT};
+        wait_words(
+            near,
+            [&] {
+                bool bad = false;
 #pragma unroll
-            for (int i = 0; i < NI; ++i) bad |= v[i] == UNSET;
-            if (!__any(bad)) break;
-            if (!near) {
-                const double *last = src + (size_t)n * nq - 1;
-                while (ld_bits(last) == UNSET)
-                    if (!pause()) break;
-            }
-            if (!pause()) break;
-            reload();
-        }
+                for (int i = 0; i < NI; ++i) bad |= v[i] == UNSET;
+                return (bool)__any(bad);
+            },
+            [&] { return ld_bits(src + (size_t)n * nq - 1) == UNSET; }, [&] { reload(); },
+            [&] {
+                if (budget.spent([&] { return __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0; })) {
+                    atomicOr(err, 1);
+                    return true;
+                }
+                __builtin_amdgcn_s_sleep(1);
+                return false;
+            });
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const int e = tid + 256 * i;
