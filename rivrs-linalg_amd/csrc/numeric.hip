@@ -3136,6 +3136,24 @@ __host__ __device__ __forceinline__ size_t tpp_lds_bytes(int m, int n) {
 constexpr size_t TPP_LDS_MAX = 158 * 1024;  // beside the workgroup's static LDS
 constexpr size_t TPP_LDS_SMALL = 38 * 1024;  // four workgroups per CU
 
+// The launches of a level's TPP fronts.
+//  * TPP_SMALL: four wavefronts per front, staged, at least four fronts to a CU.
+//  * TPP_WAVE, for more than TPP_WAVE_MIN fronts of at most a row per lane: one wavefront each, sixteen
+//    to a CU.  Four scan a line no sooner, and their idle lanes and barriers take the place of three other
+//    fronts.  Refactorization of independent systems, one / four wavefronts, ms: 24 x 24, 500 of
+//    them 0.14 / 0.12, 1000 0.17 / 0.18, 2000 0.21 / 0.27, 20000 1.10 / 2.02; 8 x 8, 1000 0.08 / 0.10,
+//    2000 0.11 / 0.14, 20000 0.54 / 0.89.
+//  * TPP_MID, for more than TPP_MID_MIN fronts of which only one fits on a CU: in place on two wavefronts
+//    until the rest is small, four to a CU.  Up to that number staging them whole is the shorter
+//    chain, and so it is where two fit.  In parts / whole, ms: 104 x 104, 512 of them 0.94 / 0.92, 700
+//    1.05 / 1.28, 3000 3.42 / 4.93; 120 x 120, 200 0.92 / 0.59, 512 1.17 / 1.08, 700 1.32 / 1.52, 3000 4.29 /
+//    5.80; 140 x 140, 512 1.56 / 1.33, 700 1.74 / 1.90, 3000 5.93 / 7.42; 100 x 100, 700 0.98 / 0.94, 6000
+//    6.14 / 6.03; past the LDS (160 x 160) 700 2.63 / 2.46, 6000 18.7 / 18.7.
+//  * TPP_WIDE: four wavefronts, staged whole or in place throughout.
+enum TppClass { TPP_WAVE = 0, TPP_SMALL = 1, TPP_MID = 2, TPP_WIDE = 3 };
+constexpr int TPP_WAVE_MIN = 1024, TPP_MID_MIN = 512;
+constexpr size_t TPP_LDS_WAVE = 10 * 1024, TPP_LDS_HALF = 79 * 1024;
+
 // Threshold partial pivoting of a front's columns from c0 on, until what is left fits in lds bytes
 // (0: to the end).  Returns the columns eliminated; the row order in lperm.
 template <int NT, int TJ, int RB, bool LB, class P>
@@ -3230,14 +3248,14 @@ __device__ __forceinline__ int tpp_run(const TppMat<P> &M, FrontDev &F, int c0, 
 
 // One workgroup per front: mode 0 the whole front, mode 1 the columns APTP left (from F.ne).  A
 // pivot step is a serial chain of scans, so its memory round trips decide: the columns still to
-// eliminate are staged in LDS where they fit (lds bytes).  Wider remainders are worked on in place
-// until the rest fits, the step's new columns of L kept in LDS (mode 1; a wide front of mode 0 is
-// worked on in place throughout, its kernel keeps to few registers).  Rows of earlier columns follow
+// eliminate are staged in LDS where they fit (lds bytes).  PARTS: wider remainders are worked on in
+// place until the rest fits, the step's new columns of L kept in LDS (without it a wide front is
+// worked on in place throughout, the kernel keeps to few registers).  Rows of earlier columns follow
 // the row order at the end of either part.
 // KKT of side 16 (fronts up to 131 x 131): about 5 us a step, 26 us with every scan through L2 and a
 // workgroup reduction of its own.  422 left-over columns at the root of KKT 45: 5.3 ms in place
 // throughout on 1024 threads, 3.8 so on 512 (24 -> 15 us a step in memory, 4.7 staged).
-template <int NT, int TJ>
+template <int NT, int TJ, bool PARTS>
 __global__ __launch_bounds__(NT) void k_tpp(FrontDev *__restrict__ fr, const int *__restrict__ flist,
                                             int mode, double u, double small, unsigned lds) {
     extern __shared__ __align__(16) double dyn[];
@@ -3270,7 +3288,7 @@ __global__ __launch_bounds__(NT) void k_tpp(FrontDev *__restrict__ fr, const int
         } else {
             lperm = F.sidx + c0;  // (written by k_collect after the factorization)
             const TppMat<gdouble *> M{G, lda, m, n};
-            if (NT > 256 && (size_t)m * 16 <= lds) {
+            if (PARTS && (size_t)m * 16 <= lds) {
                 nelim = tpp_run<NT, TJ, 4, true>(M, F, c0, lperm, u, small, lds, dyn);
                 more = nelim < n && tpp_lds_bytes(m - nelim, n - nelim) <= lds;
             } else {
@@ -4678,19 +4696,24 @@ void NumericGPU::plan_level(int lv, bool reset_arena) {
     L.o_sch = stage_push(stg, sch.data(), sch.size());
     L.nsch = sch.size();
     const size_t o_maps = stage_push(stg, maps.data(), maps.size());
-    // (small: staged in LDS with four workgroups per CU)
     auto tpp_need = [&](int s) { return tpp_lds_bytes(m_[s], k_[s]); };
-    const auto tpp_mid = std::stable_partition(tpp_list.begin(), tpp_list.end(),
-                                               [&](int s) { return tpp_need(s) <= TPP_LDS_SMALL; });
-    L.ntpp_small = tpp_mid - tpp_list.begin();
-    L.tpp_lds[0] = L.tpp_lds[1] = 0;
-    for (size_t i = 0; i < tpp_list.size(); ++i)
-        if (tpp_need(tpp_list[i]) <= TPP_LDS_MAX) {
-            size_t &b = L.tpp_lds[i < L.ntpp_small ? 0 : 1];
-            b = std::max(b, tpp_need(tpp_list[i]));
-        }
+    auto tpp_wave = [&](int s) { return m_[s] <= 64 && tpp_need(s) <= TPP_LDS_WAVE; };
+    auto tpp_mid = [&](int s) { return tpp_need(s) > TPP_LDS_HALF && tpp_need(s) <= TPP_LDS_MAX; };
+    const bool waves = std::count_if(tpp_list.begin(), tpp_list.end(), tpp_wave) > TPP_WAVE_MIN;
+    const bool mids = std::count_if(tpp_list.begin(), tpp_list.end(), tpp_mid) > TPP_MID_MIN;
+    auto tpp_class = [&](int s) {
+        return waves && tpp_wave(s) ? TPP_WAVE : tpp_need(s) <= TPP_LDS_SMALL ? TPP_SMALL : mids && tpp_mid(s) ? TPP_MID : TPP_WIDE;
+    };
+    std::stable_sort(tpp_list.begin(), tpp_list.end(), [&](int a, int b) { return tpp_class(a) < tpp_class(b); });
+    std::fill(L.ntpp, L.ntpp + 4, 0);
+    std::fill(L.tpp_lds, L.tpp_lds + 4, 0);
+    for (int s : tpp_list) {
+        const int c = tpp_class(s);
+        ++L.ntpp[c];
+        if (tpp_need(s) <= TPP_LDS_MAX) L.tpp_lds[c] = std::max(L.tpp_lds[c], tpp_need(s));
+    }
+    L.tpp_lds[TPP_MID] = std::min(L.tpp_lds[TPP_MID], TPP_LDS_SMALL);
     L.o_tpp = stage_push(stg, tpp_list.data(), tpp_list.size());
-    L.ntpp = tpp_list.size();
     L.o_aptp = stage_push(stg, aptp_list.data(), aptp_list.size());
     // extend-add items per round; map fields hold blob offsets until the device copy exists
     std::vector<std::vector<EaItem>> ea_rounds(nrounds);
@@ -5007,16 +5030,15 @@ void NumericGPU::enqueue_level(int lv, const double *d_val, const double *d_scal
             hipLaunchKernelGGL(k_extend_add, dim3((unsigned)L.n_ea[r]), dim3(256), 0, stream_, d_fr_,
                                (const EaItem *)D(L.o_ea[r]));
     // ---- TPP fronts ----
-    if (L.ntpp) {
-        // fronts whose staged columns leave room for several workgroups per CU first, then the rest
-        // (so that one wide front does not take the other fronts' residency)
-        for (int c = 0; c < 2; ++c) {
-            const size_t n = c ? L.ntpp - L.ntpp_small : L.ntpp_small;
-            if (!n) continue;
-            hipLaunchKernelGGL((k_tpp<256, 4>), dim3((unsigned)n), dim3(256), L.tpp_lds[c], stream_, d_fr_,
-                               (const int *)D(L.o_tpp) + (c ? L.ntpp_small : 0), 0, o_.threshold, o_.small,
-                               (unsigned)L.tpp_lds[c]);
-        }
+    // (launches of their own: one wide front does not take the other fronts' residency)
+    const int *tpp = (const int *)D(L.o_tpp);
+    for (int c = 0; c < 4; ++c) {
+        const unsigned n = (unsigned)L.ntpp[c], lds = (unsigned)L.tpp_lds[c];
+        if (!n) continue;
+        const auto kernel = c == TPP_WAVE ? k_tpp<64, 2, false> : c == TPP_MID ? k_tpp<128, 4, true> : k_tpp<256, 4, false>;
+        hipLaunchKernelGGL(kernel, dim3(n), dim3(c == TPP_WAVE ? 64 : c == TPP_MID ? 128 : 256), lds, stream_, d_fr_, tpp, 0,
+                           o_.threshold, o_.small, lds);
+        tpp += n;
     }
     // ---- APTP fronts ----
     if (na > 0) {
@@ -5102,7 +5124,7 @@ void NumericGPU::enqueue_level(int lv, const double *d_val, const double *d_scal
             la_pending = false;
         }
         if (o_.failed_pivot_tpp)
-            hipLaunchKernelGGL((k_tpp<512, 4>), dim3(na), dim3(512), TPP_LDS_MAX, stream_, d_fr_, dl, 1, o_.threshold,
+            hipLaunchKernelGGL((k_tpp<512, 4, true>), dim3(na), dim3(512), TPP_LDS_MAX, stream_, d_fr_, dl, 1, o_.threshold,
                                o_.small, (unsigned)TPP_LDS_MAX);
     }
     // ---- kept factor columns of the pooled fronts: final from here on, read beside the

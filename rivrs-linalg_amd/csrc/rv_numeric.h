@@ -204,8 +204,8 @@ private:
         std::vector<size_t> o_ea, n_ea;
         int nf = 0, na = 0, max_outer = 0;
         unsigned prec_gen = 0;
-        size_t ntpp_small = 0, tpp_lds[2] = {0, 0};  // TPP fronts staged in little LDS, LDS per launch
-        size_t nsch = 0, ntpp = 0, nk2 = 0, nk3 = 0, nf0 = 0, nf1 = 0;
+        size_t ntpp[4] = {}, tpp_lds[4] = {};  // TPP fronts per launch (TppClass) and its LDS
+        size_t nsch = 0, nk2 = 0, nk3 = 0, nf0 = 0, nf1 = 0;
         size_t o_zl = 0, nzl = 0;  // lower-triangle zeroing items (front, first column)
         size_t o_kf = 0, nkf = 0;  // factor-column copy items (front, chunk)
         std::vector<int> ninner;
