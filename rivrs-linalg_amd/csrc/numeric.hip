@@ -1048,11 +1048,12 @@ __device__ __forceinline__ void stores_done_barrier() {
 // ===========================================================================
 // Symmetric line permutation for a sequence of at most MAX_IB swap_symmetric calls (factor.rs:452-505):
 // the composite touches at most 2 MAX_IB lines U.  Outside U x U every other line q is independent:
-// a thread loads its q's entries of up to 32 touched lines (whole cycles of the permutation, all
+// a thread loads its q's entries of up to RL touched lines (whole cycles of the permutation, all
 // loads of a round in flight) and stores them to the lines' new places; the U x U entries go
-// through S.swapbuf.  CO: device-scope accesses to the front (inside the persistent launch, where
+// through S.swapbuf.  RL: MAX_IB, or half of that where a launch of thousands of workgroups, most of them
+// without a swap, should hold eight wavefronts per SIMD (k_block_finish).  CO: device-scope accesses to the front (inside the persistent launch, where
 // the panels share the other lines).
-// Out of line: its registers stay out of the callers' common path.  Snapshotting whole lines to
+// apply_swaps is out of line: its registers stay out of the callers' common path.  Snapshotting whole lines to
 // memory one element and round trip at a time took a quarter of the factorization of a KKT system
 // with many delays (side 45: 28.4 ms, 21.9 so); by the leader of the persistent launch alone the
 // lines still took 88 us a block, shared between its workgroups the step went from 17.9 to 13.6 ms.
@@ -1062,10 +1063,11 @@ struct SwapLds {
     int from[2 * MAX_IB];  // line i receives line from[i] (indices into U)
     int ptmp[2 * MAX_IB];
     int mv[2 * MAX_IB];    // moved lines cycle by cycle: destination index, + 64 where a cycle ends
-    int gend[2 * MAX_IB];  // rounds of at most MAX_IB moves (whole cycles): end in mv
-    int n, nmv, ng;        // (ng = 0: a cycle of more than MAX_IB lines)
+    int gend[2 * MAX_IB];  // rounds of at most RL moves (whole cycles): end in mv
+    int n, nmv, ng;        // (ng = 0: a cycle of more than RL lines)
 };
 // The plan of a sequence of nsw swaps (all threads; ends with the barrier).
+template <int RL>
 __device__ __forceinline__ void swap_plan(SwapLds &W, const int *sa, const int *sb, int nsw) {
     static_assert(MAX_IB == 32, "a touched line per lane");
     const int lane = threadIdx.x & 63;
@@ -1101,8 +1103,8 @@ __device__ __forceinline__ void swap_plan(SwapLds &W, const int *sa, const int *
                 ++k;
                 c = nx;
             } while (c != first);
-            longc |= k - k0 > MAX_IB;
-            if (k - g0 > MAX_IB) {
+            longc |= k - k0 > RL;
+            if (k - g0 > RL) {
                 if (lane == 0) W.gend[ng] = k0;
                 ++ng;
                 g0 = k0;
@@ -1120,7 +1122,7 @@ __device__ __forceinline__ void swap_plan(SwapLds &W, const int *sa, const int *
 
 // The touched lines' crossings with the lines [q_begin, q_end) outside U; a wavefront takes 64 of
 // these and one round.
-template <bool CO>
+template <bool CO, int RL>
 __device__ __forceinline__ void swap_lines(FrontDev &F, const SwapLds &W, int q_begin, int q_end) {
     constexpr int AUX = CO ? 16 : 0;
     typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
@@ -1143,23 +1145,23 @@ __device__ __forceinline__ void swap_lines(FrontDev &F, const SwapLds &W, int q_
         if (ng > 0) {
             const int g0 = g > 0 ? __builtin_amdgcn_readfirstlane(W.gend[g > 0 ? g - 1 : 0]) : 0;
             const int n = __builtin_amdgcn_readfirstlane(W.gend[g]) - g0;
-            double v[MAX_IB];
+            double v[RL];
 #pragma unroll
-            for (int s = 0; s < MAX_IB; ++s)
+            for (int s = 0; s < RL; ++s)
                 if (s < n) {
                     const int u = __builtin_amdgcn_readlane(ul, __builtin_amdgcn_readlane(fl, __builtin_amdgcn_readlane(ml, g0 + s)));
                     const unsigned off = in ? 8u * ((unsigned)max(q, u) + (unsigned)min(q, u) * (unsigned)m) : CO_OOB;
                     v[s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(ra, (int)off, 0, AUX));
                 }
 #pragma unroll
-            for (int s = 0; s < MAX_IB; ++s)
+            for (int s = 0; s < RL; ++s)
                 if (s < n) {
                     const int u = __builtin_amdgcn_readlane(ul, __builtin_amdgcn_readlane(ml, g0 + s));
                     const unsigned off = in ? 8u * ((unsigned)max(q, u) + (unsigned)min(q, u) * (unsigned)m) : CO_OOB;
                     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v[s]), ra, (int)off, 0, AUX);
                 }
         } else if (in) {
-            // a long cycle, or a front past 8 GB: along each cycle, the first entry kept aside
+            // a long cycle, or a front of 1 GiB (order 11586) or more: along each cycle, the first entry kept aside
             double first = 0.0;
             bool start = true;
             for (int s = 0; s < nmv; ++s) {
@@ -1219,27 +1221,33 @@ __device__ __forceinline__ void swap_cross(FrontDev &F, AptpState &S, SwapLds &W
 }
 
 // The whole permutation by one workgroup.
-__device__ __attribute__((noinline)) void apply_swaps(FrontDev &F, AptpState &S, const int *sa, const int *sb, int nsw,
-                                                      SwapLds &W) {
-    swap_plan(W, sa, sb, nsw);
+template <int RL>
+__device__ __forceinline__ void apply_swaps_inline(FrontDev &F, AptpState &S, const int *sa, const int *sb, int nsw,
+                                                   SwapLds &W) {
+    swap_plan<RL>(W, sa, sb, nsw);
     if (W.nmv > 0) {
         swap_cross<false>(F, S, W);
-        swap_lines<false>(F, W, 0, F.m);
+        swap_lines<false, RL>(F, W, 0, F.m);
     }
     __syncthreads();
+}
+
+__device__ __attribute__((noinline)) void apply_swaps(FrontDev &F, AptpState &S, const int *sa, const int *sb, int nsw,
+                                                      SwapLds &W) {
+    apply_swaps_inline<MAX_IB>(F, S, sa, sb, nsw, W);
 }
 
 // Inside the persistent launch the permutation is shared: the leader's part (part < 0), and part of
 // np of the other lines.  Ends with the workgroup's stores complete.
 __device__ __forceinline__ void apply_swaps_shared(FrontDev &F, AptpState &S, const int *sa, const int *sb,
                                                              int nsw, SwapLds &W, int part, int np) {
-    swap_plan(W, sa, sb, nsw);
+    swap_plan<MAX_IB>(W, sa, sb, nsw);
     if (W.nmv > 0) {
         if (part < 0) {
             swap_cross<true>(F, S, W);
         } else {
             const int per = (F.m + np - 1) / np;
-            swap_lines<true>(F, W, min(part * per, F.m), min((part + 1) * per, F.m));
+            swap_lines<true, MAX_IB>(F, W, min(part * per, F.m), min((part + 1) * per, F.m));
         }
     }
     stores_done_barrier();
@@ -1672,7 +1680,9 @@ __global__ __launch_bounds__(256) void k_block_finish(FrontDev *__restrict__ fr,
         s_end = end_pos;
     }
     __syncthreads();
-    apply_swaps(F, S, sa, sb, nsw, sw);
+    // (with the swaps of RL = MAX_IB out of line the launch took 196 registers: 50 us for 4000 fronts
+    // without a failed column, 16 so)
+    if (nsw > 0) apply_swaps_inline<MAX_IB / 2>(F, S, sa, sb, nsw, sw);
     if (tid == 0) {
         S.kpos = k + nelim;
         S.end_pos = s_end;
