@@ -2796,8 +2796,15 @@ __device__ void outer_begin(FrontDev &F, AptpState &S, int ob, int nb, int ib) {
 // End of an outer block: failed columns move to the end of the remaining fully-summed
 // region (factor.rs:2195-2206), counters advance; the last block records ne.  Returns false
 // when the front has no outer block ob or only one outer block (then it has no block ob + 1
-// either); the return is the same for every thread of the workgroup.
-__device__ bool outer_end(FrontDev &F, AptpState &S, int ob, int nb, int la) {
+// either); the return is the same for every thread of the workgroup.  A front that ends with columns
+// left over joins the list `left` (its length, then the fronts) that k_tpp_left works through.
+__device__ bool outer_end(FrontDev *__restrict__ fr, int front, AptpState &S, int ob, int nb, int la,
+                          int *__restrict__ left) {
+    FrontDev &F = fr[front];
+    auto last = [&](int ne) {
+        F.ne = ne;
+        if (ne < F.k) left[1 + atomicAdd(left, 1)] = front;
+    };
     const bool deferred = !(F.flags & FRONT_ALLFS);
     const int p = F.k;
     const bool two = p > nb;
@@ -2808,7 +2815,7 @@ __device__ bool outer_end(FrontDev &F, AptpState &S, int ob, int nb, int la) {
     __shared__ int nsw;
     const int tid = threadIdx.x;
     if (!two) {
-        if (tid == 0) F.ne = S.kpos;
+        if (tid == 0) last(S.kpos);
         return false;
     }
     const int obne = S.kpos - S.ob_start;
@@ -2846,19 +2853,21 @@ __device__ bool outer_end(FrontDev &F, AptpState &S, int ob, int nb, int la) {
     if (tid == 0) {
         S.gne += obne;
         S.remaining -= S.ob_cols;
-        if (ob == nouter - 1) F.ne = S.gne;
+        if (ob == nouter - 1) last(S.gne);
     }
     return true;
 }
 
 // The first outer block of every front of a level: the APTP state is installed from its staged
 // initial value (scratch pointers, fail_min = INT_MAX, the rest zero), then outer block 0 starts.
+// Clears the list of fronts with columns left over.
 __global__ __launch_bounds__(256) void k_outer_first(FrontDev *__restrict__ fr,
                                                      AptpState *__restrict__ st,
                                                      const AptpState *__restrict__ init,
                                                      const int *__restrict__ flist, int nb, int ib,
-                                                     ChainSync *__restrict__ cs) {
+                                                     ChainSync *__restrict__ cs, int *__restrict__ left) {
     if (cs) chain_reset(cs[blockIdx.x]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *left = 0;
     FrontDev &F = fr[flist[blockIdx.x]];
     AptpState &S = st[blockIdx.x];
     const AptpState &I = init[blockIdx.x];
@@ -2872,8 +2881,9 @@ __global__ __launch_bounds__(256) void k_outer_first(FrontDev *__restrict__ fr,
 
 __global__ __launch_bounds__(256) void k_outer_end(FrontDev *__restrict__ fr,
                                                    AptpState *__restrict__ st,
-                                                   const int *__restrict__ flist, int ob, int nb) {
-    outer_end(fr[flist[blockIdx.x]], st[blockIdx.x], ob, nb, 0);
+                                                   const int *__restrict__ flist, int ob, int nb,
+                                                   int *__restrict__ left) {
+    outer_end(fr, flist[blockIdx.x], st[blockIdx.x], ob, nb, 0, left);
 }
 
 // The end of outer block ob and the start of ob + 1 in one launch (one workgroup per front).
@@ -2882,18 +2892,19 @@ __global__ __launch_bounds__(256) void k_outer_end(FrontDev *__restrict__ fr,
 __global__ __launch_bounds__(512) void k_outer_next(FrontDev *__restrict__ fr,
                                                     AptpState *__restrict__ st,
                                                     const int *__restrict__ flist, int ob, int nb,
-                                                    int ib, ChainSync *__restrict__ cs, int la) {
+                                                    int ib, ChainSync *__restrict__ cs, int la,
+                                                    int *__restrict__ left) {
     if (cs) chain_reset(cs[blockIdx.x]);
-    FrontDev &F = fr[flist[blockIdx.x]];
+    const int front = flist[blockIdx.x];
     AptpState &S = st[blockIdx.x];
-    if (!outer_end(F, S, ob, nb, la)) return;
+    if (!outer_end(fr, front, S, ob, nb, la, left)) return;
     __syncthreads();
-    outer_begin(F, S, ob + 1, nb, ib);
+    outer_begin(fr[front], S, ob + 1, nb, ib);
 }
 
 // ===========================================================================
 // Threshold partial pivoting (tpp_factor / tpp_factor_rect, factor.rs:2268-2947).
-// mode 0: whole front from column 0; mode 1: fallback from F.ne.
+// Of whole fronts (k_tpp) or of the columns that APTP left over (k_tpp_left).
 // ===========================================================================
 // Raw buffer loads (gfx9 resource: stride 0, range-checked against num_records): an offset at or
 // beyond the range loads zero without touching memory.
@@ -3256,7 +3267,7 @@ __device__ __forceinline__ int tpp_run(const TppMat<P> &M, FrontDev &F, int c0, 
     return nelim;
 }
 
-// One workgroup per front: mode 0 the whole front, mode 1 the columns APTP left (from F.ne).  A
+// A front's columns from c0 on by one workgroup.  A
 // pivot step is a serial chain of scans, so its memory round trips decide: the columns still to
 // eliminate are staged in LDS where they fit (lds bytes).  PARTS: wider remainders are worked on in
 // place until the rest fits, the step's new columns of L kept in LDS (without it a wide front is
@@ -3266,13 +3277,9 @@ __device__ __forceinline__ int tpp_run(const TppMat<P> &M, FrontDev &F, int c0, 
 // workgroup reduction of its own.  422 left-over columns at the root of KKT 45: 5.3 ms in place
 // throughout on 1024 threads, 3.8 so on 512 (24 -> 15 us a step in memory, 4.7 staged).
 template <int NT, int TJ, bool PARTS>
-__global__ __launch_bounds__(NT) void k_tpp(FrontDev *__restrict__ fr, const int *__restrict__ flist,
-                                            int mode, double u, double small, unsigned lds) {
-    extern __shared__ __align__(16) double dyn[];
-    FrontDev &F = fr[flist[blockIdx.x]];
+__device__ __forceinline__ void tpp_front(FrontDev &F, int c0, double u, double small, unsigned lds, double *dyn) {
     const size_t lda = F.m;
     const int tid = threadIdx.x;
-    int c0 = (mode == 0) ? 0 : F.ne;
     for (bool more = c0 < F.k; more;) {
         const int n = F.k - c0, m = F.m - c0;
         gdouble *G = gbl(F.F) + c0 + c0 * lda;
@@ -3353,6 +3360,29 @@ __global__ __launch_bounds__(NT) void k_tpp(FrontDev *__restrict__ fr, const int
         }
         c0 += nelim;
         __syncthreads();
+    }
+}
+
+// Whole fronts, one workgroup each.
+template <int NT, int TJ, bool PARTS>
+__global__ __launch_bounds__(NT) void k_tpp(FrontDev *__restrict__ fr, const int *__restrict__ flist, double u,
+                                            double small, unsigned lds) {
+    extern __shared__ __align__(16) double dyn[];
+    tpp_front<NT, TJ, PARTS>(fr[flist[blockIdx.x]], 0, u, small, lds, dyn);
+}
+
+// The columns APTP left over, of the fronts that have some.  Its LDS lets one workgroup onto a CU, so
+// TPP_LEFT_WG of them take the fronts of the list in turn: a workgroup for every front of the level
+// cost 60 us at 4000 fronts of order 40 (280 at order 180), most of them without such a column.
+constexpr int TPP_LEFT_WG = 256;
+template <int NT, int TJ>
+__global__ __launch_bounds__(NT) void k_tpp_left(FrontDev *__restrict__ fr, const int *__restrict__ left, double u,
+                                                 double small, unsigned lds) {
+    extern __shared__ __align__(16) double dyn[];
+    const int n = left[0];
+    for (int f = blockIdx.x; f < n; f += gridDim.x) {
+        FrontDev &F = fr[left[1 + f]];
+        tpp_front<NT, TJ, true>(F, F.ne, u, small, lds, dyn);
     }
 }
 
@@ -4926,6 +4956,7 @@ void NumericGPU::plan_level(int lv, bool reset_arena) {
         L.dS = (AptpState *)scratch_.alloc((size_t)na * sizeof(AptpState));
         L.dSnap[0] = (AptpState *)scratch_.alloc((size_t)na * sizeof(AptpState));
         L.dSnap[1] = (AptpState *)scratch_.alloc((size_t)na * sizeof(AptpState));
+        L.dleft = (int *)scratch_.alloc((size_t)(na + 1) * sizeof(int));
         L.o_hs = stage_push(stg, hs.data(), hs.size());
     }
     // device copy of the blob; extend-add map fields become device addresses
@@ -5046,7 +5077,7 @@ void NumericGPU::enqueue_level(int lv, const double *d_val, const double *d_scal
         const unsigned n = (unsigned)L.ntpp[c], lds = (unsigned)L.tpp_lds[c];
         if (!n) continue;
         const auto kernel = c == TPP_WAVE ? k_tpp<64, 2, false> : c == TPP_MID ? k_tpp<128, 4, true> : k_tpp<256, 4, false>;
-        hipLaunchKernelGGL(kernel, dim3(n), dim3(c == TPP_WAVE ? 64 : c == TPP_MID ? 128 : 256), lds, stream_, d_fr_, tpp, 0,
+        hipLaunchKernelGGL(kernel, dim3(n), dim3(c == TPP_WAVE ? 64 : c == TPP_MID ? 128 : 256), lds, stream_, d_fr_, tpp,
                            o_.threshold, o_.small, lds);
         tpp += n;
     }
@@ -5058,7 +5089,7 @@ void NumericGPU::enqueue_level(int lv, const double *d_val, const double *d_scal
         for (int ob = 0; ob < L.max_outer; ++ob) {
             if (ob == 0)
                 hipLaunchKernelGGL(k_outer_first, dim3(na), dim3(256), 0, stream_, d_fr_, dS,
-                                   (const AptpState *)D(L.o_hs), dl, nb, ib, L.dC);
+                                   (const AptpState *)D(L.o_hs), dl, nb, ib, L.dC, L.dleft);
             if (L.chain_ch && L.n_chain[ob]) ++chain_launches_;
             if (L.chain_ch == 64 && L.n_chain[ob])
                 hipLaunchKernelGGL(k_aptp_outer<64>, dim3((unsigned)L.n_chain[ob]), dim3(256), 0, stream_, d_fr_,
@@ -5109,9 +5140,9 @@ void NumericGPU::enqueue_level(int lv, const double *d_val, const double *d_scal
             }
             if (ob + 1 < L.max_outer)
                 hipLaunchKernelGGL(k_outer_next, dim3(na), dim3(512), 0, stream_, d_fr_, dS, dl, ob, nb, ib, L.dC,
-                                   la ? 1 : 0);
+                                   la ? 1 : 0, L.dleft);
             else
-                hipLaunchKernelGGL(k_outer_end, dim3(na), dim3(256), 0, stream_, d_fr_, dS, dl, ob, nb);
+                hipLaunchKernelGGL(k_outer_end, dim3(na), dim3(256), 0, stream_, d_fr_, dS, dl, ob, nb, L.dleft);
             if (la) {
                 // forked once block ob + 1 can start, so that its persistent launch and this update
                 // begin dispatching together (an update dispatched first would hold every slot)
@@ -5134,8 +5165,8 @@ void NumericGPU::enqueue_level(int lv, const double *d_val, const double *d_scal
             la_pending = false;
         }
         if (o_.failed_pivot_tpp)
-            hipLaunchKernelGGL((k_tpp<512, 4, true>), dim3(na), dim3(512), TPP_LDS_MAX, stream_, d_fr_, dl, 1, o_.threshold,
-                               o_.small, (unsigned)TPP_LDS_MAX);
+            hipLaunchKernelGGL((k_tpp_left<512, 4>), dim3(std::min(na, TPP_LEFT_WG)), dim3(512), TPP_LDS_MAX, stream_,
+                               d_fr_, L.dleft, o_.threshold, o_.small, (unsigned)TPP_LDS_MAX);
     }
     // ---- kept factor columns of the pooled fronts: final from here on, read beside the
     // contribution GEMMs (which only read them) on stream2_, joined after the collect (measured

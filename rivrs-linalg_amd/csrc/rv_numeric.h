@@ -192,6 +192,7 @@ private:
         // copies of the APTP states for outer updates run beside the next outer block (by
         // outer-block parity, as the two W buffers o_wp1 / o_wp1b)
         AptpState *dSnap[2] = {nullptr, nullptr};
+        int *dleft = nullptr;  // fronts with columns left over: their number, then the fronts
         // contribution tiles per update precision (RV_PREC_* index)
         std::array<size_t, 4> o_ct{}, nct{};
         // outer-update tiles per outer block: [0] reference order (k_outer_exact), [1] FP32,

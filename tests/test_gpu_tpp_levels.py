@@ -12,15 +12,19 @@ pytestmark = pytest.mark.gpu
 
 def _systems(shapes, seed):
     """Independent systems (k, r): two leaves of k columns coupled to a dense border of r rows; k = 0:
-    a dense system of order r.  Small diagonals, so that most pivots are 2x2 or moved."""
+    a dense system of order r, k = -1: one with large couplings between its halves, whose blocks of 32
+    columns have few acceptable pivots.  Small diagonals, so that most pivots are 2x2 or moved."""
     rng = np.random.default_rng(seed)
     rows, cols, vals, at = [], [], [], 0
     for k, r in shapes:
-        n = 2 * k + r
+        n = 2 * max(k, 0) + r
         a = rng.standard_normal((n, n))
         a[np.arange(n), np.arange(n)] *= 0.1
+        if k < 0:
+            a[n - n // 2 + np.arange(n // 2), rng.permutation(n // 2)] += 1e4
         keep = np.tril(np.ones((n, n), dtype=bool))
-        keep[k:2 * k, :k] = False
+        if k > 0:
+            keep[k:2 * k, :k] = False
         i, j = np.nonzero(keep)
         rows.append(at + i)
         cols.append(at + j)
@@ -37,6 +41,8 @@ CASES = {
     "fewer": [(0, 1 + q % 31) for q in range(1024)],
     "parts": [(30, 66 + q % 47) for q in range(600)],
     "whole": [(30, 66 + q % 47) for q in range(400)],
+    # columns that block pivoting leaves over, in some of more fronts than workgroups take them
+    "left over": [(-1 if q % 3 else 0, 40 + q % 60) for q in range(600)],
 }
 
 
