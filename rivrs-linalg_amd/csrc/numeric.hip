@@ -433,8 +433,11 @@ __device__ __forceinline__ int fresh_uniform(int x) {
 //    diagonal of the LDS copy is NaN, so a pivot's own row gets NaN multipliers and dies in the
 //    ordinary update: no masks.
 //  * Argmax: an entry's key is the high word of its magnitude with the column index in the low
-//    five bits; as a float its NaN is ignored and its order is the magnitudes' (which is why
-//    blocks with entries above 2^1000 always take the exact rule).  Keys are reduced by v_max3 and
+//    five bits; as a float its NaN is ignored and its order is the magnitudes'.  From 2^1017 on a
+//    key would be a float NaN itself, which is why blocks with entries of 2^1000 or more always take
+//    the exact rule.  (Looked at once, before the first pivot: a pivot is at least 1/sqrt 2 of the
+//    largest entry left, a 2x2's determinant half its square, so by Hadamard's inequality, as in
+//    Wilkinson's bound for complete pivoting, the entries of 32 columns grow by less than 2^10.)  Keys are reduced by v_max3 and
 //    DPP, so the winner's row is its lane and its column the key's low bits.  It stands if no
 //    other lane's key and no other entry of its row reaches its leading 15 mantissa bits;
 //    otherwise (near-equal values, ties, tiny values) the exact rule runs: largest value, then
