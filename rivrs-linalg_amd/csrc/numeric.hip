@@ -437,7 +437,7 @@ __device__ __forceinline__ int fresh_uniform(int x) {
 //    key would be a float NaN itself, which is why blocks with entries of 2^1000 or more always take
 //    the exact rule.  (Looked at once, before the first pivot: a pivot is at least 1/sqrt 2 of the
 //    largest entry left, a 2x2's determinant half its square, so by Hadamard's inequality, as in
-//    Wilkinson's bound for complete pivoting, the entries of 32 columns grow by less than 2^10.)  Keys are reduced by v_max3 and
+//    Wilkinson's bound for complete pivoting, the entries of 32 columns grow by less than 2^11.)  Keys are reduced by v_max3 and
 //    DPP, so the winner's row is its lane and its column the key's low bits.  It stands if no
 //    other lane's key and no other entry of its row reaches its leading 15 mantissa bits;
 //    otherwise (near-equal values, ties, tiny values) the exact rule runs: largest value, then
@@ -2010,7 +2010,7 @@ struct ChainLeaderLds {
     int wbp[1];
     int sa[MAX_IB], sb[MAX_IB];
     SwapLds sw;
-    int nsw, s_end, s_fail, s_upd, s_pf, s_err;
+    int nsw, s_end, s_fail, s_upd, s_err;
 };
 constexpr int CHAIN_LC_COLS = 128;  // trailing columns per round of the panel update
 struct ChainPanelLds {
@@ -2110,7 +2110,6 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
     int n1 = 0, n2 = 0;
     bool have = false;  // the current block was factored ahead; its record is out
     bool upd_prev = false;  // the panels' updates of the previous block are known complete
-    bool pf = false;    // the next block's operands are in LDS
     int bn = 0;
     if (tid == 0) L.s_err = 0;
     for (int it = 0; it < nit; ++it) {
@@ -2154,10 +2153,12 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
             }
             if (tid == 0) atomic_max_nonneg(&F.max_l_bits, bml);
             write_record(C.recs[it], k, bs, bn, end_pos, L.bp, L.bkind, L.bdiag, L.boff, L.blk);
-            pf = false;
         }
         // the next block ahead (its operands are loaded before the record goes out: the panels
-        // overwrite those rows' block entries once they have it)
+        // overwrite those rows' block entries once they have it).  A block factored ahead finds them
+        // in LDS: they were left out beside its pivots only where there is no block after it
+        // (nbs2 <= 0 or it + 2 >= nit there, so not `ahead` here) or where a column of the
+        // block before had failed, and then it was discarded.
         const bool ahead = bs > 0 && bn == bs && nbs > 0 && it + 1 < nit;
         if (!have) {
             if (ahead) load_operands<256>(L, A, lda, perm, k, bs, be, nbs, tid);
@@ -2199,7 +2200,6 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
             for (int u = 0; u < MAX_IB / 8; ++u) L.Ct[ii][jg + 8 * u] = L.Cn[ii][jg + 8 * u];
             lds_barrier();
             if (tid < MAX_IB) L.operm[tid] = L.noperm[tid];
-            if (tid == 0) L.s_pf = 0;
             next_tile_update(Lr, Wt, L.Ct, L.bkind, L.bdiag, L.boff, nbs, bs, nv);
 #pragma unroll
             for (int u = 0; u < MAX_IB / 8; ++u) L.Nv[ii][jg + 8 * u] = nv[u];
@@ -2221,7 +2221,6 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
                     return;
                 }
                 load_operands<192>(L, A, lda, perm, be, nbs, be2, nbs2, tid - 64);
-                if (tid == 64) L.s_pf = 1;
             });
             if (tid < bn2 && L.nbkind[tid] == 2) L.Ct[tid + 1][tid] = 0.0;
             if (tid < 64) pivot_coefs(L.nbkind, L.nbdiag, L.nboff, bn2, L.pc);
@@ -2272,7 +2271,6 @@ __device__ __forceinline__ void chain_leader(FrontDev &F, AptpState &S, ChainSyn
                 L.bdiag[tid] = L.nbdiag[tid];
                 L.boff[tid] = L.nboff[tid];
             }
-            pf = L.s_pf != 0;
             lds_barrier();
             bn = bn2;
             k = be;

@@ -68,7 +68,6 @@ struct SolveFront {
     long long pbase;     // offset of the front's chunk partials in P
     int m, ne;
     int fbase;           // first block flag of the front
-    int ndone;           // forward: increments of the front's done counter (rows items, 1 if fused)
     int nchk;            // backward: chunks per column block
     int ech0, ech1;      // effective children (nearest descendants with ne > 0) in ech
     int epar;            // effective parent or -1
@@ -1177,7 +1176,6 @@ void NumericGPU::prepare_solve() {
         f.m = m_[s];
         f.ne = ne_[s];
         f.fbase = fbase[li];
-        f.ndone = ndone(li);
         f.nchk = nchk[li];
         f.ech0 = ech_ptr[li];
         f.ech1 = ech_ptr[li + 1];
@@ -1284,8 +1282,17 @@ void NumericGPU::prepare_solve() {
 
 // Columns per group of right-hand sides, dealt evenly to groups of at most 4 or, past 32 columns,
 // 8.  Groups of 4 have the shorter chain step, groups of 8 read the factor half as often, which
-// counts once the groups fill the chip.  Helmholtz 40^3, both sweeps, groups of 4 / of 8: 8 columns
-// 657 / 870 us, 16: 828 / 964, 32: 1190 / 1210, 64: 1985 / 1635.
+// counts once the groups fill the chip.  How many groups do depends on the factor; the line is that of
+// Helmholtz 40^3, between the small factors, whose groups of 4 stay ahead throughout, and the large
+// ones, whose groups of 8 lead from 12 to 20 columns on.  Both sweeps, groups of at most 4 / of 8, us:
+//   columns                 8            16            32            64
+//   Helmholtz 20^3     270 /  346    269 /  355    288 /  358    345 /  384
+//   KKT side 64        489 /  685    517 /  698    584 /  720    684 /  800
+//   KKT side 128      3820 / 5860   4080 / 5890   4640 / 6220   6140 / 7040
+//   Helmholtz 40^3     657 /  875    819 /  967   1170 / 1170   1980 / 1630
+//   2-D grid 400^2     937 /  810   1560 / 1190   2930 / 2050   5780 / 3850
+//   48 KKT systems    1615 / 1588   2550 / 2135   4500 / 3330   8440 / 5860
+//   Helmholtz 64^3    2570 / 2700   3770 / 3410   6330 / 4930  11600 / 8260
 int NumericGPU::solve_group_width(int nrhs) {
     if (nrhs <= 0) return 1;
     const int most = nrhs <= 32 ? 4 : 8;
