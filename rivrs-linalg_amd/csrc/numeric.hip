@@ -3268,12 +3268,11 @@ __device__ __forceinline__ int tpp_run(const TppMat<P> &M, FrontDev &F, int c0, 
     return nelim;
 }
 
-// A front's columns from c0 on by one workgroup.  A
-// pivot step is a serial chain of scans, so its memory round trips decide: the columns still to
-// eliminate are staged in LDS where they fit (lds bytes).  PARTS: wider remainders are worked on in
-// place until the rest fits, the step's new columns of L kept in LDS (without it a wide front is
-// worked on in place throughout, the kernel keeps to few registers).  Rows of earlier columns follow
-// the row order at the end of either part.
+// A front's columns from c0 on by one workgroup.  A pivot step is a serial chain of scans, so its
+// memory round trips decide: the columns still to eliminate are staged in LDS where they fit (lds
+// bytes).  PARTS: wider remainders are worked on in place until the rest fits, the step's new columns
+// of L kept in LDS (without it a wide front is worked on in place throughout, the kernel keeps to
+// few registers).  Rows of earlier columns follow the row order at the end of either part.
 // KKT of side 16 (fronts up to 131 x 131): about 5 us a step, 26 us with every scan through L2 and a
 // workgroup reduction of its own.  422 left-over columns at the root of KKT 45: 5.3 ms in place
 // throughout on 1024 threads, 3.8 so on 512 (24 -> 15 us a step in memory, 4.7 staged).
